@@ -16,6 +16,7 @@ struct TaskDev {
   int       nsub[6];     // ceil(dim/4): 4^6 sub-tiles of the FP64 kernel per position
   int       nsubm[6];    // mixed kernel (4,4,4 | 8,8,8) boxes: ceil(dim/4), ceil(dim/8)
   int       n_sub;       // product of nsub
+  int       eq;          // equal tiles: bit 0 h1b = h2b, 1 h2b = h3b, 2 p4b = p5b, 3 p5b = p6b
   // Per output bipartition g = 3*hs + ps (hs: single hole position 0..2,
   // ps: single particle position 0..2), 6 bits each:
   //   bit0 enabled, bit1 negative sign, bit2 a1, bit3 a2, bit4 b1, bit5 b2
@@ -88,16 +89,17 @@ struct MixedDev {
 // Work queues: one per XCD.  Queue q holds the tasks qtask[qbeg[q]..qbeg[q+1])
 // in processing order; entry e owns a contiguous ticket range of its queue
 // starting at qtick[e].  A ticket is one box of the kernel (one 4^6 sub-tile
-// for FP64, one (4,4,4|8,8,8) box for mixed).  64 consecutive tickets form a
-// group of neighbouring boxes, 2^glog[p] along position p (sum of glog = 6):
-// the group shape decides which operand panels the workgroups resident on one
-// XCD share in its L2.  A task has 64 * prod(ceil(nsub[p] / 2^glog[p]))
-// tickets; tickets outside the task's box grid are skipped.
+// for FP64, one (4,4,4|8,8,8) box for mixed).  Consecutive tickets run through
+// groups of neighbouring boxes, 2^glog[p] along position p (sum of glog = 6)
+// cut at the grid's edge: the group shape decides which operand panels the
+// workgroups resident on one XCD share in its L2.  A task has one ticket per
+// box; boxes that the antisymmetry of equal tiles makes copies of another
+// (fold_weight in xt_queue.h) are passed over by the thread that claims them.
 constexpr int kQueues = 8;
 // Threads of the one workgroup that sums the task energies in a fixed order
 // (k_reduce_final); xt_sum_task_energies repeats the same order on the host.
 constexpr int kReduceThreads = 256;
-constexpr int kGroupLog2 = 6;  // 64 boxes per ticket group
+constexpr int kGroupLog2 = 6;  // 64 boxes per whole ticket group
 
 struct RunDev {
   const TaskDev*      tasks;
@@ -110,10 +112,12 @@ struct RunDev {
                                // beyond 2^62 Eh (zeroed before a run, read after it)
   unsigned long long* acc;     // [4*n_tasks] (E4 lo, E4 hi, E5 lo, E5 hi): 128-bit
                                // two's-complement fixed point, scale 2^64 per Eh
-  unsigned long long* cost;    // [n_tasks] summed workgroup wall-clock ticks (optional)
+  unsigned long long* cost;    // [n_tasks] summed workgroup wall-clock ticks, a box's times its
+                               // fold weight (optional)
   unsigned long long* prog;    // [kQueues] host-mapped mirror of the ticket counters (optional)
   int                 n_tasks;
   int                 glog[6];  // ticket group shape (log2 extent per position, sum 6)
+  int                 fold;     // 1: skip the copies of boxes with equal tiles (fold_weight)
 };
 
 // Device allocations of the upload paths (xt_host.cpp): hipMalloc / hipFree,
@@ -136,6 +140,8 @@ int cholesky_integrals(int O, int V, long K, const double* L, double* vvoo, doub
 int build_xva(int O, int V, SpatialBufs& B, void* stream);
 // Reorders the (ai|bj) GEMM result [(a,i)][(b,j)] into vvoo[a][b][i][j].
 int launch_vvoo_order(const double* in, double* out, int O, int V, void* stream);
+// Largest |(ai|bj) - (bj|ai)| and largest |(ai|bj)| of a vvoo array (waits for the stream).
+int vvoo_asymmetry(const double* vvoo, int O, int V, double* diff, double* largest, void* stream);
 // With vvvo == nullptr the xv/xva pair is left to the caller.
 int build_operands(int O, int V, double* t2, double* ovoo, double*& vvvo, SpatialBufs& B,
                    void* stream);

@@ -279,6 +279,8 @@ int build_plan(Plan& P, int O, int V, const std::vector<int>& occ, const std::ve
     int nd1, nd2, ns1;
     slot_codes(sp, T.d1code, T.d2code, T.s1code, nd1, nd2, ns1);
     T.factor     = P.factors[k];
+    const long* b = &P.tasks[6 * k];
+    T.eq         = (b[0] == b[1]) | (b[1] == b[2]) << 1 | (b[3] == b[4]) << 2 | (b[4] == b[5]) << 3;
     for(int p = 0; p < 6; p++) T.nsubm[p] = (T.dim[p] + (p < 3 ? 3 : 7)) / (p < 3 ? 4 : 8);
     double prod = 1;
     for(int p = 0; p < 6; p++) prod *= T.dim[p];
@@ -309,6 +311,7 @@ struct xt_ctx {
   int         n_cu   = 0;
   Plan        plan;
   bool        have_plan = false, have_inputs = false;
+  bool        fold = false;  // the inputs let boxes of equal tiles be folded (set_fold)
   // device inputs (kernel layouts)
   xt::SpatialBufs in    = {};
   xt::SplitBufs   split = {};  // FP16 split operands (built on the first mixed run)
@@ -343,12 +346,12 @@ struct xt_ctx {
   // timing mode; it is dropped whenever a buffer it names is reallocated.
   hipGraphExec_t graph = nullptr;
   struct GraphKey {
-    int         precision = -1, grid = 0, timed = 0;
+    int         precision = -1, grid = 0, timed = 0, progress = 0;
     long        n_tasks   = -1;
     const void* inputs    = nullptr;
     bool        operator==(const GraphKey& k) const {
       return precision == k.precision && grid == k.grid && timed == k.timed &&
-             n_tasks == k.n_tasks && inputs == k.inputs;
+             progress == k.progress && n_tasks == k.n_tasks && inputs == k.inputs;
     }
   } graph_key;
 
@@ -677,6 +680,19 @@ void xt::track_free(void* p) {
 
 extern "C" {
 
+// Boxes of equal tiles are folded (fold_weight, xt_queue.h) where the singles
+// term is antisymmetric too.  t3 is so by the way its operands are formed; the
+// singles term is if vvoo has the symmetry (ai|bj) = (bj|ai) that the upload
+// asks for.  Integrals that miss it by more than their own rounding (1e-13 of
+// the largest; products over Cholesky vectors miss it by a few 1e-16) are run
+// over every box.
+static int set_fold(xt_ctx* c) {
+  double    diff = 0.0, largest = 0.0;
+  const int err = xt::vvoo_asymmetry(c->in.vvoo, c->plan.O, c->plan.V, &diff, &largest, c->stream);
+  c->fold       = !err && diff <= 1e-13 * largest;
+  return err;
+}
+
 static int upload_common(xt_ctx* c, const double* eo, const double* ev, const double* t1,
                          const double* t2, const double* vvoo, const double* ovoo,
                          const double* vvvo) {
@@ -716,6 +732,7 @@ static int upload_common(xt_ctx* c, const double* eo, const double* ev, const do
     return rc;
   }
   int err = xt::build_operands((int) o, (int) v, t2_d, ovoo_d, vvvo_d, c->in, st);
+  if(!err) err = set_fold(c);
   if(err) {
     cleanup();
     return fail(err == (int) hipErrorOutOfMemory ? XT_ENOMEM : XT_EHIP,
@@ -788,6 +805,7 @@ int xt_upload_cholesky(xt_ctx* c, const double* eps_occ, const double* eps_vir, 
     err = xt::build_operands((int) o, (int) v, t2_d, ovoo_d, none, c->in, st);
   }
   if(!err) err = xt::build_xva((int) o, (int) v, c->in, st);
+  if(!err) err = set_fold(c);
   if(err) {
     cleanup();
     return fail(err == (int) hipErrorOutOfMemory ? XT_ENOMEM : XT_EHIP,
@@ -900,10 +918,23 @@ struct Queues {
   std::vector<long long> tick, total;
 };
 
-// Tickets of task T under group shape glog (one group of 64 boxes per
-// ceil(n/2^glog) cell of the task's box grid).
+// Tickets of task T under group shape glog: one per box.
 static long long task_tickets(const xt::TaskDev& T, const int* glog, bool mixed) {
   return xt::task_ticket_count(mixed ? T.nsubm : T.nsub, glog);
+}
+
+// Share of a task's boxes that run when the copies under the exchange of
+// equal tiles are skipped.
+static double fold_share(const xt::TaskDev& T, bool mixed) {
+  const int* nb    = mixed ? T.nsubm : T.nsub;
+  double     share = 1.0;
+  for(int s = 0; s < 6; s += 3) {
+    const int    e = (T.eq >> (s ? 2 : 0)) & 3;
+    const double n = nb[e == 2 ? s + 1 : s];  // boxes along the equal positions
+    if(e == 3) share *= (n + 1) * (n + 2) / (6 * n * n);
+    else if(e) share *= (n + 1) / (2 * n);
+  }
+  return share;
 }
 
 static Queues build_queues(const Plan& P, const std::vector<int>& sel, int schedule,
@@ -1028,10 +1059,13 @@ static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
   R.err     = c->d_qctr + xt::kQueues;
   R.acc     = c->d_acc;
   R.cost    = o.record_task_time ? c->d_cost : nullptr;
-  R.prog    = c->d_prog;
+  // the mirror in host memory costs a PCIe store per ticket, which the kernel's
+  // end waits for: only where the caller asked for progress lines
+  R.prog    = o.progress_ms > 0 ? c->d_prog : nullptr;
   for(int q = 0; q < xt::kQueues; q++) __atomic_store_n(&c->h_prog[q], 0ull, __ATOMIC_RELAXED);
   R.n_tasks = (int) nt;
   for(int p = 0; p < 6; p++) R.glog[p] = glog[p];
+  R.fold = c->fold ? 1 : 0;
   long long tickets = 0;
   for(long long t: Q.total) tickets += t;
   // the FP64 kernel's LDS and registers fit three workgroups on a CU, the
@@ -1067,6 +1101,7 @@ static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
   key.precision = o.precision;
   key.grid      = grid;
   key.timed     = o.record_task_time ? 1 : 0;
+  key.progress  = o.progress_ms > 0 ? 1 : 0;
   key.n_tasks   = nt;
   key.inputs    = mixed ? (const void*) c->split.v[0] : (const void*) c->in.xv;
   if(!c->graph || !(c->graph_key == key)) {
@@ -1095,7 +1130,8 @@ static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
   return report_progress(c, o, Q);
 }
 
-// Summed workgroup time of each task (ms), from wall-clock ticks.
+// Summed workgroup time of each task (ms), from wall-clock ticks; a box that
+// stands for its copies (fold_weight) counts once for each.
 static int task_times(xt_ctx* c, long nt, float* task_ms) {
   std::vector<unsigned long long> ticks(nt);
   XT_HIP(hipMemcpy(ticks.data(), c->d_cost, nt * 8, hipMemcpyDeviceToHost));
@@ -1608,7 +1644,9 @@ int xt_learn_schedule(xt_ctx* c, xt_mlp* m, const xt_opts* opts, long n_sample, 
   std::vector<double> cost(n);
   for(long k = 0; k < n; k++) {
     const double fl = c->plan.dev[k].flops;
-    const double cc = fl * std::exp(mu + sd * (double) y[k]);
+    // predicted time of every box, times the share of them that runs
+    const double cc = fl * std::exp(mu + sd * (double) y[k]) *
+                      (c->fold ? fold_share(c->plan.dev[k], opts->precision == XT_PREC_MIXED) : 1.0);
     cost[k]         = (std::isfinite(cc) && cc > 0.0) ? cc : fl;
   }
   c->learned_cost = cost;

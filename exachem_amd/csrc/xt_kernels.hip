@@ -362,6 +362,7 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
 __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) {
   __shared__ Smem               sm;
   __shared__ int                s_task;
+  __shared__ int                s_weight;  // thread 0: boxes that its box stands for
   __shared__ int                s_entry;   // thread 0: entry of its last ticket on the current queue
   __shared__ int                s_cur;     // thread 0: task of the running sums
   __shared__ unsigned long long s_sum[4];  // thread 0: E4 lo, hi, E5 lo, hi of s_cur not yet added
@@ -379,33 +380,35 @@ __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) 
     for(;;) {
       __syncthreads();  // previous sub-tile finished with LDS and s_task
       if(tid == 0) {
-        const unsigned long long t = atomicAdd(&R.qctr[q], 1ull);
-        // progress mirror in host memory (tickets taken so far, approximate)
-        if(R.prog) __hip_atomic_store(&R.prog[q], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         int ti = -1;  // -1: queue exhausted
-        if((long long) t < R.qtotal[q]) {
+        for(;;) {
+          const unsigned long long t = atomicAdd(&R.qctr[q], 1ull);
+          // progress mirror in host memory (tickets taken so far, approximate)
+          if(R.prog) __hip_atomic_store(&R.prog[q], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          if((long long) t >= R.qtotal[q]) break;
           const int e = queue_entry_from(R.qbeg, R.qtick, q, (long long) t, s_entry);
           s_entry     = e;
           ti          = R.qtask[e];
           const TaskDev& T = R.tasks[ti];
-          // ticket -> sub-tile: the low bits select the box inside its group
-          int sub[6];
-          if(ticket_box((long long) t - R.qtick[e], T.nsub, R.glog, sub)) {
+          int            sub[6];
+          const bool     in = ticket_box((long long) t - R.qtick[e], T.nsub, R.glog, sub);
+          // a copy of another box under the exchange of equal tiles is passed over
+          s_weight = !in ? 0 : R.fold ? fold_weight(T.eq, sub) : 1;
+          ti       = s_weight ? ti : -1;
+          if(ti < 0) continue;
 #pragma unroll
-            for(int p = 0; p < 6; p++) {
-              sm.sub[p] = sub[p];
-              sm.dim[p] = T.dim[p];
-              sm.off[p] = T.off[p];
-            }
+          for(int p = 0; p < 6; p++) {
+            sm.sub[p] = sub[p];
+            sm.dim[p] = T.dim[p];
+            sm.off[p] = T.off[p];
           }
-          else ti = -2;  // a ticket past the task's sub-tile grid (its last group overhangs)
+          break;
         }
         s_task = ti;
       }
       __syncthreads();
       const int ti = s_task;
-      if(ti == -1) break;
-      if(ti == -2) continue;
+      if(ti < 0) break;
       const TaskDev&           T  = R.tasks[ti];
       const unsigned long long t0 = wall_clock64();
       double                   e4, e5;
@@ -415,8 +418,9 @@ __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) 
           sums_flush(R, s_cur, s_sum);
           s_cur = ti;
         }
-        sums_add(R, s_sum, e4, e5);
-        if(R.cost) atomicAdd(&R.cost[ti], wall_clock64() - t0);
+        sums_add(R, s_sum, s_weight * e4, s_weight * e5);
+        // a box's time counts for its copies too, so a task's time follows its extents
+        if(R.cost) atomicAdd(&R.cost[ti], s_weight * (wall_clock64() - t0));
       }
     }
   }
@@ -603,6 +607,54 @@ int launch_vvoo_order(const double* in, double* out, int O, int V, void* stream)
   hipLaunchKernelGGL(k_vvoo_order, dim3(nblk(n)), dim3(256), 0, (hipStream_t) stream, in, out,
                      (long) O, (long) V);
   return (int) hipGetLastError();
+}
+
+// Largest |(ai|bj) - (bj|ai)| and largest |(ai|bj)| of vvoo, as the bits of
+// non-negative doubles (ordered like the values): out[0], out[1].
+__global__ void __launch_bounds__(256) k_vvoo_asym(const double* __restrict__ vvoo, long O, long V,
+                                                   unsigned long long* out) {
+  const unsigned o = (unsigned) O, oo = o * o;
+  double         d = 0.0, m = 0.0;
+  for(long p = blockIdx.x; p < V * V; p += gridDim.x) {  // one (a, b) pair at a time
+    const long    a = p / V, b = p - a * V;
+    const double* x = vvoo + p * oo;
+    const double* y = vvoo + (b * V + a) * oo;
+    for(unsigned q = threadIdx.x; q < oo; q += blockDim.x) {
+      const unsigned i = q / o, j = q - i * o;
+      const double   u = x[q];
+      m                = fmax(m, fabs(u));
+      if(a <= b) d = fmax(d, fabs(u - y[j * o + i]));
+    }
+  }
+#pragma unroll
+  for(int k = 32; k >= 1; k >>= 1) {
+    d = fmax(d, __shfl_xor(d, k, 64));
+    m = fmax(m, __shfl_xor(m, k, 64));
+  }
+  if((threadIdx.x & 63) == 0) {
+    atomicMax(&out[0], (unsigned long long) __double_as_longlong(d));
+    atomicMax(&out[1], (unsigned long long) __double_as_longlong(m));
+  }
+}
+
+int vvoo_asymmetry(const double* vvoo, int O, int V, double* diff, double* largest, void* stream) {
+  hipStream_t         st = (hipStream_t) stream;
+  unsigned long long* d  = nullptr;
+  hipError_t          e;
+  if((e = hipMalloc((void**) &d, 2 * sizeof(*d)))) return (int) e;
+  int rc = launch_zero_u64(d, 2, stream);
+  if(!rc) {
+    hipLaunchKernelGGL(k_vvoo_asym, dim3((unsigned) std::min<long>((long) V * V, 4096)), dim3(256), 0,
+                       st, vvoo, (long) O, (long) V, d);
+    rc = (int) hipGetLastError();
+  }
+  double h[2] = {0.0, 0.0};
+  if(!rc) rc = (int) hipMemcpyAsync(h, d, sizeof h, hipMemcpyDeviceToHost, st);
+  if(!rc) rc = (int) hipStreamSynchronize(st);
+  (void) hipFree(d);
+  *diff    = h[0];
+  *largest = h[1];
+  return rc;
 }
 
 int launch_zero_u64(unsigned long long* p, long n, void* stream) {

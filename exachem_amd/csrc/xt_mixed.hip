@@ -639,6 +639,7 @@ __device__ __forceinline__ void box_energy(MSmem& sm, const MixedDev& M, uint64_
 __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
   __shared__ MSmem              sm;
   __shared__ int                s_task;
+  __shared__ int                s_weight;  // thread 0: boxes that its box stands for
   __shared__ int                s_entry;   // thread 0: entry of its last ticket on the current queue
   __shared__ int                s_cur;     // thread 0: task of the running sums
   __shared__ unsigned long long s_sum[4];  // thread 0: E4 lo, hi, E5 lo, hi of s_cur not yet added
@@ -656,34 +657,36 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
     for(;;) {
       __syncthreads();
       if(tid == 0) {
-        const unsigned long long t = atomicAdd(&R.qctr[q], 1ull);
-        // progress mirror in host memory (tickets taken so far, approximate)
-        if(R.prog) __hip_atomic_store(&R.prog[q], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         int ti = -1;  // -1: queue exhausted
-        if((long long) t < R.qtotal[q]) {
+        for(;;) {
+          const unsigned long long t = atomicAdd(&R.qctr[q], 1ull);
+          // progress mirror in host memory (tickets taken so far, approximate)
+          if(R.prog) __hip_atomic_store(&R.prog[q], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          if((long long) t >= R.qtotal[q]) break;
           const int e = queue_entry_from(R.qbeg, R.qtick, q, (long long) t, s_entry);
           s_entry     = e;
           ti          = R.qtask[e];
           const TaskDev& T = R.tasks[ti];
-          // ticket -> box: the low bits select the box inside its group
-          int sub[6];
-          if(ticket_box((long long) t - R.qtick[e], T.nsubm, R.glog, sub)) {
+          int            sub[6];
+          const bool     in = ticket_box((long long) t - R.qtick[e], T.nsubm, R.glog, sub);
+          // a copy of another box under the exchange of equal tiles is passed over
+          s_weight = !in ? 0 : R.fold ? fold_weight(T.eq, sub) : 1;
+          ti       = s_weight ? ti : -1;
+          if(ti < 0) continue;
 #pragma unroll
-            for(int p = 0; p < 6; p++) {
-              sm.sub[p]  = sub[p];
-              sm.dim[p]  = T.dim[p];
-              sm.off[p]  = T.off[p];
+          for(int p = 0; p < 6; p++) {
+            sm.sub[p]  = sub[p];
+            sm.dim[p]  = T.dim[p];
+            sm.off[p]  = T.off[p];
               sm.tile[p] = T.tile[p];
-            }
           }
-          else ti = -2;  // a ticket past the task's box grid (its last group overhangs)
+          break;
         }
         s_task = ti;
       }
       __syncthreads();
       const int ti = s_task;
-      if(ti == -1) break;
-      if(ti == -2) continue;
+      if(ti < 0) break;
       if(tid >= 64 && tid < 64 + 18) sm.scale[tid - 64] = M.pscale[18 * (size_t) ti + tid - 64];
       {
         float4* t4 = reinterpret_cast<float4*>(sm.t3);
@@ -707,8 +710,9 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
           sums_flush(R, s_cur, s_sum);
           s_cur = ti;
         }
-        sums_add(R, s_sum, e4, e5);
-        if(R.cost) atomicAdd(&R.cost[ti], wall_clock64() - t0);
+        sums_add(R, s_sum, s_weight * e4, s_weight * e5);
+        // a box's time counts for its copies too, so a task's time follows its extents
+        if(R.cost) atomicAdd(&R.cost[ti], s_weight * (wall_clock64() - t0));
       }
     }
   }

@@ -14,12 +14,13 @@
 
 namespace xt {
 
-// Tickets of a task whose box grid is nbox[0..5] boxes along (h1,h2,h3,p4,p5,p6)
-// under group shape glog: one group of 2^kGroupLog2 tickets per cell of the
-// grid cut into 2^glog[p] boxes along each position.
+// Tickets of a task whose box grid is nbox[0..5] boxes along (h1,h2,h3,p4,p5,p6):
+// one per box (a group of the grid cut into 2^glog[p] boxes along each
+// position has fewer tickets where it overhangs the grid's edge).
 XT_HD inline long long task_ticket_count(const int* nbox, const int* glog) {
-  long long n = 1ll << kGroupLog2;
-  for(int p = 0; p < 6; p++) n *= (nbox[p] + (1 << glog[p]) - 1) >> glog[p];
+  (void) glog;
+  long long n = 1;
+  for(int p = 0; p < 6; p++) n *= nbox[p];
   return n;
 }
 
@@ -59,26 +60,62 @@ XT_HD inline int queue_entry_from(const int* qbeg, const long long* qtick, int q
   return lo;
 }
 
-// Box named by a task's local ticket: the high bits pick the group (mixed
-// radix over the group grid, h1 fastest), the low kGroupLog2 bits the box
-// inside it (glog[0] bits for h1, then glog[1] for h2, ...).  Returns false
-// for a ticket whose box lies outside the grid (groups overhang the grid edge).
-// 32-bit arithmetic: the host runs no task of 2^31 or more tickets.
+// Box named by a task's local ticket, groups of boxes one after the other
+// (h1's group index fastest) and inside a group the boxes with h1 fastest.  An
+// edge group is cut to the grid, so every ticket names a box: with whole
+// groups of 64 a task of few boxes (tiles of one or two boxes) had several
+// times as many tickets as boxes, each with its atomic, its decode and two
+// barriers (O=7, V=22: 100,000 tickets for 12,000 boxes).  Along position p
+// (p6 down to h1) a slab of 2^glog[p] boxes holds L = 2^glog[p] * (boxes of
+// the faster positions) * (this group's extents along the slower ones)
+// tickets, and only the last slab is shorter.  Returns false only for a
+// ticket outside the task.  32-bit arithmetic: the host runs no task of 2^31
+// or more tickets.
 XT_HD inline bool ticket_box(long long local, const int* nbox, const int* glog, int* sub) {
-  unsigned  box   = (unsigned) (local >> kGroupLog2);
-  const int inb   = (int) (local & ((1 << kGroupLog2) - 1));
-  bool      ok    = true;
-  int       shift = 0;
+  unsigned below[7];  // boxes of the positions before p
+  below[0] = 1;
+#pragma unroll
+  for(int p = 0; p < 6; p++) below[p + 1] = below[p] * (unsigned) nbox[p];
+  if(local < 0 || (unsigned long long) local >= below[6]) return false;
+  unsigned rem = (unsigned) local, above = 1, ext[6];
+#pragma unroll
+  for(int p = 5; p >= 0; p--) {
+    const int      gl = glog[p];
+    const unsigned nb = (unsigned) nbox[p], per = below[p] * above;  // tickets per box row
+    const unsigned first = ((rem / per) >> gl) << gl;                // < nb
+    rem -= first * per;
+    ext[p] = nb - first < (1u << gl) ? nb - first : 1u << gl;
+    sub[p] = (int) first;
+    above *= ext[p];
+  }
 #pragma unroll
   for(int p = 0; p < 6; p++) {
-    const int      gl = glog[p];
-    const unsigned nb = (unsigned) ((nbox[p] + (1 << gl) - 1) >> gl);
-    sub[p]            = ((int) (box % nb) << gl) + ((inb >> shift) & ((1 << gl) - 1));
-    box /= nb;
-    shift += gl;
-    ok = ok && sub[p] < nbox[p];
+    const unsigned q = rem / ext[p];
+    sub[p] += (int) (rem - q * ext[p]);
+    rem = q;
   }
-  return ok;
+  return true;
+}
+
+// Antisymmetry of the triples: where two holes (or two particles) of a task
+// lie on the same spin-orbital tile, exchanging them changes only the sign of
+// t3 and of the singles term, so boxes whose positions are a permutation of
+// another's add the same energy.  eq holds bit 0 for h1b = h2b, 1 for
+// h2b = h3b, 2 for p4b = p5b, 3 for p5b = p6b (tiles ascend within each
+// triple, so h1b = h3b implies both).  Returns how many boxes the ascending
+// one stands for (its energy is multiplied by that), 0 for the others, which
+// are skipped.  Summed over a grid the weights give its box count.
+XT_HD inline int fold_triple(int e, int a, int b, int c) {
+  if((e & 1) && a > b) return 0;
+  if((e & 2) && b > c) return 0;
+  if(e == 3) return a == b ? (b == c ? 1 : 3) : (b == c ? 3 : 6);
+  if(e == 1) return a == b ? 1 : 2;
+  if(e == 2) return b == c ? 1 : 2;
+  return 1;
+}
+XT_HD inline int fold_weight(int eq, const int* sub) {
+  return fold_triple(eq & 3, sub[0], sub[1], sub[2]) *
+         fold_triple((eq >> 2) & 3, sub[3], sub[4], sub[5]);
 }
 
 }  // namespace xt
