@@ -58,18 +58,20 @@ struct SpatialBufs {
 // Split FP16 operands of the mixed-precision kernel.  Array j (same order as
 // the FP64 operand arrays: 0 t2h, 1 t2ha, 2 ovk, 3 ovka, 4 xv, 5 xva, 6 t2p,
 // 7 t2pa) holds, for each contraction run (row) r, the values
-// y = x * 2^e[block(r)] split as y ~ hi + lo (FP16 each), stored per 8
-// consecutive k as [hi x8][lo x8]; rows are padded to Kp16 = roundup(K, 16)
-// with zeros.  A block is the set of rows whose three row coordinates fall in
+// y = x * 2^e[block(r)] split as y ~ hi + lo (FP16 each).  K is padded to Kp16
+// = roundup(K, 16) with zeros.  A row's three coordinates are a pair and the
+// coordinate that the kernel's lanes run over (i of t2h[a][b][i] and
+// xv[c][b][i]; a of ovk[i][a][j], whose pair is (i, j), and of t2p[i][j][a]):
+// stored [pair][k / 8][row][hi x8 | lo x8], so that neighbouring rows at one k
+// are one run.  A block is the set of rows whose three row coordinates fall in
 // one (tile, tile, tile) triple of the tiling; its exponent puts the block's
 // largest |y| in [2^13, 2^14) (per-tile amplitude scaling), so the scale of a
 // whole contraction part of a task is one number.
 constexpr int kOperands = 8;
 struct SplitBufs {
-  unsigned char* v[kOperands];     // [rows][Kp16/8][2][8] halves
+  unsigned char* v[kOperands];     // [pair][Kp16/8][row][2][8] halves
   int*           eblk[kOperands];  // [blocks] exponents, row-coordinate tile order
   long           rows[kOperands];
-  unsigned char* zero;             // zero row, 4 * max(Kp16) bytes
   float*         pscale;           // [task][18] contraction part scales (0 for parts off)
   long           pscale_n;         // tasks pscale was built for
 };
@@ -82,7 +84,6 @@ struct MixedDev {
   const double*        vvoo;
   const unsigned char* v[kOperands];
   const int*           eblk[kOperands];
-  const unsigned char* zero;  // zero row (4 * max(Ko, Kv) bytes): rows outside a tile read it
   const float*         pscale;  // [task][18] part scales (build_part_scales)
 };
 

@@ -381,8 +381,6 @@ struct xt_ctx {
       split.v[j] = nullptr;
       split.eblk[j] = nullptr;
     }
-    if(split.zero) (void) hipFree(split.zero);
-    split.zero = nullptr;
     if(split.pscale) (void) hipFree(split.pscale);
     split.pscale   = nullptr;
     split.pscale_n = 0;
@@ -879,7 +877,6 @@ static xt::MixedDev mixed_dev(const xt_ctx* c) {
     M.v[j]    = c->split.v[j];
     M.eblk[j] = c->split.eblk[j];
   }
-  M.zero   = c->split.zero;
   M.pscale = c->split.pscale;
   M.nto    = P.noab / 2;
   M.ntv    = P.nvab / 2;

@@ -3,10 +3,13 @@
 // Same task / bipartition decomposition as the FP64 kernel, with larger
 // workgroup boxes and 16-bit matrix cores:
 //   * a workgroup owns a (4,4,4 | 8,8,8) box of t3[h1,h2,h3,p4,p5,p6]
-//     (32768 elements, FP32 in LDS, never in HBM);
+//     (32768 elements, FP32 in LDS, never in HBM), cut to the task tile at its
+//     edges;
 //   * each bipartition g (single hole hs + particle pair | hole pair +
-//     single particle ps) is a 256 x 128 GEMM: M = (hs,pA,pB) 4*8*8,
-//     N = (hA,hB,ps) 4*4*8, K = h7 (d1) then p7 (d2);
+//     single particle ps) is a GEMM of up to 256 x 128: M = (hs,pA,pB),
+//     N = (ps,hA,hB), K = h7 (d1) then p7 (d2).  Only rows and columns inside
+//     the tile are numbered, so an edge box has fewer 32-row and 32-column
+//     MFMA tiles (wave_tiles);
 //   * operands are pre-split FP16 pairs y = hi + lo of x * 2^e, with one
 //     power-of-two exponent per (tile, tile, tile) block of rows (per-tile
 //     amplitude scaling: the block's max |y| lies in [2^13, 2^14)); every
@@ -15,22 +18,32 @@
 //     task lie in one block per operand, so the part's scale (both exponents
 //     and the spin-orbital signs) is one number, applied when the part ends and
 //     its result is added into the FP32 box;
-//   * eight waves (two per SIMD, so one wave's LDS and VALU work overlaps the
-//     other's MFMAs); wave w owns the 32 M rows of particle pB = w, loaded
-//     from L2/HBM straight into registers in the MFMA operand layout.  The B
-//     panel (shared by all waves) goes through a double-buffered LDS stage.
-//     A register ring keeps PF chunks of loads in flight across part and
-//     bipartition boundaries; every thread issues the same loads for every
-//     chunk (rows outside the tile read a zero row), so the compiler's wait
-//     counts follow the ring; one barrier per K chunk;
-//   * MFMAs are not skipped: rows and columns outside the task tile read the
-//     zero row and add zeros (a branch per MFMA costs more issue time than
-//     the skipped work; a branch per chunk for a wave whose row tile is
-//     outside makes the compiler spill 25 registers);
-//   * the flush into the box adds precomputed per-lane, per-row and
-//     per-column index parts (disjoint bit fields of the box index); the d1
-//     part of a bipartition carries its accumulators into the d2 part, so a
-//     bipartition flushes once;
+//   * eight waves (two per SIMD); in a whole box wave w owns the 32 M rows of
+//     particle pB = w, loaded from L2/HBM straight into registers in the MFMA
+//     operand layout.  The B panel (shared by all waves) goes through a
+//     double-buffered LDS stage.  A register ring keeps PF chunks of loads in
+//     flight across part and bipartition boundaries; every thread issues the
+//     same loads for every chunk, so the compiler's wait counts follow the
+//     ring; one barrier per K chunk;
+//   * what bounds the K loop: the L1 takes one cycle per cache line that a
+//     wave's load touches.  With each row's K run contiguous a load of 32 rows
+//     touched 64 (67 cycles measured, against 18 where four lanes share a
+//     line), 1,200 L1 cycles per 16-k chunk beside 768 of MFMA.  The split
+//     arrays therefore hold the rows of one (x, y) pair side by side per 8 k
+//     (SplitBufs), so that the four hs of a quad of lanes, and the eight ps of
+//     a B column group, are one run.  With that, a wave's own instruction
+//     stream was the next bound (one instruction per four cycles: the loop's
+//     tests, cursor moves and late fragment reads added to the MFMAs instead
+//     of running under them).  Both and the numbering of rows inside the tile:
+//     24 tasks of O=40, V=300 26.8 -> 24.6 ms, 40 uneven tasks of O=48, V=384
+//     124 -> 105.7 ms.  What is left beside the MFMAs of a whole box (about
+//     1,440 cycles per chunk): 240 of loads that hit L1, 200 of L2 misses,
+//     200 of fragment reads, each by timing a build without it;
+//   * the flush into the box adds per-row and per-column offsets from LDS
+//     tables; the box index xors the particle bits into the hole bits (swz) so
+//     that the lanes of every bipartition's flush, and those of the energy
+//     sweeps, fall on 64 distinct banks; the d1 part of a bipartition carries
+//     its accumulators into the d2 part, so a bipartition flushes once;
 //   * energy: one FP64 reciprocal of the denominator per element (from
 //     separable hole and particle sums), E4 in FP64, then t3/D is kept in
 //     place for the s1 sweeps (FP32 products, FP64 sums); task partials are
@@ -47,10 +60,15 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float    f16v __attribute__((ext_vector_type(16)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
+// an operand base read from LDS is a generic pointer to the compiler, whose
+// flat loads would also count as LDS operations
+typedef const __attribute__((address_space(1))) u4v* global_u4;
 
 constexpr int NT  = 512;
-constexpr int NW  = NT / 64;  // waves; wave w owns M rows 32w..32w+31
-constexpr int NN  = 128;      // bipartition columns (hA, hB, ps)
+constexpr int NW  = NT / 64;  // waves
+constexpr int NM  = 256;      // bipartition rows (hs, pA, pB) of a whole box
+constexpr int NN  = 128;      // bipartition columns (ps, hA, hB) of a whole box
 constexpr int KC  = 16;       // K per chunk (one MFMA K step)
 constexpr int BOX = 32768;
 constexpr int PF  = 4;        // ring depth: chunks whose loads are in flight per thread
@@ -58,19 +76,18 @@ constexpr int S1P = 3;        // s1 slots staged per sweep
 // the unrolled ring loop picks stage and fragment buffers by s & 1, which is
 // the chunk's parity only when the ring depth is even
 static_assert(PF % 2 == 0, "ring depth must be even");
-// chunk it is multiplied from ring[it % PF] while chunk it+1's scale and
-// chunk it+2's B piece are read from the next two slots
-static_assert(PF >= 3, "the ring must hold the current chunk and the next two");
+// while chunk it is multiplied from slot it % PF, chunk it+2's B piece is staged
+// and the A loads of chunk it+PF-1 go to another slot
+static_assert(PF >= 4, "the ring must hold the current chunk, the next two and one in flight");
 
 struct __align__(16) MSmem {
   float t3[BOX];
   union {
     struct {
-      uint4 hi[2][2][NN];  // [buffer][k half][column]: FP16 hi of 8 k
-      uint4 lo[2][2][NN];  // FP16 lo of the same 8 k
+      uint4 hi[2][2][NN];  // [buffer][k half][column]: FP16 hi of 8 k (planes 0, 1 of read_frags)
+      uint4 lo[2][2][NN];  // FP16 lo of the same 8 k (planes 2, 3)
     } g;
     struct {
-      double dh[64];   // e_h1 + e_h2 + e_h3 over the box's holes   (index h1 | h2<<2 | h3<<4)
       double dp[512];  // e_p4 + e_p5 + e_p6 over the box's particles (p4 | p5<<3 | p6<<6)
     } d;
     struct {
@@ -78,10 +95,18 @@ struct __align__(16) MSmem {
       float v1[S1P][1088];  // [slot][hk + 4 hj + 16 pc + 128 pb]; p4 slots (hk + 4 hj) * 68 + 8 pc + pb
     } s;
   } u;
+  unsigned short rowt[9][NM];  // box index part of row m of bipartition g
+  unsigned short colt[9][NN];  // box index part of column n
   double eps[36];  // h1,h2,h3 (4 each) at 0,4,8; p4,p5,p6 (8 each) at 12,20,28
   double red[2 * NW];
   float  scale[18];  // scale of each contraction part of the box's task
-  int    sub[6], dim[6], off[6], tile[6];
+  int    start[6];   // first orbital of the box per position
+  int    ext[6];     // orbitals of the box inside the task tile
+  int    rc[9];      // rows | columns << 16 of bipartition g
+  struct {
+    uint64_t a, b;              // addresses of the operand rows of the box's first orbitals
+    unsigned             a1, a2, b1, b2;  // bytes per orbital of pA, pB, hA, hB
+  } part[18];
 };
 
 // bit position of each t3 index in the box layout (2 bits per hole, 3 per particle)
@@ -89,6 +114,17 @@ __host__ __device__ constexpr int sh(int pos) { return pos < 3 ? 2 * pos : 6 + 3
 __host__ __device__ constexpr int ext(int pos) { return pos < 3 ? 4 : 8; }
 __host__ __device__ constexpr int pair_a(int s) { return s == 0 ? 1 : 0; }
 __host__ __device__ constexpr int pair_b(int s) { return s == 2 ? 1 : 2; }
+
+// Storage index of box element e = sum idx << sh: the particle bits are xored
+// into the six hole bits (the LDS bank).  A flush's 64 lanes differ in the
+// three ps bits, two hA bits and the low pA bit; these masks make the six
+// independent for every bipartition (hA is h1 or h2: masks 5 and 10 have a bit
+// in both), and the energy sweeps' lanes differ in the hole bits alone.  The
+// map is linear, so a row's part and a column's part combine by xor.
+__host__ __device__ constexpr int swz(int e) {
+  const int p4 = (e >> 6) & 7, p56 = ((e >> 9) ^ (e >> 12)) & 7, x = p4 ^ p56;
+  return e ^ ((p56 & 1) ? 5 : 0) ^ ((x & 2) ? 10 : 0) ^ ((x & 4) ? 16 : 0) ^ ((p4 & 1) ? 32 : 0);
+}
 
 __device__ __forceinline__ void pair_of(int s, int& a, int& b) {
   a = pair_a(s);
@@ -102,188 +138,258 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 __device__ __forceinline__ h8 as_h8(uint4 u) { return __builtin_bit_cast(h8, u); }
+// The thread index as a value the compiler cannot see through: what a phase
+// derives from it is computed in that phase instead of being held in registers
+// (or spilled) through the others.
+__device__ __forceinline__ int thread_id() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-// One K part of a bipartition as seen by one thread: the A row of its lane
-// (M row 32w + lane%32, k half lane/32), its 16-byte piece of a B column
-// (column tid/4, piece tid%4 = [hi k0-7 | lo k0-7 | hi k8-15 | lo k8-15]) and
-// the part's scale (the same for every thread).  Rows outside the tile read
-// the zero row, so every thread issues the same loads for every chunk and the
-// compiler's wait counts follow the ring.
-struct Part {
-  const unsigned char* pa;
-  const unsigned char* pb;
-  float                sc;  // sign * 2^-(eA + eB)
-  int                  nch;
-};
-
-// One ring slot: the loads of one K chunk plus what its consumers need.
-struct Slot {
-  uint4 a[2];  // hi, lo of this lane's 8 k
-  uint4 b;     // this thread's B piece
-  float sc;    // scale of the chunk's part
-};
-
-// Operand array, row and coefficient of the term c1*x - c2*y of a
-// spin-orbital element (bits bx, by of the part code): both terms -> the
-// antisymmetrised array (holding x - y), one term -> the plain array.
-__host__ __device__ __forceinline__ void choose_term(unsigned c, unsigned bx, unsigned by, int both,
-                                                     int single, int rx, int ry, int& arr, int& row,
-                                                     float& coef) {
-  const bool hx = (c & bx) != 0, hy = (c & by) != 0;
-  arr  = hx && hy ? both : single;
-  row  = hx ? rx : ry;
-  coef = (hx || hy) ? (hx ? 1.f : -1.f) : 0.f;
+// n / e for 0 <= n < 256 and 1 <= e <= 8 (the half keeps the product at least
+// 1/16 from an integer, far beyond the reciprocal's error)
+__device__ __forceinline__ int small_div(int n, int e) {
+  return (int) (((float) n + 0.5f) * __builtin_amdgcn_rcpf((float) e));
+}
+// Coordinates of item n of a (fast a, then b, then c) numbering of extents ea, eb.
+__device__ __forceinline__ void split3(int n, int ea, int eb, int& a, int& b, int& c) {
+  const int t = small_div(n, ea);
+  a           = n - t * ea;
+  c           = small_div(t, eb);
+  b           = t - c * eb;
 }
 
-// Part gp = 2*g + (d2 ? 1 : 0) of bipartition g for this thread; gp = 18 is
-// the zero part that pads the chunk count to a multiple of the ring depth.
-__device__ __forceinline__ Part part_setup(const MSmem& sm, const MixedDev& M, int gp,
-                                           unsigned code) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n = tid >> 2, piece = tid & 3;
-  Part      P;
-  if(gp >= 18) {
-    P.pa  = M.zero + 32 * (lane >> 5);
-    P.pb  = M.zero + 16 * piece;
-    P.sc  = 0.f;
-    P.nch = 1;
-    return P;
-  }
-  const int g = gp >> 1, d2 = gp & 1;
-  const int hs = g / 3, ps = g % 3;
-  int       hA, hB, pA, pB;
+// Operand array and first-term flag of the term c1*x - c2*y of a spin-orbital
+// element (bits bx, by of the part code): both terms -> the antisymmetrised
+// array (holding x - y), one term -> the plain array.
+__host__ __device__ __forceinline__ void choose_term(unsigned c, unsigned bx, unsigned by, int both,
+                                                     int single, int& arr, bool& first, float& coef) {
+  const bool hx = (c & bx) != 0, hy = (c & by) != 0;
+  arr   = hx && hy ? both : single;
+  first = hx;
+  coef  = (hx || hy) ? (hx ? 1.f : -1.f) : 0.f;
+}
+
+// MFMA tiles of one wave in a bipartition of R rows and C columns: row tile
+// rt and column tiles ct .. ct + nj - 1 (32 each).  Five to eight row tiles:
+// one each, all columns.  Up to four (two): two (four) waves share a row tile
+// and split its columns, so that every SIMD has work (waves w and w + 4 share
+// one).
+struct WaveTiles {
+  int nj, rt, ct;
+};
+__device__ __forceinline__ WaveTiles wave_tiles(int rc, int wave) {
+  const int mt = ((rc & 0xffff) + 31) >> 5, nt = ((rc >> 16) + 31) >> 5;
+  const int lg = mt > 4 ? 3 : mt > 2 ? 2 : mt > 1 ? 1 : 0;  // row tiles rounded up to 2^lg
+  const int rt = wave & ((1 << lg) - 1), part = wave >> lg;  // 2^(3-lg) shares of the columns
+  const int per = (nt + (1 << (3 - lg)) - 1) >> (3 - lg);
+  WaveTiles W;
+  W.rt = rt;
+  W.ct = part * per;
+  W.nj = rt < mt ? max(0, min(per, nt - W.ct)) : 0;
+  return W;
+}
+
+// Entry of the box's part table: where the operand rows of part gp start and
+// what the pair coordinates add (a row's neighbour along hs or ps is 32 bytes
+// away).
+__device__ __forceinline__ void part_entry(MSmem& sm, const MixedDev& M, int gp, unsigned code) {
+  const int g = gp >> 1, d2 = gp & 1, hs = g / 3, ps = g % 3;
+  int       hA, hB, pA, pB, arr;
+  bool      first;
+  float     coef;
   pair_of(hs, hA, hB);
   pair_of(ps, pA, pB);
-  const int  O = M.O, V = M.V;      // row indices stay below 2^31 (V*V*O rows at most)
-  const long K = d2 ? M.Kv : M.Ko;  // padded row length (elements)
-  // operand array, row, block and coefficient of c1*x - c2*y (both terms ->
-  // the antisymmetrised array, which holds x - y)
-  P.nch = (int) (K / KC);
-  // the box's tile data of the six positions, read together (one LDS wait);
-  // the row tests below use & so that no read sits behind a branch
-  const int sHS = sm.sub[hs], sPA = sm.sub[3 + pA], sPB = sm.sub[3 + pB];
-  const int sHA = sm.sub[hA], sHB = sm.sub[hB], sPS = sm.sub[3 + ps];
-  const int dHS = sm.dim[hs], dPA = sm.dim[3 + pA], dPB = sm.dim[3 + pB];
-  const int dHA = sm.dim[hA], dHB = sm.dim[hB], dPS = sm.dim[3 + ps];
-  const int oHS = sm.off[hs], oPA = sm.off[3 + pA], oPB = sm.off[3 + pB];
-  const int oHA = sm.off[hA], oHB = sm.off[hB], oPS = sm.off[3 + ps];
-  P.sc          = sm.scale[gp];  // per task, copied to LDS at the box start
-  int   aa, ra, ab, rb;
-  float ca, cb;
+  const long O = M.O, V = M.V, K = d2 ? M.Kv : M.Ko;
   {
-    const int  m   = 32 * wave + (lane & 31);
-    const int  gHS = 4 * sHS + (m & 3), gPA = 8 * sPA + ((m >> 2) & 7), gPB = 8 * sPB + (m >> 5);
-    const bool mok = (gHS < dHS) & (gPA < dPA) & (gPB < dPB);
-    const int  HS = oHS + (mok ? gHS : 0), PA = oPA + (mok ? gPA : 0), PB = oPB + (mok ? gPB : 0);
-    if(!d2)  // t2h[a][b][i]: rows (pA,pB,hs) or (pB,pA,hs)
-      choose_term(code, 4, 8, 1, 0, (PA * V + PB) * O + HS, (PB * V + PA) * O + HS, aa, ra, ca);
-    else  // xv[c][b][i]: rows (pB,pA,hs) or (pA,pB,hs)
-      choose_term(code, 4, 8, 5, 4, (PB * V + PA) * O + HS, (PA * V + PB) * O + HS, aa, ra, ca);
-    P.pa = (mok & (ca != 0.f)) ? M.v[aa] + (long) ra * K * 4 + 32 * (lane >> 5)
-                               : M.zero + 32 * (lane >> 5);
+    // t2h[a][b][i]: pairs (pA,pB) or (pB,pA); xv[c][b][i]: (pB,pA) or (pA,pB); row hs
+    choose_term(code, 4, 8, d2 ? 5 : 1, d2 ? 4 : 0, arr, first, coef);
+    const bool pa_slow = first == (d2 == 0);
+    const long PA = sm.start[3 + pA], PB = sm.start[3 + pB], one = K * O * 4;
+    sm.part[gp].a  = (uint64_t) M.v[arr] + (pa_slow ? PA * V + PB : PB * V + PA) * one + 32l * sm.start[hs];
+    sm.part[gp].a1 = (unsigned) (pa_slow ? V * one : one);
+    sm.part[gp].a2 = (unsigned) (pa_slow ? one : V * one);
   }
   {
-    const int  gHA = 4 * sHA + (n & 3), gHB = 4 * sHB + ((n >> 2) & 3), gPS = 8 * sPS + (n >> 4);
-    const bool nok = (gHA < dHA) & (gHB < dHB) & (gPS < dPS);
-    const int  HA = oHA + (nok ? gHA : 0), HB = oHB + (nok ? gHB : 0), PS = oPS + (nok ? gPS : 0);
-    if(!d2)  // ovk[i][a][j]: rows (hB,ps,hA) or (hA,ps,hB)
-      choose_term(code, 16, 32, 3, 2, (HB * V + PS) * O + HA, (HA * V + PS) * O + HB, ab, rb, cb);
-    else  // t2p[i][j][a]: rows (hA,hB,ps) or (hB,hA,ps)
-      choose_term(code, 16, 32, 7, 6, (HA * O + HB) * V + PS, (HB * O + HA) * V + PS, ab, rb, cb);
-    P.pb = (nok & (cb != 0.f)) ? M.v[ab] + (long) rb * K * 4 + 16 * piece : M.zero + 16 * piece;
+    // ovk: pairs (hB,hA) or (hA,hB); t2p: (hA,hB) or (hB,hA); row ps
+    choose_term(code, 16, 32, d2 ? 7 : 3, d2 ? 6 : 2, arr, first, coef);
+    const bool ha_slow = first == (d2 != 0);
+    const long HA = sm.start[hA], HB = sm.start[hB], one = K * V * 4;
+    sm.part[gp].b  = (uint64_t) M.v[arr] + (ha_slow ? HA * O + HB : HB * O + HA) * one + 32l * sm.start[3 + ps];
+    sm.part[gp].b1 = (unsigned) (ha_slow ? O * one : one);
+    sm.part[gp].b2 = (unsigned) (ha_slow ? one : O * one);
   }
-  return P;
 }
 
-// Issues the loads of chunk ch of part P (always the same three loads).
-__device__ __forceinline__ void fetch(const Part& P, int ch, Slot& s) {
-  const uint4* q = reinterpret_cast<const uint4*>(P.pa + (long) ch * 64);
-  s.a[0]         = q[0];
-  s.a[1]         = q[1];
-  s.b            = *reinterpret_cast<const uint4*>(P.pb + (long) ch * 64);
-  s.sc           = P.sc;
+// This thread's source of one operand in part d2 of bipartition g, as a base
+// shared by the workgroup and a 32-bit offset (the pair strides times seven
+// stay below 2^32 for arrays that fit the device): the A row of its lane (row
+// 32 rt + lane%32, k half lane/32), or its 16-byte piece of a B column (column
+// tid%128, piece tid/128 = [hi k0-7 | lo k0-7 | hi k8-15 | lo k8-15]).  Rows
+// and columns past the last read the last one: their products are never
+// flushed.
+struct Src {
+  uint64_t base;
+  unsigned off;
+  __device__ __forceinline__ global_u4 at() const { return (global_u4) (base + off); }
+};
+__device__ __forceinline__ uint64_t uni64(uint64_t u) {
+  return (uint64_t) (unsigned) uni((int) (u >> 32)) << 32 | (uint64_t) (unsigned) uni((int) (unsigned) u);
+}
+__device__ __forceinline__ Src src_a(const MSmem& sm, const MixedDev& M, int g, int d2) {
+  const int   tid = thread_id(), lane = tid & 63, wave = uni(tid >> 6);
+  const int   hs = g / 3, ps = g % 3, pA = pair_a(ps), pB = pair_b(ps);
+  const auto& E  = sm.part[2 * g + d2];
+  const int   rc = uni(sm.rc[g]);
+  const int   v  = sm.rowt[g][min(32 * wave_tiles(rc, wave).rt + (lane & 31), (rc & 0xffff) - 1)];
+  Src         S;
+  S.base = uni64(E.a);
+  S.off  = ((v >> sh(3 + pA)) & 7) * E.a1 + ((v >> sh(3 + pB)) & 7) * E.a2 +
+          ((swz(v) >> sh(hs)) & 3) * 32u + (unsigned) (lane >> 5) * 32u * (unsigned) M.O;
+  return S;
+}
+__device__ __forceinline__ Src src_b(const MSmem& sm, const MixedDev& M, int g, int d2) {
+  const int   tid = thread_id(), piece = uni(tid >> 7);
+  const int   hs = g / 3, ps = g % 3, hA = pair_a(hs), hB = pair_b(hs);
+  const auto& E = sm.part[2 * g + d2];
+  const int   v = sm.colt[g][min(tid & 127, (uni(sm.rc[g]) >> 16) - 1)], h = swz(v);
+  Src         S;
+  S.base = uni64(E.b);
+  S.off  = ((h >> sh(hA)) & 3) * E.b1 + ((h >> sh(hB)) & 3) * E.b2 + ((v >> sh(3 + ps)) & 7) * 32u +
+          (unsigned) (piece >> 1) * 32u * (unsigned) M.V + 16u * (piece & 1);
+  return S;
 }
 
-// Writes a chunk's B pieces into LDS buffer `buf`.
-__device__ __forceinline__ void stage(MSmem& sm, const Slot& s, int buf) {
-  const int tid = threadIdx.x, n = tid >> 2, piece = tid & 3;
+// Writes a chunk's B piece into LDS buffer `buf` (a wave writes 64 consecutive
+// columns of one plane).
+__device__ __forceinline__ void stage(MSmem& sm, u4v b, int buf) {
+  const int tid = threadIdx.x, n = tid & 127, piece = tid >> 7;
   uint4*    plane = (piece & 1) ? &sm.u.g.lo[buf][piece >> 1][n] : &sm.u.g.hi[buf][piece >> 1][n];
-  *plane          = s.b;
+  *plane          = __builtin_bit_cast(uint4, b);
 }
 
 struct Frags {
   h8 bhi[4], blo[4];
 };
 
-__device__ __forceinline__ void read_frags(const MSmem& sm, int buf, Frags& F) {
-  const int lane = threadIdx.x & 63, kh = lane >> 5;
+// Fragment of one column tile: plane 0, 1 hi of buffer 0, 1; planes 2, 3 lo.
+__device__ __forceinline__ h8 read_frag(const uint4* col, int plane) { return as_h8(col[2 * NN * plane]); }
+
+// acc[j] += ahi bhi[j], then ahi blo[j] (mfma_hi); acc[j] += alo bhi[j]
+// (mfma_lo), for j < nj.  In assembly because of the branch: around builtins
+// the compiler kept a copy of the 64 accumulators per path (up to 691 spilled
+// registers).  The blocks are closed towards the rest of the code: the nops in
+// front cover a vector write of the accumulators before them (flush),
+// acc_ready() a read after them; matrix instructions on the same accumulators
+// need none between them.
+__device__ __forceinline__ void mfma_hi(int nj, h8 a, const h8 (&bh)[4], const h8 (&bl)[4], f16v (&acc)[4]) {
+  asm volatile(
+    "s_nop 1\n\t"
+    "s_cmp_lt_i32 %[nj], 4\n\t"
+    "s_cbranch_scc1 .Lnj3_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c0], %[a], %[h0], %[c0]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c1], %[a], %[h1], %[c1]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c2], %[a], %[h2], %[c2]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c3], %[a], %[h3], %[c3]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c0], %[a], %[l0], %[c0]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c1], %[a], %[l1], %[c1]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c2], %[a], %[l2], %[c2]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c3], %[a], %[l3], %[c3]\n\t"
+    "s_branch .Lnj0_%=\n"
+    ".Lnj3_%=:\n\t"
+    "s_cmp_lt_i32 %[nj], 1\n\t"
+    "s_cbranch_scc1 .Lnj0_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c0], %[a], %[h0], %[c0]\n\t"
+    "s_cmp_lt_i32 %[nj], 2\n\t"
+    "s_cbranch_scc1 .Lnj1_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c1], %[a], %[h1], %[c1]\n\t"
+    "s_cmp_lt_i32 %[nj], 3\n\t"
+    "s_cbranch_scc1 .Lnj2_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c2], %[a], %[h2], %[c2]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c2], %[a], %[l2], %[c2]\n"
+    ".Lnj2_%=:\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c1], %[a], %[l1], %[c1]\n"
+    ".Lnj1_%=:\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c0], %[a], %[l0], %[c0]\n"
+    ".Lnj0_%=:\n"
+    : [c0] "+v"(acc[0]), [c1] "+v"(acc[1]), [c2] "+v"(acc[2]), [c3] "+v"(acc[3])
+    : [nj] "s"(nj), [a] "v"(a), [h0] "v"(bh[0]), [h1] "v"(bh[1]), [h2] "v"(bh[2]), [h3] "v"(bh[3]),
+      [l0] "v"(bl[0]), [l1] "v"(bl[1]), [l2] "v"(bl[2]), [l3] "v"(bl[3])
+    : "scc");
+}
+__device__ __forceinline__ void mfma_lo(int nj, h8 a, const h8 (&bh)[4], f16v (&acc)[4]) {
+  asm volatile(
+    "s_nop 1\n\t"
+    "s_cmp_lt_i32 %[nj], 4\n\t"
+    "s_cbranch_scc1 .Lnj3_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c0], %[a], %[h0], %[c0]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c1], %[a], %[h1], %[c1]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c2], %[a], %[h2], %[c2]\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c3], %[a], %[h3], %[c3]\n\t"
+    "s_branch .Lnj0_%=\n"
+    ".Lnj3_%=:\n\t"
+    "s_cmp_lt_i32 %[nj], 1\n\t"
+    "s_cbranch_scc1 .Lnj0_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c0], %[a], %[h0], %[c0]\n\t"
+    "s_cmp_lt_i32 %[nj], 2\n\t"
+    "s_cbranch_scc1 .Lnj0_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c1], %[a], %[h1], %[c1]\n\t"
+    "s_cmp_lt_i32 %[nj], 3\n\t"
+    "s_cbranch_scc1 .Lnj0_%=\n\t"
+    "v_mfma_f32_32x32x16_f16 %[c2], %[a], %[h2], %[c2]\n"
+    ".Lnj0_%=:\n"
+    : [c0] "+v"(acc[0]), [c1] "+v"(acc[1]), [c2] "+v"(acc[2]), [c3] "+v"(acc[3])
+    : [nj] "s"(nj), [a] "v"(a), [h0] "v"(bh[0]), [h1] "v"(bh[1]), [h2] "v"(bh[2]), [h3] "v"(bh[3])
+    : "scc");
+}
+
+// Waits until vector instructions may read or write the accumulators (19 wait
+// states cover the longest matrix instruction in flight).
+__device__ __forceinline__ void acc_ready(f16v (&acc)[4]) {
+  asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+}
+
+// Adds the scaled accumulators of a bipartition into the box (the first
+// bipartition of a box stores instead) and clears them.  D layout of
+// v_mfma_f32_32x32x16_f16: register q of lane l holds row 8*(q/4) + 4*(l/32)
+// + q%4, column l%32.  Rows and columns past the last have table entries
+// outside the tile (nothing reads those elements).
+__device__ __forceinline__ void flush(MSmem& sm, int g, const WaveTiles& W, float sc, bool store,
+                                      f16v (&acc)[4]) {
+  const int tid = thread_id();
+  const int lane = tid & 63;
+  int       ro[4][4];
+#pragma unroll
+  for(int qq = 0; qq < 4; qq++) {
+    const ushort4 r = *reinterpret_cast<const ushort4*>(&sm.rowt[g][32 * W.rt + 8 * qq + 4 * (lane >> 5)]);
+    ro[qq][0]       = r.x;
+    ro[qq][1]       = r.y;
+    ro[qq][2]       = r.z;
+    ro[qq][3]       = r.w;
+  }
 #pragma unroll
   for(int j = 0; j < 4; j++) {
-    F.bhi[j] = as_h8(sm.u.g.hi[buf][kh][32 * j + (lane & 31)]);
-    F.blo[j] = as_h8(sm.u.g.lo[buf][kh][32 * j + (lane & 31)]);
-  }
-}
-
-// 32x128x16 of this wave: three passes over its 4 accumulators.  Column
-// tiles outside the task tile are not skipped: their B rows are the zero row,
-// and a branch per MFMA costs more issue time than the skipped MFMA.
-__device__ __forceinline__ void mfma_chunk(const Slot& s, const Frags& F, f16v (&acc)[4]) {
-  const h8 ahi = as_h8(s.a[0]), alo = as_h8(s.a[1]);
+    if(j < W.nj) {
+      const int co = sm.colt[g][32 * (W.ct + j) + (lane & 31)];
+      if(store) {
 #pragma unroll
-  for(int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ahi, F.bhi[j], acc[j], 0, 0, 0);
-#pragma unroll
-  for(int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ahi, F.blo[j], acc[j], 0, 0, 0);
-#pragma unroll
-  for(int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(alo, F.bhi[j], acc[j], 0, 0, 0);
-}
-
-// Adds the scaled accumulators of a bipartition with row hole HS into the
-// box and clears them.  D layout of v_mfma_f32_32x32x16_f16: register q of
-// lane l holds row 8*(q/4) + 4*(l/32) + q%4, column l%32.  With
-//   m = 32 wave + 8 (q/4) + 4 (lane/32) + q%4: hs = m & 3, pA = (m >> 2) & 7, pB = m >> 5
-//   n = 32 j + lane%32:                       hA = n & 3, hB = (n >> 2) & 3, ps = n >> 4
-// the t3 index of (q, j) is a per-lane base plus a j part plus a q/4 part plus
-// (q%4) << sh(HS).  For HS = 0 (h1, the fastest t3 index) the four q%4 are
-// consecutive floats and go through one 16-byte LDS read and write.
-template<int HS>
-__device__ __forceinline__ void flush_h(MSmem& sm, int ps, float sc, f16v (&acc)[4]) {
-  constexpr int hA = pair_a(HS), hB = pair_b(HS), shs = sh(HS);
-  const int     pA = pair_a(ps), pB = pair_b(ps);
-  const int     lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int     spa = sh(3 + pA), sps = sh(3 + ps);
-  const int     base = ((lane >> 5) << spa) | (wave << sh(3 + pB)) | ((lane & 3) << sh(hA)) |
-                   (((lane >> 2) & 3) << sh(hB)) | (((lane >> 4) & 1) << sps);
-#pragma unroll
-  for(int qq = 0; qq < 4; qq++)
-#pragma unroll
-    for(int j = 0; j < 4; j++) {
-      const int o = base + ((2 * j) << sps) + ((2 * qq) << spa);
-      if constexpr(HS == 0) {
-        float4* p = reinterpret_cast<float4*>(&sm.t3[o]);  // o is a multiple of 4
-        float4  v = *p;
-        v.x += acc[j][4 * qq + 0] * sc;
-        v.y += acc[j][4 * qq + 1] * sc;
-        v.z += acc[j][4 * qq + 2] * sc;
-        v.w += acc[j][4 * qq + 3] * sc;
-        *p = v;
+        for(int q = 0; q < 16; q++) sm.t3[ro[q >> 2][q & 3] ^ co] = acc[j][q] * sc;
       }
       else {
+        float v[16];
 #pragma unroll
-        for(int r = 0; r < 4; r++) sm.t3[o + (r << shs)] += acc[j][4 * qq + r] * sc;
+        for(int q = 0; q < 16; q++) v[q] = sm.t3[ro[q >> 2][q & 3] ^ co];
+#pragma unroll
+        for(int q = 0; q < 16; q++) sm.t3[ro[q >> 2][q & 3] ^ co] = v[q] + acc[j][q] * sc;
       }
     }
+  }
 #pragma unroll
   for(int j = 0; j < 4; j++)
 #pragma unroll
     for(int q = 0; q < 16; q++) acc[j][q] = 0.f;
-}
-
-__device__ __forceinline__ void flush(MSmem& sm, int g, float sc, f16v (&acc)[4]) {
-  switch(g / 3) {
-    case 0: flush_h<0>(sm, g % 3, sc, acc); break;
-    case 1: flush_h<1>(sm, g % 3, sc, acc); break;
-    default: flush_h<2>(sm, g % 3, sc, acc); break;
-  }
 }
 
 __device__ __forceinline__ bool part_on(uint64_t d1, uint64_t d2, int gp) {
@@ -295,101 +401,194 @@ __device__ __forceinline__ unsigned part_code(uint64_t d1, uint64_t d2, int gp) 
   return (unsigned) (c >> (6 * (gp >> 1))) & 63u;
 }
 
-// Whether this wave's row tile (pB = wave) of bipartition g lies inside the
-// task tile; a wave outside it has only zero rows and skips its flushes.
-__device__ __forceinline__ unsigned tile_mask(const MSmem& sm, int g) {
-  const int ps = g % 3, pB = pair_b(ps), wave = threadIdx.x >> 6;
-  return 8 * sm.sub[3 + pB] + wave < sm.dim[3 + pB] ? 1u : 0u;
+// Row and column tables of the nine bipartitions of a box of extents sm.ext.
+// Padding rows (columns) of the last 32 get an index outside the tile: some
+// extent of their side is short wherever there is one.
+__device__ __forceinline__ void box_tables(MSmem& sm) {
+  for(int x = thread_id(); x < 9 * (NM + NN); x += NT) {
+    const int  g = x / (NM + NN), y = x - g * (NM + NN), hs = g / 3, ps = g % 3;
+    const bool row = y < NM;
+    int        hA, hB, pA, pB;
+    pair_of(hs, hA, hB);
+    pair_of(ps, pA, pB);
+    const int q0 = row ? hs : 3 + ps, q1 = row ? 3 + pA : hA, q2 = row ? 3 + pB : hB;
+    const int e0 = sm.ext[q0], e1 = sm.ext[q1], e2 = sm.ext[q2], n = row ? y : y - NM;
+    int       a, b, c;
+    split3(n, e0, e1, a, b, c);
+    if(c >= e2) {
+      a = e0 < ext(q0) ? e0 : 0;
+      b = e0 < ext(q0) ? 0 : e1 < ext(q1) ? e1 : 0;
+      c = e0 < ext(q0) || e1 < ext(q1) ? 0 : e2 & (ext(q2) - 1);
+    }
+    const int v = swz((a << sh(q0)) | (b << sh(q1)) | (c << sh(q2)));
+    if(row) sm.rowt[g][n] = (unsigned short) v;
+    else sm.colt[g][n] = (unsigned short) v;
+    if(y == 0) sm.rc[g] = e0 * e1 * e2 | (sm.ext[3 + ps] * sm.ext[hA] * sm.ext[hB]) << 16;
+  }
 }
 
 __device__ __forceinline__ void box_contract(MSmem& sm, const MixedDev& M, uint64_t d1, uint64_t d2) {
+  // the d1 and d2 equations of a bipartition are enabled together (both
+  // contract an index of the same spin), n1 chunks of h7 and then n2 of p7
+  unsigned on = 0;
+#pragma unroll
+  for(int g = 0; g < 9; g++) on |= (unsigned) ((d1 >> (6 * g)) & 1) << g;
+  on = uni(on);
+  if(on == 0) {
+    for(int e = threadIdx.x; e < BOX; e += NT) sm.t3[e] = 0.f;
+    return;
+  }
+  const int n1 = M.Ko / KC, n2 = M.Kv / KC, nb = n1 + n2;
+  // chunk count padded to a multiple of the ring depth, so the loop body is
+  // the same for every chunk; the chunks past the end repeat the last loads
+  // and are not flushed
+  const int total_pad = (__builtin_popcount(on) * nb + PF - 1) / PF * PF;
+  const int tid = thread_id(), wave = uni(tid >> 6), lane = tid & 63;
+  const long sa = 64l * M.O, sb = 64l * M.V;  // bytes per chunk
+  auto next = [&](int g) {  // enabled bipartition after g, or 9
+    const unsigned rest = g < 8 ? on >> (g + 1) : 0u;
+    return rest ? g + 1 + __builtin_ctz(rest) : 9;
+  };
   f16v acc[4];
 #pragma unroll
   for(int j = 0; j < 4; j++)
 #pragma unroll
     for(int q = 0; q < 16; q++) acc[j][q] = 0.f;
-  int total = 0, gp0 = -1;
-  for(int gp = 0; gp < 18; gp++)
-    if(part_on(d1, d2, gp)) {
-      total += (gp & 1) ? M.Kv / KC : M.Ko / KC;
-      if(gp0 < 0) gp0 = gp;
-    }
-  if(total == 0) return;
-  // chunk count padded with zero chunks to a multiple of the ring depth, so
-  // the loop body is the same for every chunk
-  const int total_pad = (total + PF - 1) / PF * PF;
-  // fetch cursor (runs PF chunks ahead of the MFMAs); past the last part it
-  // stays on the zero part
-  int  fgp = gp0, fch = 0;
-  Part fp  = part_setup(sm, M, fgp, part_code(d1, d2, fgp));
-  auto fetch_next = [&](Slot& s) {
-    fetch(fp, fch, s);
-    if(++fch == fp.nch) {
-      fch = 0;
-      if(fgp < 18) {
-        do {
-          ++fgp;
-        } while(fgp < 18 && !part_on(d1, d2, fgp));
-        fp = part_setup(sm, M, fgp, fgp < 18 ? part_code(d1, d2, fgp) : 0u);
-      }
-    }
+  const int g0 = __builtin_ctz(on);
+  // load cursors, one per operand: A runs PF - 1 chunks ahead of the MFMAs (a
+  // slot is free once its chunk is multiplied), B runs PF ahead (its slot is
+  // free once its piece is in LDS), so that a piece is loaded two iterations
+  // before it is staged.  Past the last bipartition a cursor repeats its last
+  // chunk.
+  struct Cursor {
+    Src src;
+    int g, d2, left;  // bipartition, part, chunks left in the part
   };
-  Slot ring[PF];
+  auto advance = [&](Cursor& c, bool isa, long step) {
+    if(--c.left) {
+      c.src.base += step;
+      return;
+    }
+    c.d2 ^= 1;
+    if(!c.d2) {
+      const int ng = next(c.g);
+      if(ng == 9) {
+        c.d2   = 1;
+        c.left = 1;
+        return;
+      }
+      c.g = ng;
+    }
+    c.left = c.d2 ? n2 : n1;
+    c.src  = isa ? src_a(sm, M, c.g, c.d2) : src_b(sm, M, c.g, c.d2);
+  };
+  Cursor ca = {src_a(sm, M, g0, 0), g0, 0, n1}, cb = {src_b(sm, M, g0, 0), g0, 0, n1};
+  u4v    ra[PF][2], rb[PF];  // hi, lo of this lane's 8 k; this thread's B piece
+  auto   load_a = [&](u4v(&a)[2]) {
+    a[0] = ca.src.at()[0];
+    a[1] = ca.src.at()[1];
+    advance(ca, true, sa);
+  };
+  auto load_b = [&](u4v& b) {
+    b = *cb.src.at();
+    advance(cb, false, sb);
+  };
 #pragma unroll
-  for(int s = 0; s < PF; s++) fetch_next(ring[s]);
-  // compute cursor
-  int      cgp = gp0, cch = 0, cn = (cgp & 1) ? M.Kv / KC : M.Ko / KC;
-  unsigned cmask = __builtin_amdgcn_readfirstlane(tile_mask(sm, cgp >> 1));
-  Frags    F[2];
+  for(int s = 0; s < PF; s++) {
+    load_b(rb[s]);
+    if(s < PF - 1) load_a(ra[s]);
+  }
+  // compute cursor, and the position of the chunk whose fragments are read next
+  int          cg = g0, cd2 = 0, cleft = n1, rleft = nb;
+  bool         store = true;
+  WaveTiles    W = wave_tiles(uni(sm.rc[cg]), wave);
+  const uint4* col0 = &sm.u.g.hi[0][lane >> 5][lane & 31];
+  const uint4* col[4];
+  auto         set_cols = [&](int ct) {
+#pragma unroll
+    for(int j = 0; j < 4; j++) col[j] = col0 + 32 * ((ct + j) & 3);
+  };
+  set_cols(W.ct);
+  Frags F[2];
   // prologue: chunks 0 and 1 staged, fragments of chunk 0 read
-  __syncthreads();  // previous box's energy sweeps are done with the union area
-  stage(sm, ring[0], 0);
-  stage(sm, ring[1], 1);
+  stage(sm, rb[0], 0);
+  stage(sm, rb[1], 1);
   __syncthreads();
-  read_frags(sm, 0, F[0]);
+#pragma unroll
+  for(int j = 0; j < 4; j++) {
+    F[0].bhi[j] = read_frag(col[j], 0);
+    F[0].blo[j] = read_frag(col[j], 2);
+  }
   __syncthreads();
-  // iteration it (chunk it: A in ring[it % PF], B fragments in F[it & 1]):
-  //   read fragments of chunk it+1 (buffer (it+1)&1) while the MFMAs of
-  //   chunk it run, stage chunk it+2 into buffer it&1 (its fragments were
-  //   read before the previous barrier), flush at the end of a part, refill
-  //   ring[it % PF] with chunk it+PF, barrier.
+  // iteration it (chunk it: A in ra[it % PF], B fragments in F[it & 1]): stage
+  // chunk it+2 into buffer it&1 (its fragments were read before the previous
+  // barrier), read the fragments of chunk it+1 (buffer (it+1)&1) and issue the
+  // loads into the slots that became free, around the twelve MFMAs; flush at
+  // the end of a bipartition; one barrier.  A wave issues one instruction per
+  // four cycles and two waves share a SIMD, so beside 768 cycles of MFMA the
+  // loop has room for few others: the cursors count down to their next part,
+  // and everything else about a part sits behind those four tests (the tests
+  // and cursor moves took 62 scalar instructions and 25 branches a chunk).
 #pragma unroll 1
   for(int it0 = 0; it0 < total_pad; it0 += PF) {
 #pragma unroll
     for(int s = 0; s < PF; s++) {
-      read_frags(sm, (s + 1) & 1, F[(s + 1) & 1]);
-      mfma_chunk(ring[s], F[s & 1], acc);
-      stage(sm, ring[(s + 2) % PF], s & 1);
-      if(++cch == cn) {
-        int ngp = cgp;
-        do {
-          ++ngp;
-        } while(ngp < 18 && !part_on(d1, d2, ngp));
-        // A d1 part followed by the d2 part of the same bipartition adds into
-        // the same box elements: its accumulators carry over, rescaled by the
-        // ratio of the two part scales (both +-2^k, so the ratio is exact;
-        // the next chunk, first of the d2 part, holds the d2 scale).  Ratios
-        // outside 2^+-60 flush instead, keeping the FP32 range.
-        bool carry = false;
-        if(!(cgp & 1) && ngp == cgp + 1) {
-          const float r = ring[s].sc / ring[(s + 1) % PF].sc;
-          carry         = fabsf(r) >= 0x1p-60f && fabsf(r) <= 0x1p60f;
+      if(--rleft == 0) {
+        rleft        = nb;
+        const int ng = next(cg);
+        set_cols(wave_tiles(uni(sm.rc[ng < 9 ? ng : cg]), wave).ct);
+      }
+      Frags &Fc = F[s & 1], &Fn = F[(s + 1) & 1];
+      const h8 ahi = __builtin_bit_cast(h8, ra[s][0]), alo = __builtin_bit_cast(h8, ra[s][1]);
+      stage(sm, rb[(s + 2) % PF], s & 1);
+#pragma unroll
+      for(int j = 0; j < 4; j++) Fn.bhi[j] = read_frag(col[j], (s + 1) & 1);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma_hi(W.nj, ahi, Fc.bhi, Fc.blo, acc);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for(int j = 0; j < 4; j++) Fn.blo[j] = read_frag(col[j], 2 + ((s + 1) & 1));
+      load_b(rb[s]);
+      load_a(ra[(s + PF - 1) % PF]);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma_lo(W.nj, alo, Fc.bhi, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      if(--cleft == 0) {
+        // The d1 part of a bipartition carries its accumulators into the d2
+        // part (the same box elements), rescaled by the ratio of the two part
+        // scales (both +-2^k, so the ratio is exact).  Ratios outside 2^+-60
+        // flush instead, keeping the FP32 range.
+        const float sc    = sm.scale[2 * cg + cd2];
+        bool        carry = false;
+        acc_ready(acc);
+        if(!cd2) {
+          const float r = sc / sm.scale[2 * cg + 1];
+          carry         = uni(fabsf(r) >= 0x1p-60f && fabsf(r) <= 0x1p60f);
           if(carry)
 #pragma unroll
             for(int j = 0; j < 4; j++)
 #pragma unroll
               for(int q = 0; q < 16; q++) acc[j][q] *= r;
         }
-        if(!carry && cmask) flush(sm, cgp >> 1, ring[s].sc, acc);
-        cch = 0;
-        cgp = ngp;
-        cn    = cgp < 18 ? ((cgp & 1) ? M.Kv / KC : M.Ko / KC) : 0x7fffffff;
-        cmask = __builtin_amdgcn_readfirstlane(cgp < 18 ? tile_mask(sm, cgp >> 1) : 0u);
+        if(!carry) {
+          flush(sm, cg, W, sc, store, acc);
+          store = false;
+        }
+        cd2 ^= 1;
+        cleft = n2;
+        if(!cd2) {
+          const int ng = next(cg);
+          cleft        = ng < 9 ? n1 : total_pad;  // past the last one only padding chunks are left
+          if(ng < 9) {
+            cg = ng;
+            W  = wave_tiles(uni(sm.rc[cg]), wave);
+          }
+        }
       }
-      fetch_next(ring[s]);
       __syncthreads();
     }
   }
+  acc_ready(acc);  // the padding chunks' instructions are done with the registers
 }
 
 // Denominator reciprocal in FP64: hardware estimate refined by two Newton
@@ -403,21 +602,22 @@ __device__ __forceinline__ double recip(double d) {
 }
 
 // s1 term of S1P slots starting at S0, staged in LDS: returns this thread's
-// sum over its elements of (t3/D) * s.  W = t3/D is already in sm.t3 (zero
-// outside the tile), T1 and V blocks are zero outside the tile.
+// sum over its elements of (t3/D) * s.  W = t3/D is already in sm.t3 for the
+// threads inside the tile (zero where p5 is outside), T1 and V blocks are zero
+// outside the tile.
 //
-// The thread's elements e = tid + NT*rr are every (p5, p6) = (rr & 7, rr >> 3)
-// for its own (h1, h2, h3, p4) (the bits of tid), and the slots of one sweep
-// share their particle position pa = S0/3.  So a sweep needs one T1 value and
+// The thread's elements are every (p5, p6) for its own (h1, h2, h3, p4) (the
+// bits of tid; tb is their storage index), and the slots of one sweep share
+// their particle position pa = S0/3.  So a sweep needs one T1 value and
 // 64 V values per slot (pa = p4), or 8 and 8 (pa = p5, p6): each is read from
 // LDS once instead of once per element.  Per element the slots are summed in
 // FP32 in slot order and the products W*s added in FP64 in element order, as
 // an element-by-element loop would.
 template<int S0>
-__device__ __forceinline__ double s1_sweep(const MSmem& sm) {
+__device__ __forceinline__ double s1_sweep(const MSmem& sm, int tb, int n6) {
   static_assert(S0 % 3 == 0 && S1P == 3, "a sweep covers the three slots of one pa");
   constexpr int pa = S0 / 3;
-  const int     tid = threadIdx.x;
+  const int     tid = thread_id();
   const int     hidx[3] = {tid & 3, (tid >> 2) & 3, (tid >> 4) & 3};
   const int     p4 = (tid >> 6) & 7;
   int           vb[S1P], th[S1P];  // per slot: h part of the V index, T1 hole index
@@ -437,8 +637,9 @@ __device__ __forceinline__ double s1_sweep(const MSmem& sm) {
     // these slots are stored with pb (= p5) contiguous: the 8 values of one p6
     // are two 16-byte reads
 #pragma unroll 1
-    for(int p6 = 0; p6 < 8; p6++) {
-      float4 v[S1P][2];
+    for(int p6 = 0; p6 < n6; p6++) {
+      const int tp = tb ^ swz(p6 << 12);
+      float4    v[S1P][2];
 #pragma unroll
       for(int q = 0; q < S1P; q++) {
         const float4* r = reinterpret_cast<const float4*>(&sm.u.s.v1[q][vb[q] * 68 + 8 * p6]);
@@ -454,7 +655,7 @@ __device__ __forceinline__ double s1_sweep(const MSmem& sm) {
           const int    i = p5 & 3;
           sv += t[q] * (i == 0 ? h.x : i == 1 ? h.y : i == 2 ? h.z : h.w);
         }
-        es += (double) (sm.t3[tid + NT * (p5 + 8 * p6)] * sv);
+        es += (double) (sm.t3[tp ^ swz(p5 << 9)] * sv);
       }
     }
   }
@@ -469,8 +670,9 @@ __device__ __forceinline__ double s1_sweep(const MSmem& sm) {
       for(int k = 0; k < 8; k++)
         hold[q][k] = pa == 1 ? sm.u.s.t1[q][k * 4 + th[q]] : sm.u.s.v1[q][vb[q] + 16 * k + 128 * p4];
 #pragma unroll 1
-    for(int p6 = 0; p6 < 8; p6++) {
-      float per[S1P];
+    for(int p6 = 0; p6 < n6; p6++) {
+      const int tp = tb ^ swz(p6 << 12);
+      float     per[S1P];
 #pragma unroll
       for(int q = 0; q < S1P; q++)
         per[q] = pa == 1 ? sm.u.s.v1[q][vb[q] + 16 * p6 + 128 * p4] : sm.u.s.t1[q][p6 * 4 + th[q]];
@@ -479,7 +681,7 @@ __device__ __forceinline__ double s1_sweep(const MSmem& sm) {
         float sv = 0.f;
 #pragma unroll
         for(int q = 0; q < S1P; q++) sv += pa == 1 ? hold[q][p5] * per[q] : per[q] * hold[q][p5];
-        es += (double) (sm.t3[tid + NT * (p5 + 8 * p6)] * sv);
+        es += (double) (sm.t3[tp ^ swz(p5 << 9)] * sv);
       }
     }
   }
@@ -498,7 +700,7 @@ struct S1Regs {
 template<int S0>
 __device__ __forceinline__ void s1_load(const MSmem& sm, const MixedDev& M, uint64_t s1code,
                                         S1Regs& R) {
-  const int  tid = threadIdx.x;
+  const int  tid = thread_id();
   const long O = M.O, V = M.V;
 #pragma unroll
   for(int q = 0; q < S1P; q++) {
@@ -514,20 +716,19 @@ __device__ __forceinline__ void s1_load(const MSmem& sm, const MixedDev& M, uint
     pair_of(pa, pb, pc);
     if(!(c & 1)) continue;
     if(tid < 32) {
-      const int gp = 8 * sm.sub[3 + pa] + (tid >> 2), gh = 4 * sm.sub[hi] + (tid & 3);
-      if(gp < sm.dim[3 + pa] && gh < sm.dim[hi]) {
-        const double t = M.t1[(long) (sm.off[3 + pa] + gp) * O + sm.off[hi] + gh];
+      const int gp = tid >> 2, gh = tid & 3;
+      if(gp < sm.ext[3 + pa] && gh < sm.ext[hi]) {
+        const double t = M.t1[(long) (sm.start[3 + pa] + gp) * O + sm.start[hi] + gh];
         R.t[q]         = (c & 2) ? -t : t;
       }
     }
 #pragma unroll
     for(int j = 0; j < S1V; j++) {
       const int w  = tid + NT * j;
-      const int gj = 4 * sm.sub[hj] + (w & 3), gk = 4 * sm.sub[hk] + ((w >> 2) & 3),
-                gc = 8 * sm.sub[3 + pc] + ((w >> 4) & 7), gb = 8 * sm.sub[3 + pb] + (w >> 7);
-      if(gk < sm.dim[hk] && gj < sm.dim[hj] && gc < sm.dim[3 + pc] && gb < sm.dim[3 + pb]) {
-        const long K = sm.off[hk] + gk, J = sm.off[hj] + gj, PC = sm.off[3 + pc] + gc,
-                   PB = sm.off[3 + pb] + gb;
+      const int gj = w & 3, gk = (w >> 2) & 3, gc = (w >> 4) & 7, gb = w >> 7;
+      if(gk < sm.ext[hk] && gj < sm.ext[hj] && gc < sm.ext[3 + pc] && gb < sm.ext[3 + pb]) {
+        const long K = sm.start[hk] + gk, J = sm.start[hj] + gj, PC = sm.start[3 + pc] + gc,
+                   PB = sm.start[3 + pb] + gb;
         double x = 0.0;
         if(c & 4) x = M.vvoo[((PC * V + PB) * O + K) * O + J];
         if(c & 8) x -= M.vvoo[((PB * V + PC) * O + K) * O + J];
@@ -542,7 +743,7 @@ __device__ __forceinline__ void s1_load(const MSmem& sm, const MixedDev& M, uint
 // 68 rather than 64 keeps the stores of a wave on distinct banks but for pairs.
 template<int S0>
 __device__ __forceinline__ void s1_store(MSmem& sm, const S1Regs& R) {
-  const int tid = threadIdx.x;
+  const int tid = thread_id();
 #pragma unroll
   for(int q = 0; q < S1P; q++) {
     if(tid < 32) sm.u.s.t1[q][tid] = (float) R.t[q];
@@ -560,54 +761,52 @@ __device__ __forceinline__ void s1_store(MSmem& sm, const S1Regs& R) {
 // elements of the box (FP64 sums of per-element terms; t3 and s in FP32).
 __device__ __forceinline__ void box_energy(MSmem& sm, const MixedDev& M, uint64_t s1code, double& e4,
                            double& e5) {
-  const int tid = threadIdx.x;
+  const int tid = thread_id();
   S1Regs    R;
   s1_load<0>(sm, M, s1code, R);  // in flight during the E4 sweep
   // separable denominators, in the order of the reference's sum
-  for(int x = tid; x < 64 + 512; x += NT) {
-    if(x < 64) sm.u.d.dh[x] = (sm.eps[8 + (x >> 4)] + sm.eps[4 + ((x >> 2) & 3)]) + sm.eps[x & 3];
-    else {
-      const int y    = x - 64;
-      sm.u.d.dp[y] = (sm.eps[28 + (y >> 6)] + sm.eps[20 + ((y >> 3) & 7)]) + sm.eps[12 + (y & 7)];
-    }
-  }
+  for(int y = tid; y < 512; y += NT)
+    sm.u.d.dp[y] = (sm.eps[28 + (y >> 6)] + sm.eps[20 + ((y >> 3) & 7)]) + sm.eps[12 + (y & 7)];
   __syncthreads();
-  int lim[6];
+  const int    h1 = tid & 3, h2 = (tid >> 2) & 3, h3 = (tid >> 4) & 3, p4 = tid >> 6;
+  const int    n5 = uni(sm.ext[4]), n6 = uni(sm.ext[5]), tb = swz(tid);
+  const double dh = (sm.eps[8 + h3] + sm.eps[4 + h2]) + sm.eps[h1];
+  const bool   in = h1 < sm.ext[0] && h2 < sm.ext[1] && h3 < sm.ext[2] && p4 < sm.ext[3];
+  e4              = 0.0;
+  auto elem       = [&](int at, int y) {
+    const double d  = (double) sm.t3[at];
+    const double di = d * recip(dh - sm.u.d.dp[y]);
+    e4 += d * di;
+    sm.t3[at] = (float) di;
+  };
+  if(in)
+    for(int p6 = 0; p6 < n6; p6++) {
+      const int tp = tb ^ swz(p6 << 12), y = p4 + 64 * p6;
+      if(n5 == 8) {
 #pragma unroll
-  for(int p = 0; p < 6; p++) lim[p] = sm.dim[p] - ext(p) * sm.sub[p];
-  e4 = 0.0;
-#pragma unroll 2
-  for(int rr = 0; rr < BOX / NT; rr++) {
-    const int e  = tid + NT * rr;
-    bool      ok = true;
-#pragma unroll
-    for(int p = 0; p < 6; p++) ok = ok && ((e >> sh(p)) & (ext(p) - 1)) < lim[p];
-    float w = 0.f;
-    if(ok) {
-      const double d   = (double) sm.t3[e];
-      const double inv = recip(sm.u.d.dh[e & 63] - sm.u.d.dp[e >> 6]);
-      const double di  = d * inv;
-      e4 += d * di;
-      w = (float) di;
+        for(int p5 = 0; p5 < 8; p5++) elem(tp ^ swz(p5 << 9), y + 8 * p5);
+      }
+      else {
+        for(int p5 = 0; p5 < n5; p5++) elem(tp ^ swz(p5 << 9), y + 8 * p5);
+        for(int p5 = n5; p5 < 8; p5++) sm.t3[tp ^ swz(p5 << 9)] = 0.f;
+      }
     }
-    sm.t3[e] = w;
-  }
   double es = 0.0;
   if(s1code & 0x111111111ull) {
     __syncthreads();  // denominators no longer needed; W complete
     s1_store<0>(sm, R);
     s1_load<S1P>(sm, M, s1code, R);
     __syncthreads();
-    es += s1_sweep<0>(sm);
+    if(in) es += s1_sweep<0>(sm, tb, n6);
     __syncthreads();
     s1_store<S1P>(sm, R);
     s1_load<2 * S1P>(sm, M, s1code, R);
     __syncthreads();
-    es += s1_sweep<S1P>(sm);
+    if(in) es += s1_sweep<S1P>(sm, tb, n6);
     __syncthreads();
     s1_store<2 * S1P>(sm, R);
     __syncthreads();
-    es += s1_sweep<2 * S1P>(sm);
+    if(in) es += s1_sweep<2 * S1P>(sm, tb, n6);
   }
   e5                  = e4 + es;
   const int lane = tid & 63, wave = tid >> 6;
@@ -639,6 +838,7 @@ __device__ __forceinline__ void box_energy(MSmem& sm, const MixedDev& M, uint64_
 __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
   __shared__ MSmem              sm;
   __shared__ int                s_task;
+  __shared__ int                s_retable; // thread 0: the box's extents differ from the last one's
   __shared__ int                s_weight;  // thread 0: boxes that its box stands for
   __shared__ int                s_entry;   // thread 0: entry of its last ticket on the current queue
   __shared__ int                s_cur;     // thread 0: task of the running sums
@@ -648,6 +848,8 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
   if(tid == 0) {
     s_cur    = -1;
     s_sum[0] = s_sum[1] = s_sum[2] = s_sum[3] = 0ull;
+#pragma unroll
+    for(int p = 0; p < 6; p++) sm.ext[p] = 0;
   }
 #pragma unroll 1
   for(int qi = 0; qi < kQueues; qi++) {
@@ -657,7 +859,8 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
     for(;;) {
       __syncthreads();
       if(tid == 0) {
-        int ti = -1;  // -1: queue exhausted
+        int ti    = -1;  // -1: queue exhausted
+        s_retable = 0;
         for(;;) {
           const unsigned long long t = atomicAdd(&R.qctr[q], 1ull);
           // progress mirror in host memory (tickets taken so far, approximate)
@@ -675,10 +878,10 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
           if(ti < 0) continue;
 #pragma unroll
           for(int p = 0; p < 6; p++) {
-            sm.sub[p]  = sub[p];
-            sm.dim[p]  = T.dim[p];
-            sm.off[p]  = T.off[p];
-              sm.tile[p] = T.tile[p];
+            const int x = min(ext(p), T.dim[p] - ext(p) * sub[p]);
+            if(x != sm.ext[p]) s_retable = 1;
+            sm.start[p] = T.off[p] + ext(p) * sub[p];
+            sm.ext[p]   = x;
           }
           break;
         }
@@ -688,15 +891,15 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
       const int ti = s_task;
       if(ti < 0) break;
       if(tid >= 64 && tid < 64 + 18) sm.scale[tid - 64] = M.pscale[18 * (size_t) ti + tid - 64];
-      {
-        float4* t4 = reinterpret_cast<float4*>(sm.t3);
-        for(int e = tid; e < BOX / 4; e += NT) t4[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if(s_retable) box_tables(sm);
+      if(tid >= 128 && tid < 128 + 18) {
+        const TaskDev& T = R.tasks[ti];
+        part_entry(sm, M, tid - 128, part_code(T.d1code, T.d2code, tid - 128));
       }
       if(tid < 36) {
         const int p = tid < 12 ? tid / 4 : 3 + (tid - 12) / 8;
         const int i = tid < 12 ? tid % 4 : (tid - 12) % 8;
-        const int g = ext(p) * sm.sub[p] + i;
-        sm.eps[tid] = g < sm.dim[p] ? (p < 3 ? M.eo : M.ev)[sm.off[p] + g] : 0.0;
+        sm.eps[tid] = i < sm.ext[p] ? (p < 3 ? M.eo : M.ev)[sm.start[p] + i] : 0.0;
       }
       __syncthreads();
       const TaskDev&           T  = R.tasks[ti];
@@ -767,18 +970,27 @@ __global__ void k_block_exp(const short* __restrict__ er, long rows, BlockMap bm
   if(e < kNoRow) atomicMin(&eb[bm(r)], e);
 }
 
-// Split: y = x * 2^e[block(row)] = hi + lo (FP16), written per 8 k as [hi8][lo8].
-__global__ void k_split(const double* __restrict__ x, long rows, long Kin, long Kout, BlockMap bm,
-                        const int* __restrict__ eb, _Float16* __restrict__ out) {
-  const long n = rows * Kout;
+// Split: y = x * 2^e[block(row)] = hi + lo (FP16), in the order of SplitBufs:
+// one thread per 8 k of a row, neighbouring threads on neighbouring rows of a
+// pair, so that a wave writes one run of 2 KB and reads 64-byte runs.  `mid`:
+// the pair is (x, z) and the row y (the ovk arrays), else (x, y) and z.
+__global__ void __launch_bounds__(256) k_split(const double* __restrict__ x, long rows, long Kin,
+                                               long Kout, BlockMap bm, int mid,
+                                               const int* __restrict__ eb, uint4* __restrict__ out) {
+  const long R = mid ? bm.D2 : bm.D3, k8 = Kout / 8, n = rows * k8;
   for(long i = (long) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long) gridDim.x * blockDim.x) {
-    const long     row  = i / Kout, k = i % Kout;
-    const double   y    = k < Kin ? ldexp(x[row * Kin + k], eb[bm(row)]) : 0.0;
-    const _Float16 h    = (_Float16) y;
-    const _Float16 l    = (_Float16) (y - (double) h);
-    const long     base = row * Kout * 2 + (k / 8) * 16 + (k % 8);
-    out[base]           = h;
-    out[base + 8]       = l;
+    const long q = i / R, r = i - q * R, pair = q / k8, k = 8 * (q - pair * k8);
+    const long row = mid ? ((pair / bm.D3) * bm.D2 + r) * bm.D3 + pair % bm.D3 : pair * R + r;
+    const int  e   = eb[bm(row)];
+    h8         hi, lo;
+#pragma unroll
+    for(int j = 0; j < 8; j++) {
+      const double y = k + j < Kin ? ldexp(x[row * Kin + k + j], e) : 0.0;
+      hi[j]          = (_Float16) y;
+      lo[j]          = (_Float16) (y - (double) hi[j]);
+    }
+    out[2 * i]     = __builtin_bit_cast(uint4, hi);
+    out[2 * i + 1] = __builtin_bit_cast(uint4, lo);
   }
 }
 
@@ -802,14 +1014,19 @@ __global__ void k_part_scales(const TaskDev* __restrict__ tasks, int n_tasks, Mi
   const int      tHS = T.tile[hs], tHA = T.tile[hA], tHB = T.tile[hB];
   const int      tPS = T.tile[3 + ps], tPA = T.tile[3 + pA], tPB = T.tile[3 + pB];
   int            aa, ka, ab, kb;
+  bool           fa, fb;
   float          ca, cb;
   if(!d2) {  // t2h blocks (V,V,O): (pA,pB,hs) / (pB,pA,hs); ovk (O,V,O): (hB,ps,hA) / (hA,ps,hB)
-    choose_term(code, 4, 8, 1, 0, (tPA * nv + tPB) * no + tHS, (tPB * nv + tPA) * no + tHS, aa, ka, ca);
-    choose_term(code, 16, 32, 3, 2, (tHB * nv + tPS) * no + tHA, (tHA * nv + tPS) * no + tHB, ab, kb, cb);
+    choose_term(code, 4, 8, 1, 0, aa, fa, ca);
+    ka = ((fa ? tPA : tPB) * nv + (fa ? tPB : tPA)) * no + tHS;
+    choose_term(code, 16, 32, 3, 2, ab, fb, cb);
+    kb = ((fb ? tHB : tHA) * nv + tPS) * no + (fb ? tHA : tHB);
   }
   else {  // xv blocks (V,V,O): (pB,pA,hs) / (pA,pB,hs); t2p (O,O,V): (hA,hB,ps) / (hB,hA,ps)
-    choose_term(code, 4, 8, 5, 4, (tPB * nv + tPA) * no + tHS, (tPA * nv + tPB) * no + tHS, aa, ka, ca);
-    choose_term(code, 16, 32, 7, 6, (tHA * no + tHB) * nv + tPS, (tHB * no + tHA) * nv + tPS, ab, kb, cb);
+    choose_term(code, 4, 8, 5, 4, aa, fa, ca);
+    ka = ((fa ? tPB : tPA) * nv + (fa ? tPA : tPB)) * no + tHS;
+    choose_term(code, 16, 32, 7, 6, ab, fb, cb);
+    kb = ((fb ? tHA : tHB) * no + (fb ? tHB : tHA)) * nv + tPS;
   }
   const float sg = (code & 2) ? -1.f : 1.f;
   out[i]         = sg * ca * cb * ldexpf(1.f, -(M.eblk[aa][ka] + M.eblk[ab][kb]));
@@ -848,11 +1065,6 @@ int build_split(const SpatialBufs& B, int O, int V, const int* tile_o, int nto, 
   if((err = hipMemcpyAsync(dto, tile_o, sizeof(int) * o, hipMemcpyHostToDevice, st)) ||
      (err = hipMemcpyAsync(dtv, tile_v, sizeof(int) * v, hipMemcpyHostToDevice, st)))
     return done(err);
-  {
-    const size_t zb = 4 * (size_t) (ko > kv ? ko : kv);
-    if((err = hipMalloc((void**) &S.zero, zb))) return done(err);
-    if((err = hipMemsetAsync(S.zero, 0, zb, st))) return done(err);
-  }
   const long rows_max = v * v * o > o * o * v ? v * v * o : o * o * v;
   // k_row_exp runs one wave per row: 64 * rows work-items in one dispatch
   if(rows_max * 64 > (long) UINT32_MAX) return done(hipErrorInvalidConfiguration);
@@ -883,9 +1095,9 @@ int build_split(const SpatialBufs& B, int O, int V, const int* tile_o, int nto, 
     hipLaunchKernelGGL(k_block_exp, dim3((unsigned) ((rows + 255) / 256)), dim3(256), 0, st, er,
                        rows, bm, S.eblk[j]);
     // grid-stride: a dispatch's grid size is a 32-bit count of work-items
-    const long n = rows * kout;
+    const long n = rows * (kout / 8);
     hipLaunchKernelGGL(k_split, dim3((unsigned) std::min<long>((n + 255) / 256, 1l << 20)), dim3(256), 0, st, src[j], rows,
-                       kin, kout, bm, S.eblk[j], reinterpret_cast<_Float16*>(S.v[j]));
+                       kin, kout, bm, j == 2 || j == 3, S.eblk[j], reinterpret_cast<uint4*>(S.v[j]));
     if((err = hipGetLastError())) return done(err);
   }
   return done(hipStreamSynchronize(st));
