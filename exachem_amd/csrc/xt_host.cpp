@@ -308,10 +308,13 @@ struct xt_ctx {
   // tickets it takes, the host reads them while the persistent kernel runs
   unsigned long long* h_prog = nullptr;
   unsigned long long* d_prog = nullptr;
+  // largest asymmetry and element of the uploaded vvoo (queue_fold_check)
+  unsigned long long* d_asym = nullptr;
+  double*             h_asym = nullptr;
   int         n_cu   = 0;
   Plan        plan;
   bool        have_plan = false, have_inputs = false;
-  bool        fold = false;  // the inputs let boxes of equal tiles be folded (set_fold)
+  bool        fold = false;  // the inputs let boxes of equal tiles be folded (fold_allowed)
   // device inputs (kernel layouts)
   xt::SpatialBufs in    = {};
   xt::SplitBufs   split = {};  // FP16 split operands (built on the first mixed run)
@@ -440,6 +443,8 @@ int xt_create(int device, xt_ctx** out) {
   XT_HIP(hipHostMalloc((void**) &c->h_prog, sizeof(unsigned long long) * xt::kQueues,
                        hipHostMallocMapped | hipHostMallocCoherent));
   XT_HIP(hipHostGetDevicePointer((void**) &c->d_prog, c->h_prog, 0));
+  XT_HIP(hipHostMalloc((void**) &c->h_asym, 2 * sizeof(double), hipHostMallocDefault));
+  XT_HIP(hipMalloc((void**) &c->d_asym, 2 * sizeof(unsigned long long)));
   XT_HIP(hipEventCreate(&c->ev0));
   XT_HIP(hipEventCreate(&c->ev1));
   *out = c;
@@ -460,6 +465,8 @@ int xt_destroy(xt_ctx* c) {
   if(c->ev1) (void) hipEventDestroy(c->ev1);
   if(c->stream) (void) hipStreamDestroy(c->stream);
   if(c->h_prog) (void) hipHostFree(c->h_prog);
+  if(c->h_asym) (void) hipHostFree(c->h_asym);
+  if(c->d_asym) (void) hipFree(c->d_asym);
   if(c->d_gather) (void) hipFree(c->d_gather);
   delete c;
   return XT_OK;
@@ -684,12 +691,15 @@ extern "C" {
 // asks for.  Integrals that miss it by more than their own rounding (1e-13 of
 // the largest; products over Cholesky vectors miss it by a few 1e-16) are run
 // over every box.
-static int set_fold(xt_ctx* c) {
-  double    diff = 0.0, largest = 0.0;
-  const int err = xt::vvoo_asymmetry(c->in.vvoo, c->plan.O, c->plan.V, &diff, &largest, c->stream);
-  c->fold       = !err && diff <= 1e-13 * largest;
+// Queued once vvoo is on the device; fold_allowed reads the two maxima after
+// the upload's own wait for the stream.
+static int queue_fold_check(xt_ctx* c) {
+  int err = xt::launch_vvoo_asym(c->in.vvoo, c->plan.O, c->plan.V, c->d_asym, c->stream);
+  if(!err)
+    err = (int) hipMemcpyAsync(c->h_asym, c->d_asym, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
   return err;
 }
+static bool fold_allowed(const xt_ctx* c) { return c->h_asym[0] <= 1e-13 * c->h_asym[1]; }
 
 static int upload_common(xt_ctx* c, const double* eo, const double* ev, const double* t1,
                          const double* t2, const double* vvoo, const double* ovoo,
@@ -729,8 +739,8 @@ static int upload_common(xt_ctx* c, const double* eo, const double* ev, const do
     cleanup();
     return rc;
   }
-  int err = xt::build_operands((int) o, (int) v, t2_d, ovoo_d, vvvo_d, c->in, st);
-  if(!err) err = set_fold(c);
+  int err = queue_fold_check(c);
+  if(!err) err = xt::build_operands((int) o, (int) v, t2_d, ovoo_d, vvvo_d, c->in, st);
   if(err) {
     cleanup();
     return fail(err == (int) hipErrorOutOfMemory ? XT_ENOMEM : XT_EHIP,
@@ -740,6 +750,7 @@ static int upload_common(xt_ctx* c, const double* eo, const double* ev, const do
   xt::track_free(ovoo_d);
   if(vvvo_d) xt::track_free(vvvo_d);
   c->upload_peak = count.c.peak;
+  c->fold        = fold_allowed(c);
   c->have_inputs = true;
   return XT_OK;
 }
@@ -800,10 +811,10 @@ int xt_upload_cholesky(xt_ctx* c, const double* eps_occ, const double* eps_vir, 
   if(!err) {
     xt::track_free(L_d);
     L_d = nullptr;
-    err = xt::build_operands((int) o, (int) v, t2_d, ovoo_d, none, c->in, st);
+    err = queue_fold_check(c);
+    if(!err) err = xt::build_operands((int) o, (int) v, t2_d, ovoo_d, none, c->in, st);
   }
   if(!err) err = xt::build_xva((int) o, (int) v, c->in, st);
-  if(!err) err = set_fold(c);
   if(err) {
     cleanup();
     return fail(err == (int) hipErrorOutOfMemory ? XT_ENOMEM : XT_EHIP,
@@ -812,6 +823,7 @@ int xt_upload_cholesky(xt_ctx* c, const double* eps_occ, const double* eps_vir, 
   xt::track_free(t2_d);
   xt::track_free(ovoo_d);
   c->upload_peak = count.c.peak;
+  c->fold        = fold_allowed(c);
   c->have_inputs = true;
   return XT_OK;
 }

@@ -44,16 +44,6 @@ constexpr int S1_T1   = 9 * 16;    // s1 T1 blocks in LDS
 constexpr int STAGE_D = 2 * 64 * LDK;  // staging union: A,B chunks; then the s1 V blocks (9*256)
 static_assert(STAGE_D >= 9 * 256, "staging too small for the s1 V blocks");
 
-// LDS of the persistent FP64 kernel, sized for three workgroups per CU.
-struct __align__(16) Smem {
-  double t3[T3N];
-  double stage[STAGE_D];
-  double t1s[S1_T1];  // s1 T1 blocks
-  double eps[24];
-  double red[8];
-  int    sub[6], dim[6], off[6];  // current sub-tile: position, extents, offsets
-};
-
 __device__ __forceinline__ int cdiv(int a, int b) { return (a + b - 1) / b; }
 // parity sign of the single index at position x (0,1,2) within its triple:
 // (x, others ascending) is even for x=0,2 and odd for x=1.
@@ -88,98 +78,200 @@ __device__ __forceinline__ void block_sum2(SM& sm, double& a, double& b) {
   }
 }
 
-// Index of t3 element (m, n) of bipartition g in the canonical LDS layout
-// e = sum_pos idx[pos] << 2*pos (pos 0..2 = h1..h3, 3..5 = p4..p6).
-__device__ __forceinline__ int emap(int hs, int hA, int hB, int ps, int pA, int pB, int m, int n) {
-  return ((m & 3) << (2 * hs)) | (((m >> 2) & 3) << (2 * (3 + pA))) | ((m >> 4) << (2 * (3 + pB))) |
-         ((n & 3) << (2 * hA)) | (((n >> 2) & 3) << (2 * hB)) | ((n >> 4) << (2 * (3 + ps)));
+// A sub-tile at the edge of its task tile has fewer than four orbitals along
+// some positions.  Rows (hs, pA, pB) and columns (hA, hB, ps) of a bipartition
+// are numbered inside the tile only, first position fastest, so the 16-row and
+// 16-column MFMA tiles that are needed shrink with it: over the uneven tiles
+// of O=48, V=384 the 4^6 sub-tiles hold 1.79 times the tile's elements, the
+// needed MFMA tiles 1.05 times.
+__device__ __forceinline__ int small_div(int n, int e) {  // n / e, 0 <= n < 64, 1 <= e <= 4
+  return (int) (((float) n + 0.5f) * __builtin_amdgcn_rcpf((float) e));
+}
+struct Item {
+  int a, b, c;  // coordinates along the three positions of a side
+};
+__device__ __forceinline__ Item item_of(int n, int ea, int eb) {
+  Item      x;
+  const int t = small_div(n, ea);
+  x.a         = n - t * ea;
+  x.c         = small_div(t, eb);
+  x.b         = t - x.c * eb;
+  return x;
 }
 
-// The 64x64xKC MFMA step of one staged chunk: wave w computes rows
-// 32*(w>>1).. and columns 32*(w&1).. as 2x2 16x16 tiles.
-template<int KCT = KC, int LDKT = LDK>
-__device__ __forceinline__ void mfma_chunk(const double* __restrict__ As,
-                                           const double* __restrict__ Bs, v4d (&acc)[2][2]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rb = (wave >> 1) * 32, cb = (wave & 1) * 32;
-  const int lr = lane & 15, lk = lane >> 4;
-#pragma unroll
-  for(int kk = 0; kk < KCT / 4; kk++) {
-    const int k  = 4 * kk + lk;
-    double    a0 = As[(rb + lr) * LDKT + k];
-    double    a1 = As[(rb + 16 + lr) * LDKT + k];
-    double    b0 = Bs[(cb + lr) * LDKT + k];
-    double    b1 = Bs[(cb + 16 + lr) * LDKT + k];
-    acc[0][0]    = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-    acc[0][1]    = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-    acc[1][0]    = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-    acc[1][1]    = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-  }
-}
-
-// Adds the accumulator of bipartition g into the LDS t3 tile.  D layout of
-// v_mfma_f64_16x16x4f64: register r of lane l holds row 4*r + (l>>4), column
-// l&15 (the four row groups are interleaved, unlike the 16-bit forms).
-template<class SM>
-__device__ __forceinline__ void acc_to_t3(SM& sm, int g, const v4d (&acc)[2][2]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rb = (wave >> 1) * 32, cb = (wave & 1) * 32;
-  const int hs = g / 3, ps = g % 3;
-  int       hA, hB, pA, pB;
-  pair_of(hs, hA, hB);
-  pair_of(ps, pA, pB);
+// The MFMA tiles of one wave: row tiles wm and wm + 2, column tiles wn and
+// wn + 2 of the Mt x Nt that are needed; bit 2 i + j of mask is set for the
+// needed ones.  Wave w takes quadrant (w + g) % 4, so that over the bipartitions
+// every SIMD gets the larger quadrants in turn.
+struct Quad {
+  int wm, wn, mask;
+};
+__device__ __forceinline__ Quad quadrant(int g, int rows, int cols) {
+  const int w = (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + g) & 3;
+  const int mt = (rows + 15) >> 4, nt = (cols + 15) >> 4;
+  Quad      q;
+  q.wm   = w >> 1;
+  q.wn   = w & 1;
+  q.mask = 0;
 #pragma unroll
   for(int i = 0; i < 2; i++)
 #pragma unroll
     for(int j = 0; j < 2; j++)
+      if(q.wm + 2 * i < mt && q.wn + 2 * j < nt) q.mask |= 1 << (2 * i + j);
+  return q;
+}
+
+// Box index parts of the rows and columns of the current bipartition (e =
+// sum_pos idx[pos] << 2*pos, pos 0..2 = h1..h3, 3..5 = p4..p6), written by 128
+// threads.  Padding rows and columns get an index outside the tile (some
+// extent of their side is short wherever there is one).
+struct Tables {
+  unsigned short row[64], col[64];
+};
+__device__ __forceinline__ void fill_tables(Tables& t, const int* ext, int hs, int hA, int hB, int ps,
+                                            int pA, int pB) {
+  const int tid = threadIdx.x;
+  if(tid >= 128) return;
+  const bool row = tid < 64;
+  const int  q0 = row ? hs : hA, q1 = row ? 3 + pA : hB, q2 = 3 + (row ? pB : ps);
+  const int  e0 = ext[q0], e1 = ext[q1], e2 = ext[q2];
+  Item       x = item_of(tid & 63, e0, e1);
+  if(x.c >= e2) {
+    x.a = e0 < 4 ? e0 : 0;
+    x.b = e0 < 4 ? 0 : e1 < 4 ? e1 : 0;
+    x.c = e0 < 4 || e1 < 4 ? 0 : e2 & 3;
+  }
+  const unsigned short v = (unsigned short) ((x.a << (2 * q0)) | (x.b << (2 * q1)) | (x.c << (2 * q2)));
+  if(row) t.row[tid] = v;
+  else t.col[tid - 64] = v;
+}
+
+// c[i][j] += a_i b_j for the tiles of mask.  In assembly because of the
+// branches (around builtins the compiler copies the accumulators per path).
+// The nops in front cover a vector write of an operand just before; nothing is
+// needed between matrix instructions on one accumulator; acc_ready() stands
+// before a vector read or write of the accumulators.
+__device__ __forceinline__ void mfma_step(int mask, double a0, double a1, double b0, double b1,
+                                          v4d (&c)[2][2]) {
+  asm volatile(
+    "s_nop 1\n\t"
+    "s_cmp_eq_u32 %[m], 15\n\t"
+    "s_cbranch_scc0 .Lpart_%=\n\t"
+    "v_mfma_f64_16x16x4_f64 %[c00], %[a0], %[b0], %[c00]\n\t"
+    "v_mfma_f64_16x16x4_f64 %[c01], %[a0], %[b1], %[c01]\n\t"
+    "v_mfma_f64_16x16x4_f64 %[c10], %[a1], %[b0], %[c10]\n\t"
+    "v_mfma_f64_16x16x4_f64 %[c11], %[a1], %[b1], %[c11]\n\t"
+    "s_branch .Ldone_%=\n"
+    ".Lpart_%=:\n\t"
+    "s_bitcmp1_b32 %[m], 0\n\t"
+    "s_cbranch_scc0 .Ldone_%=\n\t"
+    "v_mfma_f64_16x16x4_f64 %[c00], %[a0], %[b0], %[c00]\n\t"
+    "s_bitcmp1_b32 %[m], 1\n\t"
+    "s_cbranch_scc0 .Lrow_%=\n\t"
+    "v_mfma_f64_16x16x4_f64 %[c01], %[a0], %[b1], %[c01]\n"
+    ".Lrow_%=:\n\t"
+    "s_bitcmp1_b32 %[m], 2\n\t"
+    "s_cbranch_scc0 .Ldone_%=\n\t"
+    "v_mfma_f64_16x16x4_f64 %[c10], %[a1], %[b0], %[c10]\n"
+    ".Ldone_%=:\n"
+    : [c00] "+v"(c[0][0]), [c01] "+v"(c[0][1]), [c10] "+v"(c[1][0]), [c11] "+v"(c[1][1])
+    : [m] "s"(mask), [a0] "v"(a0), [a1] "v"(a1), [b0] "v"(b0), [b1] "v"(b1)
+    : "scc");
+}
+__device__ __forceinline__ void acc_ready(v4d (&c)[2][2]) {
+  asm volatile("s_nop 15\n\ts_nop 7" : "+v"(c[0][0]), "+v"(c[0][1]), "+v"(c[1][0]), "+v"(c[1][1]));
+}
+
+// The K step of one staged chunk over the wave's MFMA tiles.
+template<int KCT = KC, int LDKT = LDK>
+__device__ __forceinline__ void mfma_chunk(const double* __restrict__ As,
+                                           const double* __restrict__ Bs, const Quad& q,
+                                           v4d (&acc)[2][2]) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for(int kk = 0; kk < KCT / 4; kk++) {
+    const int    k  = 4 * kk + lk;
+    const double a0 = As[(16 * q.wm + lr) * LDKT + k], a1 = As[(16 * q.wm + 32 + lr) * LDKT + k];
+    const double b0 = Bs[(16 * q.wn + lr) * LDKT + k], b1 = Bs[(16 * q.wn + 32 + lr) * LDKT + k];
+    mfma_step(q.mask, a0, a1, b0, b1, acc);
+  }
+}
+
+// Adds the accumulators of a bipartition into the LDS t3 tile; the first one
+// of a sub-tile stores instead (every bipartition covers every element of the
+// tile).  D layout of v_mfma_f64_16x16x4f64: register r of lane l holds row
+// 4*r + (l>>4), column l&15 (the four row groups are interleaved, unlike the
+// 16-bit forms).
+__device__ __forceinline__ void acc_to_t3(double* t3, const Tables& t, const Quad& q, bool store,
+                                          v4d (&acc)[2][2]) {
+  const int lane = threadIdx.x & 63;
+  acc_ready(acc);
+#pragma unroll
+  for(int i = 0; i < 2; i++)
+#pragma unroll
+    for(int j = 0; j < 2; j++) {
+      if(!((q.mask >> (2 * i + j)) & 1)) continue;
+      const int n = t.col[16 * (q.wn + 2 * j) + (lane & 15)];
 #pragma unroll
       for(int r = 0; r < 4; r++) {
-        const int m = rb + 16 * i + 4 * r + (lane >> 4);
-        const int n = cb + 16 * j + (lane & 15);
-        sm.t3[emap(hs, hA, hB, ps, pA, pB, m, n)] += acc[i][j][r];
+        double* p = &t3[t.row[16 * (q.wm + 2 * i) + 4 * r + (lane >> 4)] | n];
+        *p        = store ? acc[i][j][r] : *p + acc[i][j][r];
       }
+    }
 }
 
 // Energy of the finished sub-tile: t3d in LDS, s1 operands staged in LDS,
-// denominators from sm.eps.  Returns (E4, E5) partial sums in thread 0.
+// denominators from sm.eps, ext the orbitals inside the tile.  Returns (E4,
+// E5) partial sums in thread 0.
 //   T1s[s][pa][hi] (16 per slot), V1s[s][hk + 4 hj + 16 pc + 64 pb] (256 per slot)
+// A thread owns one (h1, h2, h3, p4) and runs over p5 and p6.
 template<class SM>
 __device__ __forceinline__ void subtile_energy(SM& sm, const double* T1s, const double* V1s,
-                                               const int* sub, const int* dim, unsigned s1mask,
-                                               double& e4, double& e5) {
+                                               const int* ext, unsigned s1mask, double& e4,
+                                               double& e5) {
   e4 = 0.0;
   e5 = 0.0;
+  const int tid = threadIdx.x;
+  int       idx[6];
+#pragma unroll
+  for(int p = 0; p < 4; p++) idx[p] = (tid >> (2 * p)) & 3;
+  if(idx[0] < ext[0] && idx[1] < ext[1] && idx[2] < ext[2] && idx[3] < ext[3]) {
 #pragma unroll 1
-  for(int r = 0; r < T3N / NT; r++) {
-    const int e = threadIdx.x + NT * r;
-    int       idx[6];
-    bool      ok = true;
+    for(idx[5] = 0; idx[5] < ext[5]; idx[5]++)
+#pragma unroll 1
+      for(idx[4] = 0; idx[4] < ext[4]; idx[4]++) {
+        const double d = sm.t3[tid + NT * (idx[4] + 4 * idx[5])];
+        double       s = 0.0;
 #pragma unroll
-    for(int p = 0; p < 6; p++) {
-      idx[p] = (e >> (2 * p)) & 3;
-      ok     = ok && (4 * sub[p] + idx[p] < dim[p]);
-    }
-    if(!ok) continue;
-    const double d = sm.t3[e];
-    double       s = 0.0;
-#pragma unroll
-    for(int slot = 0; slot < 9; slot++) {
-      if(!((s1mask >> slot) & 1)) continue;
-      const int pa = slot / 3, hi = slot % 3;
-      int       hj, hk, pb, pc;
-      pair_of(hi, hj, hk);
-      pair_of(pa, pb, pc);
-      s += T1s[slot * 16 + idx[3 + pa] * 4 + idx[hi]] *
-           V1s[slot * 256 + idx[hk] + 4 * idx[hj] + 16 * idx[3 + pc] + 64 * idx[3 + pb]];
-    }
-    // denominator in the reference's order (ccsd_t_all_fused_cpu.hpp:612-614)
-    const double D = sm.eps[8 + idx[2]] + sm.eps[4 + idx[1]] + sm.eps[idx[0]] -
-                     sm.eps[20 + idx[5]] - sm.eps[16 + idx[4]] - sm.eps[12 + idx[3]];
-    e4 += d * d / D;
-    e5 += d * (d + s) / D;
+        for(int slot = 0; slot < 9; slot++) {
+          if(!((s1mask >> slot) & 1)) continue;
+          const int pa = slot / 3, hi = slot % 3;
+          int       hj, hk, pb, pc;
+          pair_of(hi, hj, hk);
+          pair_of(pa, pb, pc);
+          s += T1s[slot * 16 + idx[3 + pa] * 4 + idx[hi]] *
+               V1s[slot * 256 + idx[hk] + 4 * idx[hj] + 16 * idx[3 + pc] + 64 * idx[3 + pb]];
+        }
+        // denominator in the reference's order (ccsd_t_all_fused_cpu.hpp:612-614)
+        const double D = sm.eps[8 + idx[2]] + sm.eps[4 + idx[1]] + sm.eps[idx[0]] -
+                         sm.eps[20 + idx[5]] - sm.eps[16 + idx[4]] - sm.eps[12 + idx[3]];
+        e4 += d * d / D;
+        e5 += d * (d + s) / D;
+      }
   }
   block_sum2(sm, e4, e5);
 }
+
+// LDS of the persistent FP64 kernel, sized for three workgroups per CU.
+struct __align__(16) Smem {
+  double t3[T3N];
+  double stage[STAGE_D];
+  double t1s[S1_T1];  // s1 T1 blocks
+  double eps[24];
+  double red[8];
+  Tables tab;
+  int    start[6], ext[6];  // current sub-tile: first orbitals, orbitals inside the tile
+};
 
 // ---------------------------------------------------------------------------
 // HBM-resident path: operands are formed on the fly from spatial closed-shell
@@ -209,15 +301,13 @@ __device__ __forceinline__ void fetch4(const RowPtr& rp, int k0, int Kp, double*
 
 __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, uint64_t d2code,
                                 uint64_t s1code, double& e4, double& e5) {
-  const int  tid = threadIdx.x;
-  const int  O = S.O, V = S.V;
-  const int* sub = sm.sub;
-  for(int e = tid; e < T3N; e += NT) sm.t3[e] = 0.0;
+  const int tid = threadIdx.x;
+  const int O = S.O, V = S.V;
   if(tid < 24) {
-    const int p = tid >> 2, i = tid & 3, g = 4 * sub[p] + i;
-    sm.eps[tid] = g < sm.dim[p] ? (p < 3 ? S.eo : S.ev)[sm.off[p] + g] : 0.0;
+    const int p = tid >> 2, i = tid & 3;
+    sm.eps[tid] = i < sm.ext[p] ? (p < 3 ? S.eo : S.ev)[sm.start[p] + i] : 0.0;
   }
-  __syncthreads();
+  bool store = true;  // no bipartition has been added yet
 
   const int row = tid >> 2, kq = tid & 3;
   double*   As  = sm.stage;
@@ -234,17 +324,15 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
     int       hA, hB, pA, pB;
     pair_of(hs, hA, hB);
     pair_of(ps, pA, pB);
+    const int eHS = sm.ext[hs], ePA = sm.ext[3 + pA], eHA = sm.ext[hA], eHB = sm.ext[hB];
+    const int rows = __builtin_amdgcn_readfirstlane(eHS * ePA * sm.ext[3 + pB]);
+    const int cols = __builtin_amdgcn_readfirstlane(eHA * eHB * sm.ext[3 + ps]);
+    const Quad quad = quadrant(g, rows, cols);
     // this thread's M row (hs, pA, pB) and N row (hA, hB, ps)
-    const int gHS = 4 * sub[hs] + (row & 3), gPA = 4 * sub[3 + pA] + ((row >> 2) & 3),
-              gPB = 4 * sub[3 + pB] + (row >> 4);
-    const int gHA = 4 * sub[hA] + (row & 3), gHB = 4 * sub[hB] + ((row >> 2) & 3),
-              gPS = 4 * sub[3 + ps] + (row >> 4);
-    const bool mok = gHS < sm.dim[hs] && gPA < sm.dim[3 + pA] && gPB < sm.dim[3 + pB];
-    const bool nok = gHA < sm.dim[hA] && gHB < sm.dim[hB] && gPS < sm.dim[3 + ps];
-    const size_t HS = sm.off[hs] + (mok ? gHS : 0), PA = sm.off[3 + pA] + (mok ? gPA : 0),
-                 PB = sm.off[3 + pB] + (mok ? gPB : 0);
-    const size_t HA = sm.off[hA] + (nok ? gHA : 0), HB = sm.off[hB] + (nok ? gHB : 0),
-                 PS = sm.off[3 + ps] + (nok ? gPS : 0);
+    const bool   mok = row < rows, nok = row < cols;
+    const Item   m = item_of(mok ? row : 0, eHS, ePA), n = item_of(nok ? row : 0, eHA, eHB);
+    const size_t HS = sm.start[hs] + m.a, PA = sm.start[3 + pA] + m.b, PB = sm.start[3 + pB] + m.c;
+    const size_t HA = sm.start[hA] + n.a, HB = sm.start[hB] + n.b, PS = sm.start[3 + ps] + n.c;
     // operand rows c1*x - c2*y of the spin-orbital elements: both terms ->
     // the antisymmetrised array; one term -> that array (sign folded into c)
     auto pick = [](bool ok, unsigned code, unsigned bx, unsigned by, double sgn, const double* both,
@@ -299,6 +387,7 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
     for(int c = 0; c < nc; c++) {
       const double ca = c < n1 ? a1r.c : a2r.c, cb = c < n1 ? b1r.c : b2r.c;
       __syncthreads();
+      if(c == 0) fill_tables(sm.tab, sm.ext, hs, hA, hB, ps, pA, pB);
 #pragma unroll
       for(int j = 0; j < 4; j++) {
         As[row * LDK + 4 * kq + j] = ca * ax[j];
@@ -306,10 +395,13 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
       }
       __syncthreads();
       if(c + 1 < nc) fetch(c + 1);
-      mfma_chunk(As, Bs, acc);
+      mfma_chunk(As, Bs, quad, acc);
     }
-    acc_to_t3(sm, g, acc);
+    acc_to_t3(sm.t3, sm.tab, quad, store, acc);
+    store = false;
   }
+  if(store)
+    for(int e = tid; e < T3N; e += NT) sm.t3[e] = 0.0;
 
   // ---- s1 operands: T1so(pa,hi) and <hk hj||pc pb> blocks of the sub-tile
   __syncthreads();
@@ -323,10 +415,9 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
     const int      slot = x >> 4, pai = (x >> 2) & 3, hii = x & 3;
     const unsigned c    = (unsigned) (s1code >> (4 * slot)) & 15u;
     const int      pa = slot / 3, hi = slot % 3;
-    const int      gp = 4 * sub[3 + pa] + pai, gh = 4 * sub[hi] + hii;
-    double         v  = 0.0;
-    if((c & 1) && gp < sm.dim[3 + pa] && gh < sm.dim[hi]) {
-      v = S.t1[(size_t) (sm.off[3 + pa] + gp) * O + sm.off[hi] + gh];
+    double         v = 0.0;
+    if((c & 1) && pai < sm.ext[3 + pa] && hii < sm.ext[hi]) {
+      v = S.t1[(size_t) (sm.start[3 + pa] + pai) * O + sm.start[hi] + hii];
       if(c & 2) v = -v;
     }
     T1s[x] = v;
@@ -338,12 +429,11 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
     int            hj, hk, pb, pc;
     pair_of(hi, hj, hk);
     pair_of(pa, pb, pc);
-    const int gk = 4 * sub[hk] + (w & 3), gj = 4 * sub[hj] + ((w >> 2) & 3),
-              gc = 4 * sub[3 + pc] + ((w >> 4) & 3), gb = 4 * sub[3 + pb] + (w >> 6);
-    double v = 0.0;
-    if((c & 1) && gk < sm.dim[hk] && gj < sm.dim[hj] && gc < sm.dim[3 + pc] && gb < sm.dim[3 + pb]) {
-      const size_t K = sm.off[hk] + gk, J = sm.off[hj] + gj, PC = sm.off[3 + pc] + gc,
-                   PBx = sm.off[3 + pb] + gb;
+    const int gk = w & 3, gj = (w >> 2) & 3, gc = (w >> 4) & 3, gb = w >> 6;
+    double    v  = 0.0;
+    if((c & 1) && gk < sm.ext[hk] && gj < sm.ext[hj] && gc < sm.ext[3 + pc] && gb < sm.ext[3 + pb]) {
+      const size_t K = sm.start[hk] + gk, J = sm.start[hj] + gj, PC = sm.start[3 + pc] + gc,
+                   PBx = sm.start[3 + pb] + gb;
       const double x1 = (c & 4) ? S.vvoo[((PC * V + PBx) * O + K) * O + J] : 0.0;  // (hk pc|hj pb)
       const double x2 = (c & 8) ? S.vvoo[((PBx * V + PC) * O + K) * O + J] : 0.0;  // (hk pb|hj pc)
       v               = ((c & 4) && (c & 8)) ? x1 - x2 : ((c & 4) ? x1 : -x2);
@@ -351,7 +441,7 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
     V1s[x] = v;
   }
   __syncthreads();
-  subtile_energy(sm, T1s, V1s, sm.sub, sm.dim, s1mask, e4, e5);
+  subtile_energy(sm, T1s, V1s, sm.ext, s1mask, e4, e5);
 }
 
 // Persistent kernel: workgroup b serves queue b % kQueues first (dispatch is
@@ -398,9 +488,8 @@ __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) 
           if(ti < 0) continue;
 #pragma unroll
           for(int p = 0; p < 6; p++) {
-            sm.sub[p] = sub[p];
-            sm.dim[p] = T.dim[p];
-            sm.off[p] = T.off[p];
+            sm.start[p] = T.off[p] + 4 * sub[p];
+            sm.ext[p]   = min(4, T.dim[p] - 4 * sub[p]);
           }
           break;
         }
@@ -637,24 +726,12 @@ __global__ void __launch_bounds__(256) k_vvoo_asym(const double* __restrict__ vv
   }
 }
 
-int vvoo_asymmetry(const double* vvoo, int O, int V, double* diff, double* largest, void* stream) {
-  hipStream_t         st = (hipStream_t) stream;
-  unsigned long long* d  = nullptr;
-  hipError_t          e;
-  if((e = hipMalloc((void**) &d, 2 * sizeof(*d)))) return (int) e;
-  int rc = launch_zero_u64(d, 2, stream);
-  if(!rc) {
-    hipLaunchKernelGGL(k_vvoo_asym, dim3((unsigned) std::min<long>((long) V * V, 4096)), dim3(256), 0,
-                       st, vvoo, (long) O, (long) V, d);
-    rc = (int) hipGetLastError();
-  }
-  double h[2] = {0.0, 0.0};
-  if(!rc) rc = (int) hipMemcpyAsync(h, d, sizeof h, hipMemcpyDeviceToHost, st);
-  if(!rc) rc = (int) hipStreamSynchronize(st);
-  (void) hipFree(d);
-  *diff    = h[0];
-  *largest = h[1];
-  return rc;
+int launch_vvoo_asym(const double* vvoo, int O, int V, unsigned long long* out, void* stream) {
+  const int rc = launch_zero_u64(out, 2, stream);
+  if(rc) return rc;
+  hipLaunchKernelGGL(k_vvoo_asym, dim3((unsigned) std::min<long>((long) V * V, 4096)), dim3(256), 0,
+                     (hipStream_t) stream, vvoo, (long) O, (long) V, out);
+  return (int) hipGetLastError();
 }
 
 int launch_zero_u64(unsigned long long* p, long n, void* stream) {
@@ -701,6 +778,8 @@ struct __align__(16) PSmem {
   } u;
   double eps[24];
   double red[8];
+  Tables tab;
+  int    ext[6];  // orbitals of the block inside the tile
 };
 // a K tile list entry fits two ints: K <= 4096, total K < 2^20, exec slot < 2^30
 static_assert((kMaxNoab + kMaxNvab) * 4096 + kPackedKC < (1 << 20), "K offsets must fit 20 bits");
@@ -729,11 +808,12 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
   const int*  k_n    = s1_exec + 9;
   const int4* k_list = reinterpret_cast<const int4*>(k_n + kKlistCountInts);
 
-  for(int e = tid; e < T3N; e += NT) sm.t3[e] = 0.0;
   if(tid < 24) {
     const int p = tid >> 2, i = tid & 3, g = 4 * sub[p] + i;
     sm.eps[tid] = g < dim[p] ? A.evl[p][g] : 0.0;
   }
+  if(tid < 6) sm.ext[tid] = min(4, dim[tid] - 4 * sub[tid]);
+  bool store = true;  // no bipartition has been added yet
   __syncthreads();
   double* As = sm.stage;
   double* Bs = sm.stage + 64 * PLDK;
@@ -781,27 +861,26 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
     // 16 doubles.  The d1 <ij||ka> block keeps k slowest (row + k * bstr1):
     // there thread (n1, kq) = (tid % 64, tid / 64) reads row n1 at k = 4 kq + j,
     // and an instruction reads 64 neighbouring rows.
-    // Row r of either operand: r & 3, (r >> 2) & 3, r >> 4 index the first,
-    // second and third t3 position of its side (hs, pA, pB or hA, hB, ps), so
-    // row rs + 16 j moves the third position by j.
+    // A row of either operand is (item of the first two positions of its side,
+    // third position): thread rs takes the item rs of up to 16 and j is the
+    // third position, so row rs + per * j, per the items the tile holds.
+    const int eHS = sm.ext[hs], ePA = sm.ext[3 + pA], ePB = sm.ext[3 + pB];
+    const int eHA = sm.ext[hA], eHB = sm.ext[hB], ePS = sm.ext[3 + ps];
+    const int aper = __builtin_amdgcn_readfirstlane(eHS * ePA), bper = __builtin_amdgcn_readfirstlane(eHA * eHB);
+    const Quad quad = quadrant(g, __builtin_amdgcn_readfirstlane(aper * ePB), __builtin_amdgcn_readfirstlane(bper * ePS));
     const int kk = tid & 15, rs = tid >> 4;
-    const int aHS = 4 * sub[hs] + (rs & 3), aPA = 4 * sub[3 + pA] + ((rs >> 2) & 3),
-              aPB = 4 * sub[3 + pB];
-    const int bHA = 4 * sub[hA] + (rs & 3), bHB = 4 * sub[hB] + ((rs >> 2) & 3),
-              bPS = 4 * sub[3 + ps];
-    unsigned  amask = 0, bmask = 0;  // rows inside the block, per j
-#pragma unroll
-    for(int j = 0; j < 4; j++) {
-      if(aHS < DHS && aPA < DPA && aPB + j < DPB) amask |= 1u << j;
-      if(bHA < DHA && bHB < DHB && bPS + j < DPS) bmask |= 1u << j;
-    }
+    const int ax = small_div(rs, eHS), bx = small_div(rs, eHA);
+    const int aHS = 4 * sub[hs] + rs - ax * eHS, aPA = 4 * sub[3 + pA] + ax, aPB = 4 * sub[3 + pB];
+    const int bHA = 4 * sub[hA] + rs - bx * eHA, bHB = 4 * sub[hB] + bx, bPS = 4 * sub[3 + ps];
+    // third positions inside the block
+    const unsigned amask = rs < aper ? (1u << ePB) - 1u : 0u, bmask = rs < bper ? (1u << ePS) - 1u : 0u;
     const long a1 = aPA + (aPB + aHS * DPB) * DPA;  // d1_t2 row of j = 0: [hs][pB][pA]
     const long a2 = aHS + (aPB + aPA * DPB) * DHS;  // d2_v2 row: [pA][pB][hs]
     const long b2 = bPS + (bHA + bHB * DHA) * DPS;  // d2_t2 row: [hB][hA][ps]
     const int  n1 = tid & 63, kq = tid >> 6;
-    const int  gHA = 4 * sub[hA] + (n1 & 3), gHB = 4 * sub[hB] + ((n1 >> 2) & 3),
-              gPS = 4 * sub[3 + ps] + (n1 >> 4);
-    const bool nok1  = gHA < DHA && gHB < DHB && gPS < DPS;
+    const bool nok1 = n1 < bper * ePS;
+    const Item y    = item_of(nok1 ? n1 : 0, eHA, eHB);
+    const int  gHA = 4 * sub[hA] + y.a, gHB = 4 * sub[hB] + y.b, gPS = 4 * sub[3 + ps] + y.c;
     const long rB1   = gHB + (gHA + gPS * DHA) * DHB;  // d1_v2 element of k = rB1 + k * bstr1
     const long bstr1 = DPS * DHA * DHB;
     // tile walkers (k only grows): wa for the thread's k-contiguous k, wb for
@@ -871,13 +950,16 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
 #pragma unroll 1
       for(int c = 0; c < nc; c++) {
         __syncthreads();
+        if(c == 0) fill_tables(sm.tab, sm.ext, hs, hA, hB, ps, pA, pB);
         // the masks are applied here, so that a chunk's loads are waited for
         // only after the previous chunk's MFMAs were issued
 #pragma unroll
-        for(int j = 0; j < 4; j++) As[(rs + 16 * j) * PLDK + kk] = ((oka >> j) & 1) ? sg * av[j] : 0.0;
+        for(int j = 0; j < 4; j++)
+          if((amask >> j) & 1) As[(rs + aper * j) * PLDK + kk] = ((oka >> j) & 1) ? sg * av[j] : 0.0;
         if(c * PKC >= kd2) {
 #pragma unroll
-          for(int j = 0; j < 4; j++) Bs[(rs + 16 * j) * PLDK + kk] = ((okb >> j) & 1) ? bv[j] : 0.0;
+          for(int j = 0; j < 4; j++)
+            if((bmask >> j) & 1) Bs[(rs + bper * j) * PLDK + kk] = ((okb >> j) & 1) ? bv[j] : 0.0;
         }
         else {
 #pragma unroll
@@ -885,11 +967,14 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
         }
         __syncthreads();
         if(c + 1 < nc) load(c + 1);
-        mfma_chunk<PKC, PLDK>(As, Bs, acc);
+        mfma_chunk<PKC, PLDK>(As, Bs, quad, acc);
       }
-      acc_to_t3(sm, g, acc);
+      acc_to_t3(sm.t3, sm.tab, quad, store, acc);
+      store = false;
     }
   }
+  if(store)
+    for(int e = tid; e < T3N; e += NT) sm.t3[e] = 0.0;
 
   // s1 operands from the packed buffers: t1 [hi][pa], v2 [pb][pc][hj][hk]
   __syncthreads();  // every thread is done with the tile list and the staged chunk
@@ -924,7 +1009,7 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
   }
   __syncthreads();
   double e4, e5;
-  subtile_energy(sm, T1s, V1s, sub, dim, s1mask, e4, e5);
+  subtile_energy(sm, T1s, V1s, sm.ext, s1mask, e4, e5);
   if(tid == 0) {
     A.partial[blockIdx.x]                = e4;
     A.partial[blockIdx.x + A.num_blocks] = e5;
