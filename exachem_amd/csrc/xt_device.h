@@ -171,18 +171,31 @@ struct GatherBlock {
   int    perm[4];
   double alpha;     // +1 or -1
 };
+// The same block as the kernel reads it (gather_desc): element (i0, i1, i2, i3)
+// in destination order, row-major over ext (leading extents 1 for T1), is
+// alpha * (x - y) of the terms that the spins leave, x at px + sum i sx of
+// array src, y at py + sum i sy; kS is the destination position of the first
+// term's contiguous index.
+enum GatherArray { kArrT1, kArrT2h, kArrT2p, kArrVvoo, kArrOvk, kArrXv, kGatherArrays };
+struct GatherDesc {
+  long     dst, n;
+  long     px, py, sx[4], sy[4];
+  double   alpha;
+  unsigned ext[4];
+  int      buf, src, on1, on2, kS;
+};
+GatherDesc gather_desc(const GatherBlock& B, long O, long V, long Op, long Vp);
 struct GatherSrc {
   long          O, V, Op, Vp;
   const double* t1;    // [V][O]
   const double* t2h;   // [V][V][O][Op]
-  const double* vvoo;  // [V][V][O][O]
-  const double* ovk;   // [O][V][O][Op]
-  const double* xv;    // [V][V][O][Vp], xv[c][b][i][a] = vvvo[a][c][b][i]
+  const double* a[kGatherArrays];  // t1, t2h, t2p [O][O][V][Vp], vvoo [V][V][O][O],
+                                   // ovk [O][V][O][Op], xv [V][V][O][Vp] (xv[c][b][i][a] = vvvo[a][c][b][i])
 };
 struct GatherDst {
   double* buf[6];
 };
-int launch_gather(const GatherBlock* blocks, int n_blocks, long max_elems, const GatherSrc& S,
+int launch_gather(const GatherDesc* blocks, int n_blocks, long max_elems, const GatherSrc& S,
                   const GatherDst& D, void* stream);
 // Dense spin-orbital T1 / T2 from the spatial amplitudes (either may be null).
 int launch_expand_t(const GatherSrc& S, double* t1_so, double* t2_so, void* stream);

@@ -222,4 +222,64 @@ int plan_gather(const GatherTiling& T, bool restricted, const long* t, std::vect
   return 0;
 }
 
+GatherDesc gather_desc(const GatherBlock& B, long O, long V, long Op, long Vp) {
+  GatherDesc D = {};
+  D.dst        = B.dst;
+  D.n          = B.n;
+  D.alpha      = B.alpha;
+  D.buf        = B.buf;
+  const int s0 = B.spin[0], s1 = B.spin[1], s2 = B.nd > 2 ? B.spin[2] : 0, s3 = B.nd > 2 ? B.spin[3] : 0;
+  D.on1 = s0 == s2 && s1 == s3;
+  D.on2 = s0 == s3 && s1 == s2;
+  std::array<long, 4> x = {}, y = {};  // steps of the two terms per source dimension
+  switch(B.kind) {
+    case kGatherT1:  // t1[a][i]
+      D.src = kArrT1;
+      D.on1 = s0 == s1;
+      D.on2 = 0;
+      x     = {O, 1, 0, 0};
+      break;
+    case kGatherT2:
+      if(B.perm[3] < 2) {  // the destination runs over a virtual index: t2p[i][j][a][b]
+        D.src = kArrT2p;
+        x     = {Vp, 1, O * V * Vp, V * Vp};
+        y     = {Vp, 1, V * Vp, O * V * Vp};
+      }
+      else {  // t2h[a][b][i][j]
+        D.src = kArrT2h;
+        x     = {V * O * Op, O * Op, Op, 1};
+        y     = {V * O * Op, O * Op, 1, Op};
+      }
+      break;
+    case kGatherIJAB:  // vvoo[a][b][i][j], vvoo[b][a][i][j]
+      D.src = kArrVvoo;
+      x     = {O, 1, V * O * O, O * O};
+      y     = {O, 1, O * O, V * O * O};
+      break;
+    case kGatherIJKA:  // ovk[j][a][i][k], ovk[i][a][j][k]
+      D.src = kArrOvk;
+      D.on2 = s1 == s2 && s0 == s3;
+      x     = {Op, V * O * Op, 1, O * Op};
+      y     = {V * O * Op, Op, 1, O * Op};
+      break;
+    default:  // kGatherIABC: xv[c][b][i][a], xv[b][c][i][a]
+      D.src = kArrXv;
+      x     = {Vp, 1, O * Vp, V * O * Vp};
+      y     = {Vp, 1, V * O * Vp, O * Vp};
+  }
+  for(int d = 0; d < B.nd; d++) {
+    D.px += B.start[d] * x[d];
+    D.py += B.start[d] * y[d];
+  }
+  D.kS = 3;
+  for(int k = 0; k < 4; k++) {
+    const int kk = k - (4 - B.nd);
+    D.ext[k]     = kk >= 0 ? (unsigned) B.size[B.perm[kk]] : 1u;
+    D.sx[k]      = kk >= 0 ? x[B.perm[kk]] : 0;
+    D.sy[k]      = kk >= 0 ? y[B.perm[kk]] : 0;
+    if((D.on1 || !D.on2 ? D.sx[k] : D.sy[k]) == 1 && D.ext[k] > 1) D.kS = k;
+  }
+  return D;
+}
+
 }  // namespace xt

@@ -8,62 +8,33 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdint>
 
 #include "xt_device.h"
 
 namespace xt {
 namespace {
 
-// Spin-orbital element of one of the five tensors the gathers read, formed
-// from the spatial closed-shell inputs (spin-orbital order is [alpha, beta]
-// per space).  The combination rule c1*x - c2*y and the spatial sources:
+// The spin-orbital elements the gathers read, from the spatial closed-shell
+// inputs (spin-orbital order is [alpha, beta] per space), as c1*x - c2*y:
 //   T1   t1(a,i)        = [sa=si] t1[A][I]
 //   T2   t2(a,b,i,j)    = [sa=si][sb=sj] t2[A][B][I][J] - [sa=sj][sb=si] t2[A][B][J][I]
 //   IJAB <ij||ab>       = [si=sa][sj=sb] (ai|bj) - [si=sb][sj=sa] (bi|aj)          (vvoo)
 //   IJKA <ij||ka>       = [si=sk][sj=sa] (ja|ik) - [sj=sk][si=sa] (ia|jk)          (ovoo)
 //   IABC <ia||bc>       = [si=sb][sa=sc] (ac|bi) - [si=sc][sa=sb] (ab|ci)          (vvvo)
-// with t2 read from t2h[a][b][i][Op], ovoo from ovk[i][a][j][Op] and vvvo
-// from xv[c][b][i][Vp] = vvvo[a][c][b][i].
-__device__ __forceinline__ double so_value(const GatherSrc& S, int kind, const int* sp, const long* x) {
-  const long O = S.O, V = S.V, Op = S.Op, Vp = S.Vp;
-  auto comb = [](bool c1, bool c2, double a, double b) {
-    return c1 && c2 ? a - b : (c1 ? a : (c2 ? -b : 0.0));
-  };
-  switch(kind) {
-    case kGatherT1: return sp[0] == sp[1] ? S.t1[x[0] * O + x[1]] : 0.0;
-    case kGatherT2: {
-      const bool c1 = sp[0] == sp[2] && sp[1] == sp[3], c2 = sp[0] == sp[3] && sp[1] == sp[2];
-      const long ab = (x[0] * V + x[1]) * O;
-      return comb(c1, c2, c1 ? S.t2h[(ab + x[2]) * Op + x[3]] : 0.0,
-                  c2 ? S.t2h[(ab + x[3]) * Op + x[2]] : 0.0);
-    }
-    case kGatherIJAB: {
-      const bool c1 = sp[0] == sp[2] && sp[1] == sp[3], c2 = sp[0] == sp[3] && sp[1] == sp[2];
-      return comb(c1, c2, c1 ? S.vvoo[((x[2] * V + x[3]) * O + x[0]) * O + x[1]] : 0.0,
-                  c2 ? S.vvoo[((x[3] * V + x[2]) * O + x[0]) * O + x[1]] : 0.0);
-    }
-    case kGatherIJKA: {
-      const bool c1 = sp[0] == sp[2] && sp[1] == sp[3], c2 = sp[1] == sp[2] && sp[0] == sp[3];
-      return comb(c1, c2, c1 ? S.ovk[((x[1] * V + x[3]) * O + x[0]) * Op + x[2]] : 0.0,
-                  c2 ? S.ovk[((x[0] * V + x[3]) * O + x[1]) * Op + x[2]] : 0.0);
-    }
-    default: {  // kGatherIABC
-      const bool c1 = sp[0] == sp[2] && sp[1] == sp[3], c2 = sp[0] == sp[3] && sp[1] == sp[2];
-      return comb(c1, c2, c1 ? S.xv[((x[3] * V + x[2]) * O + x[0]) * Vp + x[1]] : 0.0,
-                  c2 ? S.xv[((x[2] * V + x[3]) * O + x[0]) * Vp + x[1]] : 0.0);
-    }
-  }
-}
+// with t2 read from t2h[a][b][i][Op] or t2p[i][j][a][Vp], ovoo from
+// ovk[i][a][j][Op] and vvvo from xv[c][b][i][Vp] = vvvo[a][c][b][i].
 
-// Source dimension whose consecutive values are adjacent in memory, for the
-// term the block reads (for a T2 block that reads both terms, the first one).
-__device__ __forceinline__ int fast_dim(const GatherBlock& B) {
-  switch(B.kind) {
-    case kGatherIJKA: return 2;
-    case kGatherT2: return (B.spin[0] == B.spin[2] && B.spin[1] == B.spin[3]) ? 3 : 2;
-    default: return 1;  // T1, IJAB, IABC
+// n / d of the block's index arithmetic: a multiply by ceil(2^32 / d) where
+// that is exact (n d < 2^32, checked once per block), else a division.
+struct Div {
+  unsigned d, m;
+  bool     mul;
+  __device__ __forceinline__ Div(unsigned d_, bool mul_): d(d_), m(d_ > 1 ? 0xffffffffu / d_ + 1u : 0u), mul(mul_) {}
+  __device__ __forceinline__ unsigned operator()(unsigned n) const {
+    return mul ? (d > 1 ? __umulhi(n, m) : n) : n / d;
   }
-}
+};
 
 constexpr int GT   = 256;      // threads per gather workgroup
 constexpr int SLAB = 48 * 49;  // LDS slab (doubles): extents up to 48 with one pad column
@@ -80,75 +51,66 @@ constexpr int SLAB = 48 * 49;  // LDS slab (doubles): extents up to 48 with one 
 // of the two other positions: the slab is read along the source's contiguous
 // dimension and written along the destination's, so both sides run through
 // whole rows instead of one element per row.
-__global__ __launch_bounds__(GT) void k_gather(const GatherBlock* __restrict__ blocks, GatherSrc S,
+//
+// Bound: memory.  Per element the spin tests, the array's index rule and four
+// 32-bit divisions used to cost more than the copy: the host works the rules
+// out once per block (gather_desc), the divisions are multiplies, and T2 blocks
+// that run over a virtual index are read from t2p, whose rows are virtual.
+__global__ __launch_bounds__(GT) void k_gather(const GatherDesc* __restrict__ blocks, GatherSrc S,
                                                GatherDst D) {
-  __shared__ double  slab[SLAB];
-  const GatherBlock& B   = blocks[blockIdx.y];
-  double*            dst = D.buf[B.buf] + B.dst;
-  const int          nd  = B.nd;
-  const unsigned     n   = (unsigned) B.n;  // a block holds fewer than 2^31 doubles (host check)
-  int                sp[4] = {0, 0, 0, 0};
-#pragma unroll
-  for(int d = 0; d < 4; d++) sp[d] = d < nd ? B.spin[d] : 0;
-  // destination positions padded to four (leading extents 1): source
-  // dimension src[k] (-1 for padding) and extent E[k]
-  int src[4], E[4];
-#pragma unroll
-  for(int k = 0; k < 4; k++) {
-    const int kk = k - (4 - nd);
-    src[k]       = kk >= 0 ? B.perm[kk] : -1;
-    E[k]         = kk >= 0 ? B.size[src[k]] : 1;
-  }
-  const int fd = fast_dim(B);
-  int       kS = 3;
-#pragma unroll
-  for(int k = 0; k < 3; k++)
-    if(src[k] == fd) kS = k;
-  const unsigned ES = (unsigned) E[kS], EF = (unsigned) E[3], ld = EF + 1;
+  __shared__ double slab[SLAB];
+  const GatherDesc& B = blocks[blockIdx.y];
+  const unsigned    n = (unsigned) B.n;  // a block holds fewer than 2^31 doubles (host check)
+  double* __restrict__ dst       = D.buf[B.buf] + B.dst;
+  const double* __restrict__ src = S.a[B.src];
+  const double* __restrict__ x0  = src + B.px;
+  const double* __restrict__ y0  = src + B.py;
+  const double al  = B.alpha;
+  const bool   on1 = B.on1 != 0, on2 = B.on2 != 0;
+  auto         value = [&](long px, long py) {
+    const double x = on1 ? x0[px] : 0.0, y = on2 ? y0[py] : 0.0;
+    return al * (on1 && on2 ? x - y : on1 ? x : on2 ? -y : 0.0);
+  };
+  const int      kS = B.kS;
+  const unsigned E[4]  = {B.ext[0], B.ext[1], B.ext[2], B.ext[3]};
+  const long     sx[4] = {B.sx[0], B.sx[1], B.sx[2], B.sx[3]}, sy[4] = {B.sy[0], B.sy[1], B.sy[2], B.sy[3]};
+  const unsigned emax = max(max(E[0], E[1]), max(E[2], E[3]));
+  const bool     mul  = (unsigned long long) n * emax < (1ull << 32);
+  const unsigned ES = B.ext[kS], EF = E[3], ld = EF + 1;
   if(kS == 3 || ES * ld > (unsigned) SLAB) {
-    // 32-bit index decode: a 64-bit divide costs several times more
-    for(unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-      unsigned r = e;
-      long     x[4] = {0, 0, 0, 0};
-      for(int k = nd - 1; k >= 0; k--) {
-        const int      d  = B.perm[k];
-        const unsigned sz = (unsigned) B.size[d];
-        x[d]              = B.start[d] + (long) (r % sz);
-        r /= sz;
-      }
-      dst[e] = B.alpha * so_value(S, B.kind, sp, x);
+    const Div q3(E[3], mul), q2(E[2], mul), q1(E[1], mul);
+    for(unsigned e = blockIdx.x * GT + threadIdx.x; e < n; e += gridDim.x * GT) {
+      const unsigned r2 = q3(e), i3 = e - r2 * E[3], r1 = q2(r2), i2 = r2 - r1 * E[2], i0 = q1(r1),
+                     i1 = r1 - i0 * E[1];
+      dst[e]            = value(i0 * sx[0] + i1 * sx[1] + i2 * sx[2] + i3 * sx[3],
+                                i0 * sy[0] + i1 * sy[1] + i2 * sy[2] + i3 * sy[3]);
     }
     return;
   }
-  // the two other positions o1 < o2 index the slabs
-  const int o1 = kS == 0 ? 1 : 0, o2 = kS == 2 ? 1 : 2;
-  unsigned  st[4];
-  st[3] = 1;
-#pragma unroll
-  for(int k = 2; k >= 0; k--) st[k] = st[k + 1] * (unsigned) E[k + 1];
-  const unsigned E2 = (unsigned) E[o2], nslab = (unsigned) E[o1] * E2, nel = ES * EF;
-  const int      d1 = src[o1], d2 = src[o2], dF = src[3];
-  long           x0[4];
-#pragma unroll
-  for(int d = 0; d < 4; d++) x0[d] = d < nd ? B.start[d] : 0;
+  // the two other positions o1 < o2 index the slabs; st: destination steps
+  const int      o1 = kS == 0 ? 1 : 0, o2 = kS == 2 ? 1 : 2;
+  const unsigned st2 = E[3], st1 = st2 * E[2], st0 = st1 * E[1];
+  const unsigned E1 = o1 ? E[1] : E[0], E2 = o2 == 1 ? E[1] : E[2], nslab = E1 * E2, nel = ES * EF;
+  const Div      qs(ES, mul), qf(EF, mul), qe(E2, mul);
+  const long     sxS = B.sx[kS], syS = B.sy[kS], sxF = sx[3], syF = sy[3];
+  const long     sx1 = o1 ? sx[1] : sx[0], sy1 = o1 ? sy[1] : sy[0];
+  const long     sx2 = o2 == 1 ? sx[1] : sx[2], sy2 = o2 == 1 ? sy[1] : sy[2];
+  const unsigned d1 = o1 ? st1 : st0, d2 = o2 == 1 ? st1 : st2, dS = kS == 0 ? st0 : kS == 1 ? st1 : st2;
   // every thread of the workgroup runs the same slab loop, so the barriers
   // below are reached by all of them
   for(unsigned sl = blockIdx.x; sl < nslab; sl += gridDim.x) {
-    const unsigned a = sl / E2, b = sl - a * E2;
+    const unsigned a = qe(sl), b = sl - a * E2;
+    const long     px = a * sx1 + b * sx2, py = a * sy1 + b * sy2;
     __syncthreads();  // the previous slab's LDS reads are done
     for(unsigned e = threadIdx.x; e < nel; e += GT) {
-      const unsigned f = e / ES, s = e - f * ES;
-      long           x[4];
-#pragma unroll
-      for(int d = 0; d < 4; d++)
-        x[d] = x0[d] + (d == fd ? s : d == dF ? f : d == d1 ? a : d == d2 ? b : 0u);
-      slab[s * ld + f] = B.alpha * so_value(S, B.kind, sp, x);
+      const unsigned f = qs(e), s = e - f * ES;
+      slab[s * ld + f] = value(px + s * sxS + f * sxF, py + s * syS + f * syF);
     }
     __syncthreads();
-    const unsigned base = a * st[o1] + b * st[o2];
+    const unsigned base = a * d1 + b * d2;
     for(unsigned e = threadIdx.x; e < nel; e += GT) {
-      const unsigned s = e / EF, f = e - s * EF;
-      dst[base + s * st[kS] + f] = slab[s * ld + f];
+      const unsigned s = qf(e), f = e - s * EF;
+      dst[base + s * dS + f] = slab[s * ld + f];
     }
   }
 }
@@ -162,9 +124,7 @@ __global__ void k_expand_t(GatherSrc S, double* __restrict__ t1_so, double* __re
   if(t1_so)
     for(long a = blockIdx.y; a < nv; a += gridDim.y)
       for(long i = (long) blockIdx.x * blockDim.x + threadIdx.x; i < no; i += (long) gridDim.x * blockDim.x) {
-        const long x[4]  = {a % S.V, i % S.O, 0, 0};
-        const int  sp[4] = {(int) (a / S.V), (int) (i / S.O), 0, 0};
-        t1_so[a * no + i] = so_value(S, kGatherT1, sp, x);
+        t1_so[a * no + i] = a / S.V == i / S.O ? S.t1[(a % S.V) * S.O + i % S.O] : 0.0;
       }
   if(t2_so) {
     // spin = index >= n, spatial = index - spin * n: no divide per element
@@ -177,10 +137,53 @@ __global__ void k_expand_t(GatherSrc S, double* __restrict__ t1_so, double* __re
       for(unsigned q = blockIdx.x * blockDim.x + threadIdx.x; q < nq; q += gridDim.x * blockDim.x) {
         const unsigned i = q / uno, j = q - i * uno;
         const int      si = i >= uo, sj = j >= uo;
-        const long     x[4]  = {a - sa * S.V, b - sb * S.V, (long) (i - si * uo), (long) (j - sj * uo)};
-        const int      sp[4] = {sa, sb, si, sj};
-        row[q]               = so_value(S, kGatherT2, sp, x);
+        const long     ab = ((a - sa * S.V) * S.V + (b - sb * S.V)) * S.O, i0 = i - si * uo, j0 = j - sj * uo;
+        const bool     on1 = sa == si && sb == sj, on2 = sa == sj && sb == si;
+        const double   u = on1 ? S.t2h[(ab + i0) * S.Op + j0] : 0.0, w = on2 ? S.t2h[(ab + j0) * S.Op + i0] : 0.0;
+        row[q]           = on1 && on2 ? u - w : on1 ? u : on2 ? -w : 0.0;
       }
+    }
+  }
+}
+
+// The same T2 for occupied spaces whose O x O block fits LDS: a workgroup holds
+// t2(a, b) of one spatial pair and writes its four spin rows, each one run of
+// 16-byte stores of two elements.  Bound: the write of 8 (2V)^2 (2O)^2 bytes
+// (an element-wise kernel made two dependent reads behind spin tests per
+// element: 2.3 TB/s at O=20, V=120).  t2_so must be 16-byte aligned.
+constexpr int kExpandMaxO = 84;  // O (O + 1) doubles of LDS
+
+__global__ void __launch_bounds__(256) k_expand_t2(GatherSrc S, double* __restrict__ t2_so) {
+  extern __shared__ double t[];
+  const unsigned O = (unsigned) S.O, ld = O + 1, oo = O * O, np = 2 * oo;  // pairs of elements per row
+  const long     V = S.V, nv = 2 * V;
+  const Div      q(O, true);
+  for(long p = blockIdx.x; p < V * V; p += gridDim.x) {
+    const long a = p / V, b = p - a * V;
+    __syncthreads();  // the previous pair's reads are done
+    for(unsigned x = threadIdx.x; x < oo; x += 256) {
+      const unsigned i = q(x), j = x - i * O;
+      t[i * ld + j] = S.t2h[(p * O + i) * S.Op + j];
+    }
+    __syncthreads();
+    double2* row[4];
+#pragma unroll
+    for(int s = 0; s < 4; s++)
+      row[s] = reinterpret_cast<double2*>(t2_so + (((s >> 1) * V + a) * nv + (s & 1) * V + b) * (4l * oo));
+    for(unsigned x = threadIdx.x; x < np; x += 256) {
+      const unsigned I = q(x), J = 2 * (x - I * O), si = I >= O, i = I - si * O;  // O pairs per I
+      double         v[4][2];
+#pragma unroll
+      for(int k = 0; k < 2; k++) {
+        const unsigned sj = J + k >= O, j = J + k - sj * O;
+        const double   u = t[i * ld + j], w = t[j * ld + i];
+        v[0][k] = !si && !sj ? u - w : 0.0;
+        v[3][k] = si && sj ? u - w : 0.0;
+        v[1][k] = !si && sj ? u : si && !sj ? -w : 0.0;
+        v[2][k] = si && !sj ? u : !si && sj ? -w : 0.0;
+      }
+#pragma unroll
+      for(int s = 0; s < 4; s++) row[s][x] = make_double2(v[s][0], v[s][1]);
     }
   }
 }
@@ -188,14 +191,21 @@ __global__ void k_expand_t(GatherSrc S, double* __restrict__ t1_so, double* __re
 }  // namespace
 
 int launch_expand_t(const GatherSrc& S, double* t1_so, double* t2_so, void* stream) {
+  if(t2_so && S.O <= kExpandMaxO && ((uintptr_t) t2_so & 15) == 0) {
+    hipLaunchKernelGGL(k_expand_t2, dim3((unsigned) std::min<long>(S.V * S.V, 1l << 16)), dim3(256),
+                       (unsigned) (sizeof(double) * S.O * (S.O + 1)), (hipStream_t) stream, S, t2_so);
+    const hipError_t e = hipGetLastError();
+    if(e != hipSuccess || !t1_so) return (int) e;
+    t2_so = nullptr;  // T1 below
+  }
   const long     no = 2 * S.O, nv = 2 * S.V;
-  const unsigned gx = (unsigned) std::min<long>((no * no + 255) / 256, 64);
-  const unsigned gy = (unsigned) std::min<long>(nv * nv, 65535);
+  const unsigned gx = (unsigned) std::min<long>(((t2_so ? no * no : no) + 255) / 256, 64);
+  const unsigned gy = (unsigned) std::min<long>(t2_so ? nv * nv : nv, 65535);
   hipLaunchKernelGGL(k_expand_t, dim3(gx, gy), dim3(256), 0, (hipStream_t) stream, S, t1_so, t2_so);
   return (int) hipGetLastError();
 }
 
-int launch_gather(const GatherBlock* blocks, int n_blocks, long max_elems, const GatherSrc& S,
+int launch_gather(const GatherDesc* blocks, int n_blocks, long max_elems, const GatherSrc& S,
                   const GatherDst& D, void* stream) {
   if(n_blocks <= 0) return 0;
   if(n_blocks > 65535) return (int) hipErrorInvalidConfiguration;

@@ -332,9 +332,10 @@ struct xt_ctx {
   long                dev_tasks_n = -1;
   // device-side gather: block descriptors of the last call (device copy and
   // the host list it was uploaded from, kept alive until the next call)
-  xt::GatherBlock*              d_gather     = nullptr;
+  xt::GatherDesc*               d_gather     = nullptr;
   long                          d_gather_cap = 0;
-  std::vector<xt::GatherBlock>  h_gather;
+  std::vector<xt::GatherBlock>  h_blocks;
+  std::vector<xt::GatherDesc>   h_gather;
   long                          gather_elems = 0;  // doubles written by the last gather
   hipEvent_t          ev0 = nullptr, ev1 = nullptr;
   double              last_ms = 0.0;
@@ -1404,15 +1405,18 @@ int xt_gather_task(xt_ctx* c, const long* task, void* stream, double* d1_t2, dou
     const long lo = occ ? 0 : P.noab, hi = occ ? P.noab : P.noab + P.nvab;
     if(task[k] < lo || task[k] >= hi) return fail(XT_EINVAL, "xt_gather_task: tile index out of range");
   }
-  xt::plan_gather(gather_tiling(c), P.restricted, task, c->h_gather, s1_size, s1_exec, d1_size,
+  xt::plan_gather(gather_tiling(c), P.restricted, task, c->h_blocks, s1_size, s1_exec, d1_size,
                   d1_exec, d2_size, d2_exec, counts);
-  const long n = (long) c->h_gather.size();
+  const long n  = (long) c->h_blocks.size();
+  const long Op = (P.O + 7) / 8 * 8, Vp = (P.V + 7) / 8 * 8;
   c->gather_elems = 0;
-  for(const auto& B: c->h_gather) {
+  for(const auto& B: c->h_blocks) {
     if(B.n >= (1l << 31)) return fail(XT_EINVAL, "xt_gather_task: block of 2^31 or more doubles");
     c->gather_elems += B.n;
   }
   if(n == 0) return XT_OK;
+  c->h_gather.clear();
+  for(const auto& B: c->h_blocks) c->h_gather.push_back(xt::gather_desc(B, P.O, P.V, Op, Vp));
   XT_HIP(hipSetDevice(c->device));
   hipStream_t st = (hipStream_t) stream;
   if(n > c->d_gather_cap) {
@@ -1421,23 +1425,22 @@ int xt_gather_task(xt_ctx* c, const long* task, void* stream, double* d1_t2, dou
     if(c->d_gather) (void) hipFree(c->d_gather);
     c->d_gather     = nullptr;
     c->d_gather_cap = 0;
-    XT_HIP(hipMalloc((void**) &c->d_gather, sizeof(xt::GatherBlock) * n));
+    XT_HIP(hipMalloc((void**) &c->d_gather, sizeof(xt::GatherDesc) * n));
     c->d_gather_cap = n;
   }
-  XT_HIP(hipMemcpyAsync(c->d_gather, c->h_gather.data(), sizeof(xt::GatherBlock) * n,
+  XT_HIP(hipMemcpyAsync(c->d_gather, c->h_gather.data(), sizeof(xt::GatherDesc) * n,
                         hipMemcpyHostToDevice, st));
   long max_elems = 0;
   for(const auto& B: c->h_gather) max_elems = std::max(max_elems, B.n);
-  xt::GatherSrc S;
-  S.O    = P.O;
-  S.V    = P.V;
-  S.Op   = (P.O + 7) / 8 * 8;
-  S.Vp   = (P.V + 7) / 8 * 8;
-  S.t1   = c->in.t1;
-  S.t2h  = c->in.t2h;
-  S.vvoo = c->in.vvoo;
-  S.ovk  = c->in.ovk;
-  S.xv   = c->in.xv;
+  xt::GatherSrc S = {};
+  S.O             = P.O;
+  S.V             = P.V;
+  S.Op            = Op;
+  S.Vp            = Vp;
+  S.t1            = c->in.t1;
+  S.t2h           = c->in.t2h;
+  const double* arrays[xt::kGatherArrays] = {c->in.t1, c->in.t2h, c->in.t2p, c->in.vvoo, c->in.ovk, c->in.xv};
+  std::copy(arrays, arrays + xt::kGatherArrays, S.a);
   xt::GatherDst D = {{d1_t2, d1_v2, d2_t2, d2_v2, s1_t1, s1_v2}};
   const int     err = xt::launch_gather(c->d_gather, (int) n, max_elems, S, D, st);
   if(err) return fail(XT_EHIP, std::string("xt_gather_task: ") + hipGetErrorString((hipError_t) err));

@@ -715,12 +715,20 @@ __global__ void __launch_bounds__(256) k_vvoo_asym(const double* __restrict__ vv
       if(a <= b) d = fmax(d, fabs(u - y[j * o + i]));
     }
   }
+  __shared__ double rd[4], rm[4];
 #pragma unroll
   for(int k = 32; k >= 1; k >>= 1) {
     d = fmax(d, __shfl_xor(d, k, 64));
     m = fmax(m, __shfl_xor(m, k, 64));
   }
   if((threadIdx.x & 63) == 0) {
+    rd[threadIdx.x >> 6] = d;
+    rm[threadIdx.x >> 6] = m;
+  }
+  __syncthreads();
+  if(threadIdx.x == 0) {  // one pair of atomics per workgroup: they all meet at two addresses
+    d = fmax(fmax(rd[0], rd[1]), fmax(rd[2], rd[3]));
+    m = fmax(fmax(rm[0], rm[1]), fmax(rm[2], rm[3]));
     atomicMax(&out[0], (unsigned long long) __double_as_longlong(d));
     atomicMax(&out[1], (unsigned long long) __double_as_longlong(m));
   }
@@ -729,7 +737,7 @@ __global__ void __launch_bounds__(256) k_vvoo_asym(const double* __restrict__ vv
 int launch_vvoo_asym(const double* vvoo, int O, int V, unsigned long long* out, void* stream) {
   const int rc = launch_zero_u64(out, 2, stream);
   if(rc) return rc;
-  hipLaunchKernelGGL(k_vvoo_asym, dim3((unsigned) std::min<long>((long) V * V, 4096)), dim3(256), 0,
+  hipLaunchKernelGGL(k_vvoo_asym, dim3((unsigned) std::min<long>((long) V * V, 1024)), dim3(256), 0,
                      (hipStream_t) stream, vvoo, (long) O, (long) V, out);
   return (int) hipGetLastError();
 }
