@@ -195,23 +195,32 @@ int xt_mlp_train(xt_mlp* m, long n, const float* x, const float* t, int steps, f
   float* hist = loss_hist ? m->hist : nullptr;
   // step[1] = step[0]: base of this call's loss history
   XT_HIP(hipMemcpyAsync(m->W.step + 1, m->W.step, sizeof(int), hipMemcpyDeviceToDevice, m->stream));
-  // one Adam step captured once, replayed `steps` times
-  XT_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-  int        err = xt::mlp_train_step(m->W, n, lr, hist, m->stream);
-  hipGraph_t g   = nullptr;
-  hipError_t e   = hipStreamEndCapture(m->stream, &g);
-  if(err || e != hipSuccess) {
-    if(g) (void) hipGraphDestroy(g);
-    return xt::set_error(XT_EHIP, std::string("mlp training capture: ") +
-                                    hipGetErrorString(err ? (hipError_t) err : e));
+  // kReplay Adam steps captured once and replayed; the rest launched directly.
+  // A step is two kernels of a few microseconds, less than a graph launch takes.
+  constexpr int  kReplay = 32;
+  hipGraphExec_t ge      = nullptr;
+  hipError_t     e       = hipSuccess;
+  int            err     = 0;
+  if(steps >= 2 * kReplay) {
+    XT_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
+    for(int s = 0; s < kReplay && !err; s++) err = xt::mlp_train_step(m->W, n, lr, hist, m->stream);
+    hipGraph_t g = nullptr;
+    e            = hipStreamEndCapture(m->stream, &g);
+    if(err || e != hipSuccess) {
+      if(g) (void) hipGraphDestroy(g);
+      return xt::set_error(XT_EHIP, std::string("mlp training capture: ") +
+                                      hipGetErrorString(err ? (hipError_t) err : e));
+    }
+    e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
+    (void) hipGraphDestroy(g);
+    if(e != hipSuccess) return xt::set_error(XT_EHIP, std::string("mlp graph: ") + hipGetErrorString(e));
   }
-  hipGraphExec_t ge = nullptr;
-  e                 = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-  (void) hipGraphDestroy(g);
-  if(e != hipSuccess) return xt::set_error(XT_EHIP, std::string("mlp graph: ") + hipGetErrorString(e));
-  for(int s = 0; s < steps && e == hipSuccess; s++) e = hipGraphLaunch(ge, m->stream);
+  int left = steps;
+  for(; ge && left >= kReplay && e == hipSuccess; left -= kReplay) e = hipGraphLaunch(ge, m->stream);
+  for(; left > 0 && e == hipSuccess; left--)
+    e = (hipError_t) xt::mlp_train_step(m->W, n, lr, hist, m->stream);
   hipError_t e2 = hipStreamSynchronize(m->stream);
-  (void) hipGraphExecDestroy(ge);
+  if(ge) (void) hipGraphExecDestroy(ge);
   if(e != hipSuccess || e2 != hipSuccess)
     return xt::set_error(XT_EHIP, std::string("mlp training: ") +
                                     hipGetErrorString(e != hipSuccess ? e : e2));
