@@ -233,16 +233,12 @@ constexpr int kMaxNoab = 50, kMaxNvab = 140;
 // The launcher's packed metadata, in ints: the host arrays d1_size[7*noab],
 // d1_exec[9*noab], d2_size[7*nvab], d2_exec[9*nvab], s1_size[6], s1_exec[9],
 // then the K tile lists the host builds from them: kKlistCountInts counts
-// (one per bipartition: entries | d1 entries << 16, then padding to a
-// 16-byte boundary) and, for bipartition g = 0..8 in turn, entries + 1 int4
-// (family 0 d1 / 1 d2, exec slot, K, first packed k; the last entry holds the
-// total K in .w).  The first d2 tile starts on a multiple of kPackedKC, the
-// kernel's K chunk, so that every chunk reads one family.
+// (one per bipartition: its entries) and, for bipartition g = 0..8 in turn, an
+// int4 per enabled K tile (family 0 d1 / 1 d2, exec slot, K, 0).
 // kPackedMetaInts is the size at the reference's tile-count limits.
-constexpr int kPackedKC       = 16;
 constexpr int kKlistCountInts = 9;  // 15 + 9 ints after the size/exec arrays: 16-byte aligned
 constexpr int kPackedMetaInts =
-  16 * kMaxNoab + 16 * kMaxNvab + 15 + kKlistCountInts + 4 * 9 * (kMaxNoab + kMaxNvab + 1);
+  16 * kMaxNoab + 16 * kMaxNvab + 15 + kKlistCountInts + 4 * 9 * (kMaxNoab + kMaxNvab);
 static_assert((15 + kKlistCountInts) % 4 == 0, "tile lists must start on a 16-byte boundary");
 static_assert(kPackedMetaInts % 4 == 0, "metadata slots must keep 16-byte alignment");
 struct PackedArgs {

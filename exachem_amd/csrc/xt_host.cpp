@@ -1736,7 +1736,7 @@ int packed_prepare(const char* fn, const PackedCall& P, int* meta, int* n_meta, 
   for(size_t b = 0; b < P.nvab; b++)
     if(P.d2_size[7 * b + 6] <= 0 || P.d2_size[7 * b + 6] > 4096)
       return fail(XT_EINVAL, f + ": bad p7 tile size");
-  // the kernel keeps an exec slot in 30 bits of its LDS tile list
+  // exec slots are limited to 30 bits
   for(size_t i = 0; i < 9 * P.noab; i++)
     if(P.d1_exec[i] >= (1 << 30)) return fail(XT_EINVAL, f + ": d1 exec slot out of range");
   for(size_t i = 0; i < 9 * P.nvab; i++)
@@ -1754,39 +1754,26 @@ int packed_prepare(const char* fn, const PackedCall& P, int* meta, int* n_meta, 
   put(P.s1_exec, 9);
   // K tile lists of the nine bipartitions g = 3*hs + ps: the enabled d1
   // tiles (h7b) with their exec slot for d1 equation 3*((ps+1)%3) + hs, then
-  // the enabled d2 tiles (p7b) for d2 equation 3*ps + (hs+1)%3, packed end to
-  // end except that the d2 tiles start on a chunk boundary
+  // the enabled d2 tiles (p7b) for d2 equation 3*ps + (hs+1)%3
   // (ccsd_t_all_fused_cpu.hpp:173-270, 331-428)
   int* counts = m;
   m += xt::kKlistCountInts;
   for(int g = 0; g < 9; g++) {
     const int hs = g / 3, ps = g % 3, s1d = 3 * ((ps + 1) % 3) + hs, s2d = 3 * ps + (hs + 1) % 3;
-    int       n = 0, nd1 = 0, kb = 0;
-    auto      entry = [&](int fam, int ex, int K, int k0) {
+    int       n     = 0;
+    auto      entry = [&](int fam, int ex, int K) {
       m[0] = fam;
       m[1] = ex;
       m[2] = K;
-      m[3] = k0;
+      m[3] = 0;
       m += 4;
+      n++;
     };
-    for(size_t tb = 0; tb < P.noab; tb++) {
-      const int ex = P.d1_exec[s1d + 9 * tb];
-      if(ex < 0) continue;
-      entry(0, ex, P.d1_size[3 + 7 * tb], kb);
-      kb += P.d1_size[3 + 7 * tb];
-      n++;
-    }
-    nd1 = n;
-    for(size_t tb = 0; tb < P.nvab; tb++) {
-      const int ex = P.d2_exec[s2d + 9 * tb];
-      if(ex < 0) continue;
-      if(n == nd1) kb = (kb + xt::kPackedKC - 1) / xt::kPackedKC * xt::kPackedKC;
-      entry(1, ex, P.d2_size[6 + 7 * tb], kb);
-      kb += P.d2_size[6 + 7 * tb];
-      n++;
-    }
-    entry(0, 0, 0, kb);
-    counts[g] = n | nd1 << 16;
+    for(size_t tb = 0; tb < P.noab; tb++)
+      if(P.d1_exec[s1d + 9 * tb] >= 0) entry(0, P.d1_exec[s1d + 9 * tb], P.d1_size[3 + 7 * tb]);
+    for(size_t tb = 0; tb < P.nvab; tb++)
+      if(P.d2_exec[s2d + 9 * tb] >= 0) entry(1, P.d2_exec[s2d + 9 * tb], P.d2_size[6 + 7 * tb]);
+    counts[g] = n;
   }
   *n_meta = (int) (m - meta);
   for(int i = 0; i < 6; i++) A.dim[i] = (int) P.d[i];

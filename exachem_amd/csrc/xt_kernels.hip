@@ -33,6 +33,7 @@
 namespace xt {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 constexpr int NT      = 256;       // threads per workgroup
 constexpr int KC      = 16;        // K chunk staged per LDS round
@@ -121,10 +122,18 @@ __device__ __forceinline__ Quad quadrant(int g, int rows, int cols) {
   return q;
 }
 
-// Box index parts of the rows and columns of the current bipartition (e =
-// sum_pos idx[pos] << 2*pos, pos 0..2 = h1..h3, 3..5 = p4..p6), written by 128
-// threads.  Padding rows and columns get an index outside the tile (some
+// Box index part of a row or column (sum_pos idx[pos] << 2*pos, pos 0..2 =
+// h1..h3, 3..5 = p4..p6).  Padding ones get an index outside the tile (some
 // extent of their side is short wherever there is one).
+__device__ __forceinline__ unsigned short box_index(Item x, int e0, int e1, int e2, int q0, int q1, int q2) {
+  if(x.c >= e2) {
+    x.a = e0 < 4 ? e0 : 0;
+    x.b = e0 < 4 ? 0 : e1 < 4 ? e1 : 0;
+    x.c = e0 < 4 || e1 < 4 ? 0 : e2 & 3;
+  }
+  return (unsigned short) ((x.a << (2 * q0)) | (x.b << (2 * q1)) | (x.c << (2 * q2)));
+}
+// Those of the current bipartition of the per-task kernel, written by 128 threads.
 struct Tables {
   unsigned short row[64], col[64];
 };
@@ -135,13 +144,7 @@ __device__ __forceinline__ void fill_tables(Tables& t, const int* ext, int hs, i
   const bool row = tid < 64;
   const int  q0 = row ? hs : hA, q1 = row ? 3 + pA : hB, q2 = 3 + (row ? pB : ps);
   const int  e0 = ext[q0], e1 = ext[q1], e2 = ext[q2];
-  Item       x = item_of(tid & 63, e0, e1);
-  if(x.c >= e2) {
-    x.a = e0 < 4 ? e0 : 0;
-    x.b = e0 < 4 ? 0 : e1 < 4 ? e1 : 0;
-    x.c = e0 < 4 || e1 < 4 ? 0 : e2 & 3;
-  }
-  const unsigned short v = (unsigned short) ((x.a << (2 * q0)) | (x.b << (2 * q1)) | (x.c << (2 * q2)));
+  const unsigned short v = box_index(item_of(tid & 63, e0, e1), e0, e1, e2, q0, q1, q2);
   if(row) t.row[tid] = v;
   else t.col[tid - 64] = v;
 }
@@ -186,10 +189,11 @@ __device__ __forceinline__ void acc_ready(v4d (&c)[2][2]) {
 template<int KCT = KC, int LDKT = LDK>
 __device__ __forceinline__ void mfma_chunk(const double* __restrict__ As,
                                            const double* __restrict__ Bs, const Quad& q,
-                                           v4d (&acc)[2][2]) {
+                                           v4d (&acc)[2][2], int len = KCT) {
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
 #pragma unroll
   for(int kk = 0; kk < KCT / 4; kk++) {
+    if(4 * kk >= len) break;
     const int    k  = 4 * kk + lk;
     const double a0 = As[(16 * q.wm + lr) * LDKT + k], a1 = As[(16 * q.wm + 32 + lr) * LDKT + k];
     const double b0 = Bs[(16 * q.wn + lr) * LDKT + k], b1 = Bs[(16 * q.wn + 32 + lr) * LDKT + k];
@@ -220,56 +224,89 @@ __device__ __forceinline__ void acc_to_t3(double* t3, const Tables& t, const Qua
     }
 }
 
-// Energy of the finished sub-tile: t3d in LDS, s1 operands staged in LDS,
-// denominators from sm.eps, ext the orbitals inside the tile.  Returns (E4,
-// E5) partial sums in thread 0.
+// Energy of the finished sub-tile: t3d in LDS, s1 operands staged in LDS (zero
+// for slots that are off), denominators from sm.eps, ext the orbitals inside the
+// tile.  Returns (E4, E5) partial sums in thread 0.
 //   T1s[s][pa][hi] (16 per slot), V1s[s][hk + 4 hj + 16 pc + 64 pb] (256 per slot)
-// A thread owns one (h1, h2, h3, p4) and runs over p5 and p6.
+// A thread owns one (h1, h2, h3, p4) and runs over p5 and p6.  Bound by vector
+// instructions: what depends on p6 or p5 alone is read once for it (99 reads for
+// 16 elements, not 288).
 template<class SM>
 __device__ __forceinline__ void subtile_energy(SM& sm, const double* T1s, const double* V1s,
-                                               const int* ext, unsigned s1mask, double& e4,
-                                               double& e5) {
+                                               const int* ext, double& e4, double& e5) {
   e4 = 0.0;
   e5 = 0.0;
   const int tid = threadIdx.x;
-  int       idx[6];
+  int       h[3];
 #pragma unroll
-  for(int p = 0; p < 4; p++) idx[p] = (tid >> (2 * p)) & 3;
-  if(idx[0] < ext[0] && idx[1] < ext[1] && idx[2] < ext[2] && idx[3] < ext[3]) {
+  for(int p = 0; p < 3; p++) h[p] = (tid >> (2 * p)) & 3;
+  const int p4 = tid >> 6;
+  const int n5 = __builtin_amdgcn_readfirstlane(ext[4]), n6 = __builtin_amdgcn_readfirstlane(ext[5]);
+  if(h[0] < ext[0] && h[1] < ext[1] && h[2] < ext[2] && p4 < ext[3]) {
+    // slot 3 pa + hi: T1(p, hi) V1(hj, hk, pb, pc)
+    double    t0[3], t2[3][4], v1[3][4];
+    const double *T[3], *V[3];
+#pragma unroll
+    for(int hi = 0; hi < 3; hi++) {
+      int hj, hk;
+      pair_of(hi, hj, hk);
+      T[hi]  = T1s + hi * 16 + h[hi];
+      V[hi]  = V1s + hi * 256 + h[hk] + 4 * h[hj];
+      t0[hi] = T[hi][4 * p4];
+#pragma unroll
+      for(int p6 = 0; p6 < 4; p6++) {
+        t2[hi][p6] = T[hi][6 * 16 + 4 * p6];
+        v1[hi][p6] = V[hi][3 * 256 + 16 * p6 + 64 * p4];
+      }
+    }
+    const double Dh = sm.eps[8 + h[2]] + sm.eps[4 + h[1]] + sm.eps[h[0]], D4 = sm.eps[12 + p4];
 #pragma unroll 1
-    for(idx[5] = 0; idx[5] < ext[5]; idx[5]++)
-#pragma unroll 1
-      for(idx[4] = 0; idx[4] < ext[4]; idx[4]++) {
-        const double d = sm.t3[tid + NT * (idx[4] + 4 * idx[5])];
+    for(int p5 = 0; p5 < n5; p5++) {
+      double t1[3], v2[3];
+#pragma unroll
+      for(int hi = 0; hi < 3; hi++) {
+        t1[hi] = T[hi][3 * 16 + 4 * p5];
+        v2[hi] = V[hi][6 * 256 + 16 * p5 + 64 * p4];
+      }
+#pragma unroll
+      for(int p6 = 0; p6 < 4; p6++) {
+        if(p6 >= n6) break;
+        const double d = sm.t3[tid + NT * (p5 + 4 * p6)];
         double       s = 0.0;
 #pragma unroll
-        for(int slot = 0; slot < 9; slot++) {
-          if(!((s1mask >> slot) & 1)) continue;
-          const int pa = slot / 3, hi = slot % 3;
-          int       hj, hk, pb, pc;
-          pair_of(hi, hj, hk);
-          pair_of(pa, pb, pc);
-          s += T1s[slot * 16 + idx[3 + pa] * 4 + idx[hi]] *
-               V1s[slot * 256 + idx[hk] + 4 * idx[hj] + 16 * idx[3 + pc] + 64 * idx[3 + pb]];
-        }
+        for(int hi = 0; hi < 3; hi++) s += t0[hi] * V[hi][16 * p6 + 64 * p5];
+#pragma unroll
+        for(int hi = 0; hi < 3; hi++) s += t1[hi] * v1[hi][p6];
+#pragma unroll
+        for(int hi = 0; hi < 3; hi++) s += t2[hi][p6] * v2[hi];
         // denominator in the reference's order (ccsd_t_all_fused_cpu.hpp:612-614)
-        const double D = sm.eps[8 + idx[2]] + sm.eps[4 + idx[1]] + sm.eps[idx[0]] -
-                         sm.eps[20 + idx[5]] - sm.eps[16 + idx[4]] - sm.eps[12 + idx[3]];
+        const double D = Dh - sm.eps[20 + p6] - sm.eps[16 + p5] - D4;
         e4 += d * d / D;
         e5 += d * (d + s) / D;
       }
+    }
   }
   block_sum2(sm, e4, e5);
 }
+
+// Rows and columns of a bipartition: index parts in the 4^6 box (as
+// fill_tables), of it and the next one, and the rows of the d1 and d2 operand
+// arrays, of the next one.
+struct Rows {
+  unsigned       r1[128], r2[128];
+  unsigned short e[2][128];
+};
 
 // LDS of the persistent FP64 kernel, sized for three workgroups per CU.
 struct __align__(16) Smem {
   double t3[T3N];
   double stage[STAGE_D];
-  double t1s[S1_T1];  // s1 T1 blocks
+  union {
+    Rows   tab;
+    double t1s[S1_T1];  // later: the s1 T1 blocks
+  };
   double eps[24];
   double red[8];
-  Tables tab;
   int    start[6], ext[6];  // current sub-tile: first orbitals, orbitals inside the tile
 };
 
@@ -278,126 +315,355 @@ struct __align__(16) Smem {
 // tensors (spin-orbital antisymmetrised values of <pq||rs> and T2, exactly the
 // numbers the reference's gathers would copy out of TAMM blocks).
 // ---------------------------------------------------------------------------
-// One staged operand row: pointer to its contraction run and the coefficient
-// (+-1 or 0) that folds the equation sign and the spin-orbital selection.
-struct RowPtr {
-  const double* p;
-  double        c;
-};
+__device__ __forceinline__ unsigned uni(int x) { return (unsigned) __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+  return (uint64_t) (unsigned) __builtin_amdgcn_readfirstlane((int) v) |
+         (uint64_t) (unsigned) __builtin_amdgcn_readfirstlane((int) (v >> 32)) << 32;
+}
 
-// Four consecutive k of a row (k0 a multiple of 4; rows are padded to a
-// multiple of 8, so the run stays inside the row).
-__device__ __forceinline__ void fetch4(const RowPtr& rp, int k0, int Kp, double* x) {
-  if(rp.c != 0.0 && k0 < Kp) {
-    const double2* q  = reinterpret_cast<const double2*>(rp.p + k0);
-    double2        v0 = q[0], v1 = q[1];
-    x[0] = v0.x; x[1] = v0.y; x[2] = v1.x; x[3] = v1.y;
-  }
-  else {
+// The MFMA tiles of one wave: row tiles i0 + is * i (i < ni) times column tiles
+// j0 + js * j (j < nj) of the mt x nt that are needed, dealt out as evenly as
+// four waves allow with at most four operand rows a lane.  Wave w takes the
+// share (w + g) % 4, so that over the bipartitions every SIMD gets the larger
+// ones in turn.
+struct Share {
+  int i0, is, ni, j0, js, nj;
+};
+__device__ __forceinline__ Share wave_share(int g, int rows, int cols) {
+  const int w = (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + g) & 3;
+  const int mt = (rows + 15) >> 4, nt = (cols + 15) >> 4, wm = w >> 1, wn = w & 1;
+  if(mt == 1) return {0, 1, w < nt, w, 1, 1};
+  if(nt == 1) return {w, 1, w < mt, 0, 1, 1};
+  if(mt == 3 && nt == 3) return w == 0 ? Share{0, 1, 3, 0, 1, 1} : Share{w - 1, 1, 1, 1, 1, 2};
+  if(mt == 3 && nt == 4) return {0, 1, 3, w, 1, 1};
+  if(mt == 4 && nt == 3) return {w, 1, 1, 0, 1, 3};
+  return {wm, 2, wm + 2 < mt ? 2 : 1, wn, 2, wn + 2 < nt ? 2 : 1};
+}
+
+// NI x NJ MFMA tiles of one wave over a bipartition's K, n1 units of 8 of d1 and
+// n2 of d2, two units a chunk, a last odd one alone, then added into t3 (the
+// first bipartition of a sub-tile stores instead: every bipartition covers
+// every element of the tile).  refill() writes the chunk in flight to As and Bs
+// and has the one after it loaded; refill_whole() does so for a whole chunk with
+// at least another whole one of the family to load (left() units, skip() counts
+// them off); ahead() runs before the sums are added.  neg1, neg2: signs of the
+// families' products.  Every wave passes the same barriers, with NI = NJ = 0 for
+// a wave without tiles.
+// While an FP64 matrix instruction runs, no vector instruction of any wave
+// issues on its SIMD (measured: a wave of additions beside one of matrix
+// instructions stood still until that had ended; beside the 16-bit forms it ran
+// at 80%), and waves that wait to prepare a chunk wait for the others' products.
+// So the inner loop has none: fragments at fixed LDS addresses, a refill from
+// scalar bases and fixed vector offsets, signs left to the sums.  With 30 vector
+// and 40 scalar instructions a chunk here 12 tasks of O=40, V=300 took 65.8 ms,
+// with none and 8 52.8 (FP64 matrix instructions 53% and 66% of the time).
+// Operands straight from global memory into the fragments were slower (87 ms:
+// neighbouring lanes are different rows, 64 cycles a load).
+// Lane (lr, lk) takes k = 2 lk, 2 lk + 1 of each unit: the order of k inside a
+// product is free as long as both sides agree, and this way a fragment is a
+// 16-byte read for two instructions.  D layout of v_mfma_f64_16x16x4f64: register
+// r of lane l holds row 4*r + (l>>4), column l&15 (the four row groups are
+// interleaved, unlike the 16-bit forms).
+template<int NI, int NJ, class Left, class Skip, class Whole, class Refill, class Ahead>
+__device__ __forceinline__ void wave_tiles(double* t3, const double* As, const double* Bs, const unsigned short* te,
+                                           const Share& q, bool store, int n1, int n2, bool neg1, bool neg2,
+                                           Left&& left, Skip&& skip, Whole&& refill_whole, Refill&& refill, Ahead&& ahead) {
+  constexpr int I = NI ? NI : 1, J = NJ ? NJ : 1;
+  const int     lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  int pa[I], pb[J];  // fragment rows in As and Bs, kept out of the loop
 #pragma unroll
-    for(int j = 0; j < 4; j++) x[j] = 0.0;
+  for(int i = 0; i < NI; i++) {
+    pa[i] = (16 * (q.i0 + q.is * i) + lr) * LDK + 2 * lk;
+    asm("" : "+v"(pa[i]));
+  }
+#pragma unroll
+  for(int j = 0; j < NJ; j++) {
+    pb[j] = (16 * (q.j0 + q.js * j) + lr) * LDK + 2 * lk;
+    asm("" : "+v"(pb[j]));
+  }
+  v4d acc[I][J];
+#pragma unroll
+  for(int i = 0; i < NI; i++)
+#pragma unroll
+    for(int j = 0; j < NJ; j++) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  struct Frag {
+    v2d a[I], b[J];
+  };
+  auto read = [&](Frag& f, int k) {
+#pragma unroll
+    for(int i = 0; i < NI; i++) f.a[i] = *reinterpret_cast<const v2d*>(&As[pa[i] + k]);
+#pragma unroll
+    for(int j = 0; j < NJ; j++) f.b[j] = *reinterpret_cast<const v2d*>(&Bs[pb[j] + k]);
+  };
+  auto mma = [&](const Frag& f) {
+#pragma unroll
+    for(int i = 0; i < NI; i++)
+#pragma unroll
+      for(int j = 0; j < NJ; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.a[i].x, f.b[j].x, acc[i][j], 0, 0, 0);
+#pragma unroll
+    for(int i = 0; i < NI; i++)
+#pragma unroll
+      for(int j = 0; j < NJ; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.a[i].y, f.b[j].y, acc[i][j], 0, 0, 0);
+  };
+  refill();  // the staging is free: every wave has read the last chunk before
+  bool d1 = n1 > 0;
+#pragma unroll 1
+  for(int n = d1 ? n1 : n2;;) {
+    Frag f0, f1;
+    // chunks that leave n and the load side in the middle of the family
+    const int w = max(min(n - 2, left()), 0) >> 1;
+#pragma unroll 1
+    for(int c = w; c > 0; c--) {
+      __syncthreads();
+      read(f0, 0);
+      read(f1, 8);
+      __syncthreads();
+      refill_whole();
+      mma(f0);
+      mma(f1);
+    }
+    n -= 2 * w;
+    if(w) skip(2 * w);
+    __syncthreads();
+    read(f0, 0);
+    read(f1, 8);
+    __syncthreads();
+    refill();
+    mma(f0);
+    if(n > 1) mma(f1);
+    n -= 2;
+    if(n > 0) continue;
+    if(!d1 || n2 == 0) break;
+    d1 = false;
+    n  = n2;
+    if(neg1 != neg2) {
+#pragma unroll
+      for(int i = 0; i < NI; i++)
+#pragma unroll
+        for(int j = 0; j < NJ; j++) acc[i][j] = -acc[i][j];
+    }
+  }
+  ahead();
+  const double sg = (n2 ? neg2 : neg1) ? -1.0 : 1.0;
+#pragma unroll
+  for(int i = 0; i < NI; i++)
+#pragma unroll
+    for(int j = 0; j < NJ; j++) {
+      const int c = te[64 + 16 * (q.j0 + q.js * j) + lr];
+      double*   p[4];
+#pragma unroll
+      for(int r = 0; r < 4; r++) p[r] = &t3[te[16 * (q.i0 + q.is * i) + 4 * r + lk] | c];
+      if(store) {
+#pragma unroll
+        for(int r = 0; r < 4; r++) *p[r] = sg * acc[i][j][r];
+      }
+      else {
+        double v[4];
+#pragma unroll
+        for(int r = 0; r < 4; r++) v[r] = *p[r];
+#pragma unroll
+        for(int r = 0; r < 4; r++) *p[r] = fma(sg, acc[i][j][r], v[r]);
+      }
+    }
+}
+template<class Left, class Skip, class Whole, class Refill, class Ahead>
+__device__ __forceinline__ void share_tiles(double* t3, const double* As, const double* Bs, const unsigned short* te,
+                                            const Share& q, bool store, int n1, int n2, bool neg1, bool neg2,
+                                            Left&& left, Skip&& skip, Whole&& refill_whole, Refill&& refill, Ahead&& ahead) {
+  switch(q.ni * 4 + q.nj) {
+    case 4 + 1: wave_tiles<1, 1>(t3, As, Bs, te, q, store, n1, n2, neg1, neg2, left, skip, refill_whole, refill, ahead); break;
+    case 4 + 2: wave_tiles<1, 2>(t3, As, Bs, te, q, store, n1, n2, neg1, neg2, left, skip, refill_whole, refill, ahead); break;
+    case 4 + 3: wave_tiles<1, 3>(t3, As, Bs, te, q, store, n1, n2, neg1, neg2, left, skip, refill_whole, refill, ahead); break;
+    case 8 + 1: wave_tiles<2, 1>(t3, As, Bs, te, q, store, n1, n2, neg1, neg2, left, skip, refill_whole, refill, ahead); break;
+    case 8 + 2: wave_tiles<2, 2>(t3, As, Bs, te, q, store, n1, n2, neg1, neg2, left, skip, refill_whole, refill, ahead); break;
+    case 12 + 1: wave_tiles<3, 1>(t3, As, Bs, te, q, store, n1, n2, neg1, neg2, left, skip, refill_whole, refill, ahead); break;
+    default: wave_tiles<0, 0>(t3, As, Bs, te, q, store, n1, n2, neg1, neg2, left, skip, refill_whole, refill, ahead); break;
+  }
+}
+
+// Operands of a bipartition for a sub-tile: of each family the addresses of the
+// sub-tile's first M and N row, the units of K and the sign of the product.
+// Rows c1*x - c2*y of the spin-orbital elements: both terms -> the
+// antisymmetrised array; one term -> that array, its sign in the product's.
+//   d1 M: t(pA,pB,hs,h7) - t(pA,pB,h7,hs) = t2h[pA,pB,hs,:] - t2h[pB,pA,hs,:]
+//   d1 N: (hA h7|hB ps) - (hB h7|hA ps) = ovk[hB,ps,hA,:] - ovk[hA,ps,hB,:]
+//   d2 M: (hs pA|p7 pB) - (hs pB|p7 pA) = xv[pB,pA,hs,:] - xv[pA,pB,hs,:]
+//   d2 N: t(ps,p7,hA,hB) - t(p7,ps,hA,hB) = t2p[hA,hB,ps,:] - t2p[hB,hA,ps,:]
+typedef const __attribute__((address_space(1))) char* GBytes;
+struct Runs {
+  GBytes a1, b1, a2, b2;
+  int    n1, n2;  // 0: family off
+  bool   neg1, neg2;
+};
+__device__ __forceinline__ Runs runs_of(const SpatialDev& S, const int* start, int g, unsigned c1, unsigned c2) {
+  const int hs = g / 3, ps = g % 3;
+  int       hA, hB, pA, pB;
+  pair_of(hs, hA, hB);
+  pair_of(ps, pA, pB);
+  const unsigned HS = uni(start[hs]), HA = uni(start[hA]), HB = uni(start[hB]);
+  const unsigned PS = uni(start[3 + ps]), PA = uni(start[3 + pA]), PB = uni(start[3 + pB]);
+  const uint64_t O = S.O, V = S.V;
+  auto           row = [](const double* p, uint64_t r, int K) { return (GBytes) (p + r * (unsigned) K); };
+  Runs           R;
+  R.a1   = row((c1 & 12) == 12 ? S.t2ha : S.t2h, (((c1 & 4) ? PA : PB) * V + ((c1 & 4) ? PB : PA)) * O + HS, S.Op);
+  R.b1   = row((c1 & 48) == 48 ? S.ovka : S.ovk, (((c1 & 16) ? HB : HA) * V + PS) * O + ((c1 & 16) ? HA : HB), S.Op);
+  R.a2   = row((c2 & 12) == 12 ? S.xva : S.xv, (((c2 & 4) ? PB : PA) * V + ((c2 & 4) ? PA : PB)) * O + HS, S.Vp);
+  R.b2   = row((c2 & 48) == 48 ? S.t2pa : S.t2p, (((c2 & 16) ? HA : HB) * O + ((c2 & 16) ? HB : HA)) * V + PS, S.Vp);
+  R.neg1 = ((c1 >> 1) ^ !(c1 & 4) ^ !(c1 & 16)) & 1;
+  R.neg2 = ((c2 >> 1) ^ !(c2 & 4) ^ !(c2 & 16)) & 1;
+  R.n1   = (c1 & 1) ? S.Op >> 3 : 0;
+  R.n2   = (c2 & 1) ? S.Vp >> 3 : 0;
+  return R;
+}
+// Tables of bipartition g, by 128 threads: rows relative to the sub-tile's first,
+// at most three of the slowest coordinate, which takes less than 24 bits of any
+// system whose operands fit the memory.
+__device__ __forceinline__ void fill_rows(Rows& t, int tb, const int* ext, int g, unsigned c1, unsigned c2,
+                                          unsigned O, unsigned V) {
+  const int tid = threadIdx.x, hs = g / 3, ps = g % 3;
+  if(tid >= 128) return;
+  int hA, hB, pA, pB;
+  pair_of(hs, hA, hB);
+  pair_of(ps, pA, pB);
+  const bool row = tid < 64;
+  const int  q0 = row ? hs : hA, q1 = row ? 3 + pA : hB, q2 = 3 + (row ? pB : ps);
+  const int  e0 = ext[q0], e1 = ext[q1], e2 = ext[q2];
+  Item       x  = item_of(tid & 63, e0, e1);
+  t.e[tb][tid]  = box_index(x, e0, e1, e2, q0, q1, q2);
+  if(x.c >= e2) x.a = x.b = x.c = 0;
+  const unsigned y0 = x.a, y1 = x.b, y2 = x.c;
+  if(row) {  // (hs, pA, pB)
+    t.r1[tid] = __umul24(__umul24((c1 & 4) ? y1 : y2, V) + ((c1 & 4) ? y2 : y1), O) + y0;
+    t.r2[tid] = __umul24(__umul24((c2 & 4) ? y2 : y1, V) + ((c2 & 4) ? y1 : y2), O) + y0;
+  }
+  else {  // (hA, hB, ps)
+    t.r1[tid] = __umul24(__umul24((c1 & 16) ? y1 : y0, V) + y2, O) + ((c1 & 16) ? y0 : y1);
+    t.r2[tid] = __umul24(__umul24((c2 & 16) ? y0 : y1, O) + ((c2 & 16) ? y1 : y0), V) + y2;
   }
 }
 
 __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, uint64_t d2code,
                                 uint64_t s1code, double& e4, double& e5) {
-  const int tid = threadIdx.x;
-  const int O = S.O, V = S.V;
+  const int      tid = threadIdx.x;
+  const unsigned O = S.O, V = S.V;
   if(tid < 24) {
     const int p = tid >> 2, i = tid & 3;
     sm.eps[tid] = i < sm.ext[p] ? (p < 3 ? S.eo : S.ev)[sm.start[p] + i] : 0.0;
   }
-  bool store = true;  // no bipartition has been added yet
-
+  d1code = uniform64(d1code);
+  d2code = uniform64(d2code);
+  s1code = uniform64(s1code);
+  auto code1 = [&](int g) { return (unsigned) (d1code >> (6 * g)) & 63u; };
+  auto code2 = [&](int g) { return (unsigned) (d2code >> (6 * g)) & 63u; };
+  auto next  = [&](int g) {  // first enabled bipartition from g on, or 9
+    while(g < 9 && !((code1(g) | code2(g)) & 1)) g++;
+    return g;
+  };
   const int row = tid >> 2, kq = tid & 3;
   double*   As  = sm.stage;
   double*   Bs  = sm.stage + 64 * LDK;
+  int       g   = next(0);
+  bool      store = true;  // no bipartition has been added yet
+  if(g < 9) fill_rows(sm.tab, 0, sm.ext, g, code1(g), code2(g), O, V);
+  __syncthreads();
 
+  // Chunk in flight: four k of this thread's M and N row (kq 0, 1: of the first
+  // unit, or of the only one; kq 2, 3: of the second), loaded while the chunk
+  // before is multiplied, also from one bipartition to the next.  Offsets from
+  // the sub-tile's first row stay below 2^32 bytes: they span three rows of the
+  // slowest coordinate of an array that fits the memory.
+  Runs     R;
+  GBytes   ba = nullptr, bb = nullptr;  // next chunk
+  int      left = 0, tb = 0;            // units of the family to load
+  bool     fam2 = false;
+  unsigned oa = 0, ob = 0, oa2 = 0, ob2 = 0;
+  const unsigned back = 64u * (kq >> 1);
+  v2d      ax0 = {0.0, 0.0}, ax1 = ax0, bx0 = ax0, bx1 = ax0;
+  typedef const __attribute__((address_space(1))) v2d* GD2;
+  auto load = [&]() {
+    asm("" : "+v"(oa), "+v"(ob));  // keeps scalar bases with vector offsets in the loop
+    const GD2 a = (GD2) (ba + oa), b = (GD2) (bb + ob);
+    ax0 = a[0];
+    ax1 = a[1];
+    bx0 = b[0];
+    bx1 = b[1];
+    ba += 8 * KC;
+    bb += 8 * KC;
+  };
+  auto fetch = [&]() {
+    if(left <= 0) {
+      if(!fam2 && R.n2) {
+        fam2 = true;
+        ba   = R.a2;
+        bb   = R.b2;
+        oa   = oa2;
+        ob   = ob2;
+        left = R.n2;
+      }
+      else {  // the bipartition's last chunk is on its way: read it again
+        ba -= 8 * KC;
+        bb -= 8 * KC;
+      }
+    }
+    if(left == 1) {
+      oa -= back;
+      ob -= back;
+    }
+    load();
+    left -= 2;
+  };
+  v2d* const A = reinterpret_cast<v2d*>(&As[row * LDK + 4 * kq]);
+  v2d* const B = reinterpret_cast<v2d*>(&Bs[row * LDK + 4 * kq]);
+  auto       put = [&]() {
+    A[0] = ax0;
+    A[1] = ax1;
+    B[0] = bx0;
+    B[1] = bx1;
+  };
+  auto begin = [&]() {
+    R = runs_of(S, sm.start, g, code1(g), code2(g));
+    const unsigned K1 = S.Op, K2 = S.Vp;
+    const Rows&    t = sm.tab;
+    oa   = 8 * (__umul24(t.r1[row], K1) + 4 * kq);
+    ob   = 8 * (__umul24(t.r1[64 + row], K1) + 4 * kq);
+    oa2  = 8 * (__umul24(t.r2[row], K2) + 4 * kq);
+    ob2  = 8 * (__umul24(t.r2[64 + row], K2) + 4 * kq);
+    ba   = R.a1;
+    bb   = R.b1;
+    left = R.n1;
+    fam2 = false;
+    fetch();
+  };
+  if(g < 9) begin();
 #pragma unroll 1
-  for(int g = 0; g < 9; g++) {
-    const unsigned c1 = (unsigned) (d1code >> (6 * g)) & 63u;
-    const unsigned c2 = (unsigned) (d2code >> (6 * g)) & 63u;
-    const int      n1 = (c1 & 1) ? cdiv(O, KC) : 0;
-    const int      n2 = (c2 & 1) ? cdiv(V, KC) : 0;
-    if(n1 + n2 == 0) continue;
-    const int hs = g / 3, ps = g % 3;
-    int       hA, hB, pA, pB;
+  while(g < 9) {
+    const int             gn = next(g + 1), hs = g / 3, ps = g % 3;
+    const unsigned short* te = sm.tab.e[tb];
+    int                   hA, hB, pA, pB;
     pair_of(hs, hA, hB);
     pair_of(ps, pA, pB);
-    const int eHS = sm.ext[hs], ePA = sm.ext[3 + pA], eHA = sm.ext[hA], eHB = sm.ext[hB];
-    const int rows = __builtin_amdgcn_readfirstlane(eHS * ePA * sm.ext[3 + pB]);
-    const int cols = __builtin_amdgcn_readfirstlane(eHA * eHB * sm.ext[3 + ps]);
-    const Quad quad = quadrant(g, rows, cols);
-    // this thread's M row (hs, pA, pB) and N row (hA, hB, ps)
-    const bool   mok = row < rows, nok = row < cols;
-    const Item   m = item_of(mok ? row : 0, eHS, ePA), n = item_of(nok ? row : 0, eHA, eHB);
-    const size_t HS = sm.start[hs] + m.a, PA = sm.start[3 + pA] + m.b, PB = sm.start[3 + pB] + m.c;
-    const size_t HA = sm.start[hA] + n.a, HB = sm.start[hB] + n.b, PS = sm.start[3 + ps] + n.c;
-    // operand rows c1*x - c2*y of the spin-orbital elements: both terms ->
-    // the antisymmetrised array; one term -> that array (sign folded into c)
-    auto pick = [](bool ok, unsigned code, unsigned bx, unsigned by, double sgn, const double* both,
-                   const double* x, const double* y) {
-      RowPtr r;
-      const bool hx = (code & bx) != 0, hy = (code & by) != 0;
-      r.p = hx && hy ? both : (hx ? x : y);
-      r.c = !ok || !(hx || hy) ? 0.0 : (hx ? sgn : -sgn);
-      return r;
+    const Share q = wave_share(g, __builtin_amdgcn_readfirstlane(sm.ext[hs] * sm.ext[3 + pA] * sm.ext[3 + pB]),
+                               __builtin_amdgcn_readfirstlane(sm.ext[hA] * sm.ext[hB] * sm.ext[3 + ps]));
+    auto left_units = [&]() { return left; };
+    auto skip         = [&](int n) { left -= n; };
+    auto refill_whole = [&]() {
+      put();
+      load();
     };
-    const size_t Op = S.Op, Vp = S.Vp;
-    RowPtr       a1r, b1r, a2r, b2r;
-    {
-      const double sg = (c1 & 2) ? -1.0 : 1.0;
-      const size_t xo = ((PA * V + PB) * O + HS) * Op, yo = ((PB * V + PA) * O + HS) * Op;
-      // t(pA,pB,hs,h7) - t(pA,pB,h7,hs) = t2h[pA,pB,hs,:] - t2h[pB,pA,hs,:]
-      a1r = pick(mok, c1, 4, 8, sg, S.t2ha + xo, S.t2h + xo, S.t2h + yo);
-      // (hA h7|hB ps) - (hB h7|hA ps) = ovk[hB,ps,hA,:] - ovk[hA,ps,hB,:]
-      const size_t bxo = ((HB * V + PS) * O + HA) * Op, byo = ((HA * V + PS) * O + HB) * Op;
-      b1r = pick(nok, c1, 16, 32, 1.0, S.ovka + bxo, S.ovk + bxo, S.ovk + byo);
-    }
-    {
-      const double sg = (c2 & 2) ? -1.0 : 1.0;
-      // (hs pA|p7 pB) - (hs pB|p7 pA) = xv[pB,pA,hs,:] - xv[pA,pB,hs,:]
-      const size_t xo = ((PB * V + PA) * O + HS) * Vp, yo = ((PA * V + PB) * O + HS) * Vp;
-      a2r = pick(mok, c2, 4, 8, sg, S.xva + xo, S.xv + xo, S.xv + yo);
-      // t(ps,p7,hA,hB) - t(p7,ps,hA,hB) = t2p[hA,hB,ps,:] - t2p[hB,hA,ps,:]
-      const size_t bxo = ((HA * O + HB) * V + PS) * Vp, byo = ((HB * O + HA) * V + PS) * Vp;
-      b2r = pick(nok, c2, 16, 32, 1.0, S.t2pa + bxo, S.t2p + bxo, S.t2p + byo);
-    }
-
-    v4d acc[2][2];
-#pragma unroll
-    for(int i = 0; i < 2; i++)
-#pragma unroll
-      for(int j = 0; j < 2; j++) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-
-    double    ax[4], bx[4];
-    const int nc    = n1 + n2;
-    auto      fetch = [&](int c) {
-      if(c < n1) {
-        fetch4(a1r, c * KC + 4 * kq, (int) Op, ax);
-        fetch4(b1r, c * KC + 4 * kq, (int) Op, bx);
-      }
-      else {
-        fetch4(a2r, (c - n1) * KC + 4 * kq, (int) Vp, ax);
-        fetch4(b2r, (c - n1) * KC + 4 * kq, (int) Vp, bx);
-      }
+    auto refill = [&]() {
+      put();
+      fetch();
     };
-    fetch(0);
-#pragma unroll 1
-    for(int c = 0; c < nc; c++) {
-      const double ca = c < n1 ? a1r.c : a2r.c, cb = c < n1 ? b1r.c : b2r.c;
-      __syncthreads();
-      if(c == 0) fill_tables(sm.tab, sm.ext, hs, hA, hB, ps, pA, pB);
-#pragma unroll
-      for(int j = 0; j < 4; j++) {
-        As[row * LDK + 4 * kq + j] = ca * ax[j];
-        Bs[row * LDK + 4 * kq + j] = cb * bx[j];
-      }
-      __syncthreads();
-      if(c + 1 < nc) fetch(c + 1);
-      mfma_chunk(As, Bs, quad, acc);
-    }
-    acc_to_t3(sm.t3, sm.tab, quad, store, acc);
+    auto ahead = [&]() {
+      tb ^= 1;
+      g = gn;
+      if(g < 9) begin();
+    };
+    __syncthreads();  // every wave has added the bipartition before: its tables are free
+    if(gn < 9) fill_rows(sm.tab, tb ^ 1, sm.ext, gn, code1(gn), code2(gn), O, V);
+    share_tiles(sm.t3, As, Bs, te, q, store, R.n1, R.n2, R.neg1, R.neg2, left_units, skip, refill_whole, refill, ahead);
     store = false;
   }
   if(store)
@@ -405,12 +671,8 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
 
   // ---- s1 operands: T1so(pa,hi) and <hk hj||pc pb> blocks of the sub-tile
   __syncthreads();
-  double*  T1s    = sm.t1s;
-  double*  V1s    = sm.stage;
-  unsigned s1mask = 0;
-#pragma unroll
-  for(int slot = 0; slot < 9; slot++)
-    if((s1code >> (4 * slot)) & 1) s1mask |= 1u << slot;
+  double* T1s = sm.t1s;
+  double* V1s = sm.stage;
   for(int x = tid; x < 9 * 16; x += NT) {
     const int      slot = x >> 4, pai = (x >> 2) & 3, hii = x & 3;
     const unsigned c    = (unsigned) (s1code >> (4 * slot)) & 15u;
@@ -422,26 +684,39 @@ __device__ void spatial_subtile(Smem& sm, const SpatialDev& S, uint64_t d1code, 
     }
     T1s[x] = v;
   }
-  for(int x = tid; x < 9 * 256; x += NT) {
-    const int      slot = x >> 8, w = x & 255;
-    const unsigned c    = (unsigned) (s1code >> (4 * slot)) & 15u;
-    const int      pa = slot / 3, hi = slot % 3;
-    int            hj, hk, pb, pc;
-    pair_of(hi, hj, hk);
-    pair_of(pa, pb, pc);
-    const int gk = w & 3, gj = (w >> 2) & 3, gc = (w >> 4) & 3, gb = w >> 6;
-    double    v  = 0.0;
-    if((c & 1) && gk < sm.ext[hk] && gj < sm.ext[hj] && gc < sm.ext[3 + pc] && gb < sm.ext[3 + pb]) {
-      const size_t K = sm.start[hk] + gk, J = sm.start[hj] + gj, PC = sm.start[3 + pc] + gc,
-                   PBx = sm.start[3 + pb] + gb;
-      const double x1 = (c & 4) ? S.vvoo[((PC * V + PBx) * O + K) * O + J] : 0.0;  // (hk pc|hj pb)
-      const double x2 = (c & 8) ? S.vvoo[((PBx * V + PC) * O + K) * O + J] : 0.0;  // (hk pb|hj pc)
-      v               = ((c & 4) && (c & 8)) ? x1 - x2 : ((c & 4) ? x1 : -x2);
+  {
+    // One element per slot and thread, every load in flight before the first
+    // use; offsets from the sub-tile's first element stay below 2^32 bytes, as
+    // the operand rows' do.
+    const unsigned gk = tid & 3, gj = (tid >> 2) & 3, gc = (tid >> 4) & 3, gb = tid >> 6;
+    const unsigned o1 = 8 * (__umul24(__umul24(__umul24(gc, V) + gb, O) + gk, O) + gj);
+    const unsigned o2 = 8 * (__umul24(__umul24(__umul24(gb, V) + gc, O) + gk, O) + gj);
+    double         x1[9], x2[9];
+    typedef const __attribute__((address_space(1))) double* GD;
+#pragma unroll
+    for(int slot = 0; slot < 9; slot++) {
+      const unsigned c  = (unsigned) (s1code >> (4 * slot)) & 15u;
+      const int      pa = slot / 3, hi = slot % 3;
+      int            hj, hk, pb, pc;
+      pair_of(hi, hj, hk);
+      pair_of(pa, pb, pc);
+      x1[slot] = x2[slot] = 0.0;
+      if((c & 1) && (int) gk < sm.ext[hk] && (int) gj < sm.ext[hj] && (int) gc < sm.ext[3 + pc] &&
+         (int) gb < sm.ext[3 + pb]) {
+        const uint64_t K = uni(sm.start[hk]), J = uni(sm.start[hj]), PC = uni(sm.start[3 + pc]),
+                       PB = uni(sm.start[3 + pb]);
+        if(c & 4) x1[slot] = *(GD) ((GBytes) (S.vvoo + ((PC * V + PB) * O + K) * O + J) + o1);  // (hk pc|hj pb)
+        if(c & 8) x2[slot] = *(GD) ((GBytes) (S.vvoo + ((PB * V + PC) * O + K) * O + J) + o2);  // (hk pb|hj pc)
+      }
     }
-    V1s[x] = v;
+#pragma unroll
+    for(int slot = 0; slot < 9; slot++) {
+      const unsigned c = (unsigned) (s1code >> (4 * slot)) & 15u;
+      V1s[slot * 256 + tid] = (c & 4) && (c & 8) ? x1[slot] - x2[slot] : ((c & 4) ? x1[slot] : -x2[slot]);
+    }
   }
   __syncthreads();
-  subtile_energy(sm, T1s, V1s, sm.ext, s1mask, e4, e5);
+  subtile_energy(sm, T1s, V1s, sm.ext, e4, e5);
 }
 
 // Persistent kernel: workgroup b serves queue b % kQueues first (dispatch is
@@ -768,29 +1043,24 @@ int launch_reduce(const TaskDev* tasks, int n_tasks, const unsigned long long* a
 // (ccsd_t_data_{s1,d1,d2}_new layouts, ccsd_t_all_fused_cpu.hpp index
 // arithmetic), one workgroup per 4^6 block, partials per block.
 // ---------------------------------------------------------------------------
-// LDS of the per-task kernel, sized for three workgroups per CU (12 waves):
-// the 4^6 tile, one staged K chunk of 16 (rows padded to 18 doubles, so the
-// 16x16x4 fragment reads of a half-wave hit distinct banks), which later holds
-// the s1 V blocks, and the K tile list of the current bipartition, which
-// later holds the s1 T1 blocks.
+// LDS of the per-task kernel, sized for three workgroups per CU (12 waves): the
+// 4^6 tile, one staged K chunk of 16 (rows padded to 18 doubles, so the 16x16x4
+// fragment reads of a half-wave hit distinct banks), which later holds the s1 V
+// blocks.  A chunk is of one K tile, so its addresses come from scalars and one
+// row pointer a thread (40.5 ms on six tasks of O=24, V=160; 41.9 with tiles
+// packed end to end into the chunks and a pointer per load).
 constexpr int PKC  = 16;
 constexpr int PLDK = PKC + 2;
-static_assert(PKC == kPackedKC, "the host aligns the per-task d2 tiles to the K chunk");
 static_assert(2 * 64 * PLDK >= 9 * 256, "staging too small for the s1 V blocks");
 struct __align__(16) PSmem {
   double t3[T3N];
   double stage[2 * 64 * PLDK];
-  union {
-    int2   klist[kMaxNoab + kMaxNvab + 1];  // (family | exec slot << 1, K - 1 | first k << 12)
-    double t1s[S1_T1];
-  } u;
+  double t1s[S1_T1];  // s1 T1 blocks
   double eps[24];
   double red[8];
   Tables tab;
   int    ext[6];  // orbitals of the block inside the tile
 };
-// a K tile list entry fits two ints: K <= 4096, total K < 2^20, exec slot < 2^30
-static_assert((kMaxNoab + kMaxNvab) * 4096 + kPackedKC < (1 << 20), "K offsets must fit 20 bits");
 
 __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
   __shared__ PSmem sm;
@@ -825,172 +1095,143 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
   __syncthreads();
   double* As = sm.stage;
   double* Bs = sm.stage + 64 * PLDK;
-  // decoded K tile list entry: (family, exec slot, K, first k); first k alone
-  auto kent = [&](int i) {
-    const int2 v = sm.u.klist[i];
-    return make_int4(v.x & 1, v.x >> 1, (v.y & 0xfff) + 1, (int) ((unsigned) v.y >> 12));
-  };
-  auto kbeg = [&](int i) { return (int) ((unsigned) sm.u.klist[i].y >> 12); };
+  const int kk = tid & 15, rs = tid >> 4, n1 = tid & 63;
+  const int kq = __builtin_amdgcn_readfirstlane(tid >> 6);
 
+  int first = 0;  // first list entry of the bipartition
 #pragma unroll 1
   for(int g = 0; g < 9; g++) {
+    const int   nk   = k_n[g];
+    const int4* list = k_list + first;
+    first += nk;
+    if(nk == 0) continue;
     const int hs = g / 3, ps = g % 3;
     int       hA, hB, pA, pB;
     pair_of(hs, hA, hB);
     pair_of(ps, pA, pB);
-    const double sg = -sgn_single(hs) * sgn_single(ps);
-    const long   DHS = dim[hs], DPA = dim[3 + pA], DPB = dim[3 + pB];
-    const long   DHA = dim[hA], DHB = dim[hB], DPS = dim[3 + ps];
-    v4d          acc[2][2];
+    const bool neg = sgn_single(hs) * sgn_single(ps) > 0;  // the equations' sign, put on A
+    const long DHS = dim[hs], DPA = dim[3 + pA], DPB = dim[3 + pB];
+    const long DHA = dim[hA], DHB = dim[hB], DPS = dim[3 + ps];
+    v4d        acc[2][2];
 #pragma unroll
     for(int i = 0; i < 2; i++)
 #pragma unroll
       for(int j = 0; j < 2; j++) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-    // K of this bipartition: the enabled d1 tiles (h7b), then the enabled d2
-    // tiles (p7b) from the next multiple of PKC, packed end to end and cut
-    // into chunks of PKC; each chunk reads one family.  The host lists the
-    // tiles (family, exec slot, K, first packed k) with a sentinel holding the
-    // total.  Every thread has read the previous bipartition's list before it
-    // is rewritten.
-    int koff = 0;
-    for(int gg = 0; gg < g; gg++) koff += (k_n[gg] & 0xffff) + 1;
-    const int nk = k_n[g] & 0xffff, nd1 = k_n[g] >> 16;
-    __syncthreads();
-    for(int x = tid; x <= nk; x += NT) {
-      const int4 e = k_list[koff + x];
-      sm.u.klist[x] = make_int2(e.x | (e.y << 1),
-                                (int) ((unsigned) (e.z > 0 ? e.z - 1 : 0) | ((unsigned) e.w << 12)));
-    }
-    __syncthreads();
-    const int kall = kbeg(nk), kd2 = kbeg(nd1);  // total K, first d2 k
-    // Loads run along k where the packed block keeps k contiguous (d1_t2,
-    // d2_v2, d2_t2: row * K + k): thread (kk, rs) = (tid % 16, tid / 16)
-    // reads k = kk of rows rs + 16 j, so a load instruction reads four runs of
-    // 16 doubles.  The d1 <ij||ka> block keeps k slowest (row + k * bstr1):
-    // there thread (n1, kq) = (tid % 64, tid / 64) reads row n1 at k = 4 kq + j,
-    // and an instruction reads 64 neighbouring rows.
     // A row of either operand is (item of the first two positions of its side,
     // third position): thread rs takes the item rs of up to 16 and j is the
     // third position, so row rs + per * j, per the items the tile holds.
-    const int eHS = sm.ext[hs], ePA = sm.ext[3 + pA], ePB = sm.ext[3 + pB];
-    const int eHA = sm.ext[hA], eHB = sm.ext[hB], ePS = sm.ext[3 + ps];
+    // Items and third positions outside the block read the nearest one inside.
+    const int eHS = sm.ext[hs], ePA = sm.ext[3 + pA], ePB = __builtin_amdgcn_readfirstlane(sm.ext[3 + pB]);
+    const int eHA = sm.ext[hA], eHB = sm.ext[hB], ePS = __builtin_amdgcn_readfirstlane(sm.ext[3 + ps]);
     const int aper = __builtin_amdgcn_readfirstlane(eHS * ePA), bper = __builtin_amdgcn_readfirstlane(eHA * eHB);
-    const Quad quad = quadrant(g, __builtin_amdgcn_readfirstlane(aper * ePB), __builtin_amdgcn_readfirstlane(bper * ePS));
-    const int kk = tid & 15, rs = tid >> 4;
-    const int ax = small_div(rs, eHS), bx = small_div(rs, eHA);
-    const int aHS = 4 * sub[hs] + rs - ax * eHS, aPA = 4 * sub[3 + pA] + ax, aPB = 4 * sub[3 + pB];
-    const int bHA = 4 * sub[hA] + rs - bx * eHA, bHB = 4 * sub[hB] + bx, bPS = 4 * sub[3 + ps];
-    // third positions inside the block
-    const unsigned amask = rs < aper ? (1u << ePB) - 1u : 0u, bmask = rs < bper ? (1u << ePS) - 1u : 0u;
+    const Quad quad = quadrant(g, aper * ePB, bper * ePS);
+    const bool aok = rs < aper, bok = rs < bper;
+    const int  ar = aok ? rs : 0, br = bok ? rs : 0;
+    const int  ax = small_div(ar, eHS), bx = small_div(br, eHA);
+    const int  aHS = 4 * sub[hs] + ar - ax * eHS, aPA = 4 * sub[3 + pA] + ax, aPB = 4 * sub[3 + pB];
+    const int  bHA = 4 * sub[hA] + br - bx * eHA, bHB = 4 * sub[hB] + bx, bPS = 4 * sub[3 + ps];
     const long a1 = aPA + (aPB + aHS * DPB) * DPA;  // d1_t2 row of j = 0: [hs][pB][pA]
     const long a2 = aHS + (aPB + aPA * DPB) * DHS;  // d2_v2 row: [pA][pB][hs]
     const long b2 = bPS + (bHA + bHB * DHA) * DPS;  // d2_t2 row: [hB][hA][ps]
-    const int  n1 = tid & 63, kq = tid >> 6;
-    const bool nok1 = n1 < bper * ePS;
-    const Item y    = item_of(nok1 ? n1 : 0, eHA, eHB);
+    const Item y   = item_of(n1 < bper * ePS ? n1 : 0, eHA, eHB);
     const int  gHA = 4 * sub[hA] + y.a, gHB = 4 * sub[hB] + y.b, gPS = 4 * sub[3 + ps] + y.c;
     const long rB1   = gHB + (gHA + gPS * DHA) * DHB;  // d1_v2 element of k = rB1 + k * bstr1
     const long bstr1 = DPS * DHA * DHB;
-    // tile walkers (k only grows): wa for the thread's k-contiguous k, wb for
-    // its d1 <ij||ka> k; te = tile of k, nb = first k of the next tile
-    int  tia = 0, tib = 0;
-    int4 tea = kent(0), teb = tea;
-    int  nba = kbeg(1), nbb = nba;
-    double   av[4], bv[4];
-    unsigned oka = 0, okb = 0;
-    // Issues every load of chunk c (rows outside the block and k outside a
-    // tile read the buffer's first element; oka / okb mark the valid ones), so
-    // the loads of a chunk are in flight together while the previous chunk is
-    // multiplied.
-    auto load = [&](int c) {
-      const bool d2 = c * PKC >= kd2;
-      const int  k  = c * PKC + kk;
-      bool       kok = k < kall;
-      if(kok)
-        while(k >= nba) {
-          tea = kent(++tia);
-          nba = kbeg(tia + 1);
-        }
-      const long kl = k - tea.w, K = tea.z, ex = tea.y;
-      kok           = kok && kl < K;
-      const double* pa[4];
-      const double* pb[4];
-      {
-        const double* p0 = d2 ? A.d2_v2 + A.max_d2_v2 * ex + a2 * K + kl
-                              : A.d1_t2 + A.max_d1_t2 * ex + a1 * K + kl;
-        const long    s  = d2 ? DHS * K : DPA * K;
-        oka              = kok ? amask : 0u;
-#pragma unroll
-        for(int j = 0; j < 4; j++) pa[j] = ((oka >> j) & 1) ? p0 + j * s : A.d1_t2;
-      }
+
+    // Walk over the chunks.  Current tile: it of nk, family d2, K; kt = first k
+    // of the chunk to load; pa, pb the thread's pointers there, sa, sb the
+    // strides of j.
+    int           it = 0, kt = 0, K = 0;
+    bool          d2 = false;
+    const double *pa = nullptr, *pb = nullptr;
+    long          sa = 0, sb = 0;
+    auto          tile = [&]() {
+      const int  fam = __builtin_amdgcn_readfirstlane(list[it].x);
+      const long ex  = __builtin_amdgcn_readfirstlane(list[it].y);
+      K  = __builtin_amdgcn_readfirstlane(list[it].z);
+      kt = 0;
+      d2 = fam != 0;
       if(d2) {
-        const double* p0 = A.d2_t2 + A.max_d2_t2 * ex + b2 * K + kl;
-        okb              = kok ? bmask : 0u;
-#pragma unroll
-        for(int j = 0; j < 4; j++) pb[j] = ((okb >> j) & 1) ? p0 + j * K : A.d1_v2;
+        pa = A.d2_v2 + A.max_d2_v2 * ex + a2 * K;
+        sa = DHS * K;
+        pb = A.d2_t2 + A.max_d2_t2 * ex + b2 * K;
+        sb = K;
       }
       else {
-        okb = 0;
-#pragma unroll
-        for(int j = 0; j < 4; j++) {
-          const int k1 = c * PKC + 4 * kq + j;
-          bool      ok = nok1 && k1 < kall;
-          if(ok)
-            while(k1 >= nbb) {
-              teb = kent(++tib);
-              nbb = kbeg(tib + 1);
-            }
-          const long kl1 = k1 - teb.w;
-          ok             = ok && kl1 < teb.z;
-          pb[j]          = ok ? A.d1_v2 + A.max_d1_v2 * (long) teb.y + rB1 + kl1 * bstr1 : A.d1_v2;
-          okb |= (ok ? 1u : 0u) << j;
-        }
-      }
-#pragma unroll
-      for(int j = 0; j < 4; j++) {
-        av[j] = *pa[j];
-        bv[j] = *pb[j];
+        pa = A.d1_t2 + A.max_d1_t2 * ex + a1 * K;
+        sa = DPA * K;
+        pb = A.d1_v2 + A.max_d1_v2 * ex + rB1;
+        sb = bstr1;
       }
     };
-    if(kall > 0) {
-      const int nc = cdiv(kall, PKC);
-      load(0);
+    double av[4], bv[4];
+    int    clen = 0;      // k of the loaded chunk
+    bool   cd2  = false;  // its family
+    // Issues every load of the next chunk, so that they are in flight together
+    // while the previous chunk is multiplied; k past the tile's end reads its
+    // last one.
+    auto load = [&]() {
+      if(kt == K) {
+        it++;
+        tile();
+      }
+      clen = min(PKC, K - kt);
+      cd2  = d2;
+      const double* qa = pa + kt + min(kk, clen - 1);
+#pragma unroll
+      for(int j = 0; j < 4; j++) av[j] = qa[min(j, ePB - 1) * sa];
+      if(d2) {
+        const double* qb = pb + kt + min(kk, clen - 1);
+#pragma unroll
+        for(int j = 0; j < 4; j++) bv[j] = qb[min(j, ePS - 1) * sb];
+      }
+      else {
+#pragma unroll
+        for(int j = 0; j < 4; j++) bv[j] = pb[(kt + min(4 * kq + j, clen - 1)) * sb];
+      }
+      kt += clen;
+    };
+    tile();
+    load();
+    bool more = true, lead = true;
 #pragma unroll 1
-      for(int c = 0; c < nc; c++) {
-        __syncthreads();
-        if(c == 0) fill_tables(sm.tab, sm.ext, hs, hA, hB, ps, pA, pB);
-        // the masks are applied here, so that a chunk's loads are waited for
-        // only after the previous chunk's MFMAs were issued
+    while(more) {
+      const int len = clen;
+      __syncthreads();
+      if(lead) fill_tables(sm.tab, sm.ext, hs, hA, hB, ps, pA, pB);
+      lead = false;
+      const bool kin = kk < len;
+      if(aok) {
 #pragma unroll
         for(int j = 0; j < 4; j++)
-          if((amask >> j) & 1) As[(rs + aper * j) * PLDK + kk] = ((oka >> j) & 1) ? sg * av[j] : 0.0;
-        if(c * PKC >= kd2) {
+          if(j < ePB) As[(rs + aper * j) * PLDK + kk] = kin ? (neg ? -av[j] : av[j]) : 0.0;
+      }
+      if(cd2) {
+        if(bok) {
 #pragma unroll
           for(int j = 0; j < 4; j++)
-            if((bmask >> j) & 1) Bs[(rs + bper * j) * PLDK + kk] = ((okb >> j) & 1) ? bv[j] : 0.0;
+            if(j < ePS) Bs[(rs + bper * j) * PLDK + kk] = kin ? bv[j] : 0.0;
         }
-        else {
-#pragma unroll
-          for(int j = 0; j < 4; j++) Bs[n1 * PLDK + 4 * kq + j] = ((okb >> j) & 1) ? bv[j] : 0.0;
-        }
-        __syncthreads();
-        if(c + 1 < nc) load(c + 1);
-        mfma_chunk<PKC, PLDK>(As, Bs, quad, acc);
       }
-      acc_to_t3(sm.t3, sm.tab, quad, store, acc);
-      store = false;
+      else {
+#pragma unroll
+        for(int j = 0; j < 4; j++) Bs[n1 * PLDK + 4 * kq + j] = 4 * kq + j < len ? bv[j] : 0.0;
+      }
+      __syncthreads();
+      more = kt < K || it + 1 < nk;
+      if(more) load();
+      mfma_chunk<PKC, PLDK>(As, Bs, quad, acc, len);
     }
+    acc_to_t3(sm.t3, sm.tab, quad, store, acc);
+    store = false;
   }
   if(store)
     for(int e = tid; e < T3N; e += NT) sm.t3[e] = 0.0;
 
   // s1 operands from the packed buffers: t1 [hi][pa], v2 [pb][pc][hj][hk]
   __syncthreads();  // every thread is done with the tile list and the staged chunk
-  double*  T1s    = sm.u.t1s;
-  double*  V1s    = sm.stage;
-  unsigned s1mask = 0;
-  for(int slot = 0; slot < 9; slot++)
-    if(s1_exec[slot] >= 0) s1mask |= 1u << slot;
+  double* T1s = sm.t1s;
+  double* V1s = sm.stage;
   for(int x = tid; x < 9 * 16; x += NT) {
     const int slot = x >> 4, pai = (x >> 2) & 3, hii = x & 3;
     const int pa = slot / 3, hi = slot % 3;
@@ -1001,23 +1242,29 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
           A.s1_t1[A.max_s1_t1 * (long) s1_exec[slot] + gp + (long) gh * dim[3 + pa]];
     T1s[x] = v;
   }
-  for(int x = tid; x < 9 * 256; x += NT) {
-    const int slot = x >> 8, w = x & 255;
-    const int pa = slot / 3, hi = slot % 3;
-    int       hj, hk, pb, pc;
-    pair_of(hi, hj, hk);
-    pair_of(pa, pb, pc);
-    const int gk = 4 * sub[hk] + (w & 3), gj = 4 * sub[hj] + ((w >> 2) & 3),
-              gc = 4 * sub[3 + pc] + ((w >> 4) & 3), gb = 4 * sub[3 + pb] + (w >> 6);
-    double v = 0.0;
-    if(s1_exec[slot] >= 0 && gk < dim[hk] && gj < dim[hj] && gc < dim[3 + pc] && gb < dim[3 + pb])
-      v = A.s1_v2[A.max_s1_v2 * (long) s1_exec[slot] + gk +
-                  (gj + (gc + (long) gb * dim[3 + pc]) * dim[hj]) * dim[hk]];
-    V1s[x] = v;
+  {
+    // one element per slot and thread, every load in flight before the first use
+    const int w = tid;
+    double    v[9];
+#pragma unroll
+    for(int slot = 0; slot < 9; slot++) {
+      const int pa = slot / 3, hi = slot % 3;
+      int       hj, hk, pb, pc;
+      pair_of(hi, hj, hk);
+      pair_of(pa, pb, pc);
+      const int gk = 4 * sub[hk] + (w & 3), gj = 4 * sub[hj] + ((w >> 2) & 3),
+                gc = 4 * sub[3 + pc] + ((w >> 4) & 3), gb = 4 * sub[3 + pb] + (w >> 6);
+      v[slot] = 0.0;
+      if(s1_exec[slot] >= 0 && gk < dim[hk] && gj < dim[hj] && gc < dim[3 + pc] && gb < dim[3 + pb])
+        v[slot] = A.s1_v2[A.max_s1_v2 * (long) s1_exec[slot] + gk +
+                          (gj + (gc + (long) gb * dim[3 + pc]) * dim[hj]) * dim[hk]];
+    }
+#pragma unroll
+    for(int slot = 0; slot < 9; slot++) V1s[slot * 256 + tid] = v[slot];
   }
   __syncthreads();
   double e4, e5;
-  subtile_energy(sm, T1s, V1s, sm.ext, s1mask, e4, e5);
+  subtile_energy(sm, T1s, V1s, sm.ext, e4, e5);
   if(tid == 0) {
     A.partial[blockIdx.x]                = e4;
     A.partial[blockIdx.x + A.num_blocks] = e5;
