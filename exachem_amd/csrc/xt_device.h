@@ -141,8 +141,10 @@ int cholesky_integrals(int O, int V, long K, const double* L, double* vvoo, doub
 int build_xva(int O, int V, SpatialBufs& B, void* stream);
 // Reorders the (ai|bj) GEMM result [(a,i)][(b,j)] into vvoo[a][b][i][j].
 int launch_vvoo_order(const double* in, double* out, int O, int V, void* stream);
-// out[0], out[1] = largest |(ai|bj) - (bj|ai)| and largest |(ai|bj)| of a vvoo array, as doubles.
-int launch_vvoo_asym(const double* vvoo, int O, int V, unsigned long long* out, void* stream);
+// Largest |(ai|bj) - (bj|ai)| and largest |(ai|bj)| of a vvoo array, a pair for each of *groups
+// workgroups (at most kAsymGroups), to out in host memory.
+constexpr int kAsymGroups = 2048;
+int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups, void* stream);
 // With vvvo == nullptr the xv/xva pair is left to the caller.
 int build_operands(int O, int V, double* t2, double* ovoo, double*& vvvo, SpatialBufs& B,
                    void* stream);

@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 #include <initializer_list>
 #include <mutex>
 #include <numeric>
@@ -308,9 +309,9 @@ struct xt_ctx {
   // tickets it takes, the host reads them while the persistent kernel runs
   unsigned long long* h_prog = nullptr;
   unsigned long long* d_prog = nullptr;
-  // largest asymmetry and element of the uploaded vvoo (queue_fold_check)
-  unsigned long long* d_asym = nullptr;
-  double*             h_asym = nullptr;
+  // behind it: largest asymmetry and element of the uploaded vvoo, a pair for
+  // each of n_asym workgroups (queue_fold_check)
+  int n_asym = 0;
   int         n_cu   = 0;
   Plan        plan;
   bool        have_plan = false, have_inputs = false;
@@ -441,11 +442,9 @@ int xt_create(int device, xt_ctx** out) {
   XT_HIP(hipGetDeviceProperties(&prop, device));
   c->n_cu = prop.multiProcessorCount;
   XT_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  XT_HIP(hipHostMalloc((void**) &c->h_prog, sizeof(unsigned long long) * xt::kQueues,
+  XT_HIP(hipHostMalloc((void**) &c->h_prog, sizeof(unsigned long long) * (xt::kQueues + 2 * xt::kAsymGroups),
                        hipHostMallocMapped | hipHostMallocCoherent));
   XT_HIP(hipHostGetDevicePointer((void**) &c->d_prog, c->h_prog, 0));
-  XT_HIP(hipHostMalloc((void**) &c->h_asym, 2 * sizeof(double), hipHostMallocDefault));
-  XT_HIP(hipMalloc((void**) &c->d_asym, 2 * sizeof(unsigned long long)));
   XT_HIP(hipEventCreate(&c->ev0));
   XT_HIP(hipEventCreate(&c->ev1));
   *out = c;
@@ -466,8 +465,6 @@ int xt_destroy(xt_ctx* c) {
   if(c->ev1) (void) hipEventDestroy(c->ev1);
   if(c->stream) (void) hipStreamDestroy(c->stream);
   if(c->h_prog) (void) hipHostFree(c->h_prog);
-  if(c->h_asym) (void) hipHostFree(c->h_asym);
-  if(c->d_asym) (void) hipFree(c->d_asym);
   if(c->d_gather) (void) hipFree(c->d_gather);
   delete c;
   return XT_OK;
@@ -692,15 +689,21 @@ extern "C" {
 // asks for.  Integrals that miss it by more than their own rounding (1e-13 of
 // the largest; products over Cholesky vectors miss it by a few 1e-16) are run
 // over every box.
-// Queued once vvoo is on the device; fold_allowed reads the two maxima after
-// the upload's own wait for the stream.
+// Queued once vvoo is on the device; fold_allowed reads the maxima after the
+// upload's own wait for the stream.
 static int queue_fold_check(xt_ctx* c) {
-  int err = xt::launch_vvoo_asym(c->in.vvoo, c->plan.O, c->plan.V, c->d_asym, c->stream);
-  if(!err)
-    err = (int) hipMemcpyAsync(c->h_asym, c->d_asym, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-  return err;
+  return xt::launch_vvoo_asym(c->in.vvoo, c->plan.O, c->plan.V, reinterpret_cast<double*>(c->d_prog + xt::kQueues),
+                              &c->n_asym, c->stream);
 }
-static bool fold_allowed(const xt_ctx* c) { return c->h_asym[0] <= 1e-13 * c->h_asym[1]; }
+static bool fold_allowed(const xt_ctx* c) {
+  const double* p = reinterpret_cast<const double*>(c->h_prog + xt::kQueues);
+  double        d = 0.0, m = 0.0;
+  for(int w = 0; w < c->n_asym; w++) {
+    d = std::max(d, p[2 * w]);
+    m = std::max(m, p[2 * w + 1]);
+  }
+  return d <= 1e-13 * m && d < std::numeric_limits<double>::infinity();
+}
 
 static int upload_common(xt_ctx* c, const double* eo, const double* ev, const double* t1,
                          const double* t2, const double* vvoo, const double* ovoo,

@@ -973,21 +973,24 @@ int launch_vvoo_order(const double* in, double* out, int O, int V, void* stream)
   return (int) hipGetLastError();
 }
 
-// Largest |(ai|bj) - (bj|ai)| and largest |(ai|bj)| of vvoo, as the bits of
-// non-negative doubles (ordered like the values): out[0], out[1].
+// Largest |(ai|bj) - (bj|ai)| and largest |(ai|bj)| over the pairs a <= b of each
+// workgroup, to out[2 w] and out[2 w + 1] in host memory; an element that
+// cannot be compared (NaN, or two infinities) counts as an infinite difference.
+// A wave takes one pair at a time.  Bound: one read of vvoo (O=40, V=300: 0.26 ms).
 __global__ void __launch_bounds__(256) k_vvoo_asym(const double* __restrict__ vvoo, long O, long V,
-                                                   unsigned long long* out) {
-  const unsigned o = (unsigned) O, oo = o * o;
+                                                   double* out) {
+  const unsigned o = (unsigned) O, oo = o * o, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double         d = 0.0, m = 0.0;
-  for(long p = blockIdx.x; p < V * V; p += gridDim.x) {  // one (a, b) pair at a time
-    const long    a = p / V, b = p - a * V;
+  for(long p = 4l * blockIdx.x + wave; p < V * V; p += 4l * gridDim.x) {
+    const long a = p / V, b = p - a * V;
+    if(a > b) continue;
     const double* x = vvoo + p * oo;
     const double* y = vvoo + (b * V + a) * oo;
-    for(unsigned q = threadIdx.x; q < oo; q += blockDim.x) {
+    for(unsigned q = lane; q < oo; q += 64) {
       const unsigned i = q / o, j = q - i * o;
-      const double   u = x[q];
-      m                = fmax(m, fabs(u));
-      if(a <= b) d = fmax(d, fabs(u - y[j * o + i]));
+      const double   u = x[q], v = y[j * o + i], e = fabs(u - v);
+      m                = fmax(m, fmax(fabs(u), fabs(v)));
+      if(!(e <= d)) d = e == e ? e : __builtin_inf();
     }
   }
   __shared__ double rd[4], rm[4];
@@ -996,24 +999,20 @@ __global__ void __launch_bounds__(256) k_vvoo_asym(const double* __restrict__ vv
     d = fmax(d, __shfl_xor(d, k, 64));
     m = fmax(m, __shfl_xor(m, k, 64));
   }
-  if((threadIdx.x & 63) == 0) {
-    rd[threadIdx.x >> 6] = d;
-    rm[threadIdx.x >> 6] = m;
+  if(lane == 0) {
+    rd[wave] = d;
+    rm[wave] = m;
   }
   __syncthreads();
-  if(threadIdx.x == 0) {  // one pair of atomics per workgroup: they all meet at two addresses
-    d = fmax(fmax(rd[0], rd[1]), fmax(rd[2], rd[3]));
-    m = fmax(fmax(rm[0], rm[1]), fmax(rm[2], rm[3]));
-    atomicMax(&out[0], (unsigned long long) __double_as_longlong(d));
-    atomicMax(&out[1], (unsigned long long) __double_as_longlong(m));
+  if(threadIdx.x == 0) {
+    out[2 * blockIdx.x]     = fmax(fmax(rd[0], rd[1]), fmax(rd[2], rd[3]));
+    out[2 * blockIdx.x + 1] = fmax(fmax(rm[0], rm[1]), fmax(rm[2], rm[3]));
   }
 }
-
-int launch_vvoo_asym(const double* vvoo, int O, int V, unsigned long long* out, void* stream) {
-  const int rc = launch_zero_u64(out, 2, stream);
-  if(rc) return rc;
-  hipLaunchKernelGGL(k_vvoo_asym, dim3((unsigned) std::min<long>((long) V * V, 1024)), dim3(256), 0,
-                     (hipStream_t) stream, vvoo, (long) O, (long) V, out);
+int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups, void* stream) {
+  *groups = (int) std::min<long>(((long) V * V + 3) / 4, kAsymGroups);
+  hipLaunchKernelGGL(k_vvoo_asym, dim3((unsigned) *groups), dim3(256), 0, (hipStream_t) stream, vvoo,
+                     (long) O, (long) V, out);
   return (int) hipGetLastError();
 }
 
