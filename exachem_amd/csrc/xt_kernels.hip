@@ -26,6 +26,7 @@
 #include <mutex>
 
 #include "xt_device.h"
+#include "xt_claim.h"
 #include "xt_fixed.h"
 #include "xt_queue.h"
 #include "xt_tasksums.h"
@@ -728,7 +729,7 @@ __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) 
   __shared__ Smem               sm;
   __shared__ int                s_task;
   __shared__ int                s_weight;  // thread 0: boxes that its box stands for
-  __shared__ int                s_entry;   // thread 0: entry of its last ticket on the current queue
+  __shared__ Claim              s_claim;   // thread 0; its task also for the others
   __shared__ int                s_cur;     // thread 0: task of the running sums
   __shared__ unsigned long long s_sum[4];  // thread 0: E4 lo, hi, E5 lo, hi of s_cur not yet added
   const int                     tid  = threadIdx.x;
@@ -740,40 +741,28 @@ __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) 
 #pragma unroll 1
   for(int qi = 0; qi < kQueues; qi++) {
     const int q = (home + qi) % kQueues;
-    if(tid == 0) s_entry = R.qbeg[q];
+    if(tid == 0) claim_queue(s_claim, R, q);
 #pragma unroll 1
     for(;;) {
       __syncthreads();  // previous sub-tile finished with LDS and s_task
       if(tid == 0) {
-        int ti = -1;  // -1: queue exhausted
-        for(;;) {
-          const unsigned long long t = atomicAdd(&R.qctr[q], 1ull);
-          // progress mirror in host memory (tickets taken so far, approximate)
-          if(R.prog) __hip_atomic_store(&R.prog[q], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-          if((long long) t >= R.qtotal[q]) break;
-          const int e = queue_entry_from(R.qbeg, R.qtick, q, (long long) t, s_entry);
-          s_entry     = e;
-          ti          = R.qtask[e];
-          const TaskDev& T = R.tasks[ti];
-          int            sub[6];
-          const bool     in = ticket_box((long long) t - R.qtick[e], T.nsub, R.glog, sub);
-          // a copy of another box under the exchange of equal tiles is passed over
-          s_weight = !in ? 0 : R.fold ? fold_weight(T.eq, sub) : 1;
-          ti       = s_weight ? ti : -1;
-          if(ti < 0) continue;
+        int       sub[6], weight;
+        const int ti = claim_box(s_claim, R, q, claim_ticket(R, q), false, sub, weight);
+        if(ti >= 0) {
+          s_weight         = weight;
+          const TaskDev& T = s_claim.task;
 #pragma unroll
           for(int p = 0; p < 6; p++) {
             sm.start[p] = T.off[p] + 4 * sub[p];
             sm.ext[p]   = min(4, T.dim[p] - 4 * sub[p]);
           }
-          break;
         }
         s_task = ti;
       }
       __syncthreads();
       const int ti = s_task;
       if(ti < 0) break;
-      const TaskDev&           T  = R.tasks[ti];
+      const TaskDev&           T  = s_claim.task;
       const unsigned long long t0 = wall_clock64();
       double                   e4, e5;
       spatial_subtile(sm, S, T.d1code, T.d2code, T.s1code, e4, e5);

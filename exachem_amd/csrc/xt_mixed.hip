@@ -51,6 +51,7 @@
 #include <hip/hip_runtime.h>
 
 #include "xt_device.h"
+#include "xt_claim.h"
 #include "xt_fixed.h"
 #include "xt_queue.h"
 #include "xt_tasksums.h"
@@ -840,7 +841,7 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
   __shared__ int                s_task;
   __shared__ int                s_retable; // thread 0: the box's extents differ from the last one's
   __shared__ int                s_weight;  // thread 0: boxes that its box stands for
-  __shared__ int                s_entry;   // thread 0: entry of its last ticket on the current queue
+  __shared__ Claim              s_claim;   // thread 0; its task also for the others
   __shared__ int                s_cur;     // thread 0: task of the running sums
   __shared__ unsigned long long s_sum[4];  // thread 0: E4 lo, hi, E5 lo, hi of s_cur not yet added
   const int                     tid  = threadIdx.x;
@@ -854,28 +855,17 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
 #pragma unroll 1
   for(int qi = 0; qi < kQueues; qi++) {
     const int q = (home + qi) % kQueues;
-    if(tid == 0) s_entry = R.qbeg[q];
+    if(tid == 0) claim_queue(s_claim, R, q);
 #pragma unroll 1
     for(;;) {
       __syncthreads();
       if(tid == 0) {
-        int ti    = -1;  // -1: queue exhausted
-        s_retable = 0;
-        for(;;) {
-          const unsigned long long t = atomicAdd(&R.qctr[q], 1ull);
-          // progress mirror in host memory (tickets taken so far, approximate)
-          if(R.prog) __hip_atomic_store(&R.prog[q], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-          if((long long) t >= R.qtotal[q]) break;
-          const int e = queue_entry_from(R.qbeg, R.qtick, q, (long long) t, s_entry);
-          s_entry     = e;
-          ti          = R.qtask[e];
-          const TaskDev& T = R.tasks[ti];
-          int            sub[6];
-          const bool     in = ticket_box((long long) t - R.qtick[e], T.nsubm, R.glog, sub);
-          // a copy of another box under the exchange of equal tiles is passed over
-          s_weight = !in ? 0 : R.fold ? fold_weight(T.eq, sub) : 1;
-          ti       = s_weight ? ti : -1;
-          if(ti < 0) continue;
+        int       sub[6], weight;
+        const int ti = claim_box(s_claim, R, q, claim_ticket(R, q), true, sub, weight);
+        s_retable    = 0;
+        if(ti >= 0) {
+          s_weight         = weight;
+          const TaskDev& T = s_claim.task;
 #pragma unroll
           for(int p = 0; p < 6; p++) {
             const int x = min(ext(p), T.dim[p] - ext(p) * sub[p]);
@@ -883,7 +873,6 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
             sm.start[p] = T.off[p] + ext(p) * sub[p];
             sm.ext[p]   = x;
           }
-          break;
         }
         s_task = ti;
       }
@@ -893,7 +882,7 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
       if(tid >= 64 && tid < 64 + 18) sm.scale[tid - 64] = M.pscale[18 * (size_t) ti + tid - 64];
       if(s_retable) box_tables(sm);
       if(tid >= 128 && tid < 128 + 18) {
-        const TaskDev& T = R.tasks[ti];
+        const TaskDev& T = s_claim.task;
         part_entry(sm, M, tid - 128, part_code(T.d1code, T.d2code, tid - 128));
       }
       if(tid < 36) {
@@ -902,7 +891,7 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
         sm.eps[tid] = i < sm.ext[p] ? (p < 3 ? M.eo : M.ev)[sm.start[p] + i] : 0.0;
       }
       __syncthreads();
-      const TaskDev&           T  = R.tasks[ti];
+      const TaskDev&           T  = s_claim.task;
       const unsigned long long t0 = wall_clock64();
       box_contract(sm, M, T.d1code, T.d2code);
       __syncthreads();
