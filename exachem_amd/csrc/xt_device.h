@@ -98,7 +98,7 @@ struct MixedDev {
 // (fold_weight in xt_queue.h) are passed over by the thread that claims them.
 constexpr int kQueues = 8;
 // Threads of the one workgroup that sums the task energies in a fixed order
-// (k_reduce_final); xt_sum_task_energies repeats the same order on the host.
+// (k_reduce); xt_sum_task_energies repeats the same order on the host.
 constexpr int kReduceThreads = 256;
 constexpr int kGroupLog2 = 6;  // 64 boxes per whole ticket group
 
@@ -149,9 +149,14 @@ int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups,
 int build_operands(int O, int V, double* t2, double* ovoo, double*& vvvo, SpatialBufs& B,
                    void* stream);
 int launch_spatial_fp64(const SpatialDev& S, const RunDev& R, int grid, void* stream);
+// Into host memory: the task energies (task_h) and E4, E5 and 1 where *err is
+// set, else 0 (e45); task_e is device memory.
 int launch_reduce(const TaskDev* tasks, int n_tasks, const unsigned long long* acc,
-                  double* task_e, double* e45, void* stream);
-int launch_zero_u64(unsigned long long* p, long n, void* stream);
+                  const unsigned long long* err, double* task_e, double* task_h, double* e45,
+                  void* stream);
+// Clears zero[0, nz) and copies dst[0, n) = src[0, n) (src in host memory).
+int launch_begin(unsigned long long* zero, long nz, unsigned long long* dst,
+                 const unsigned long long* src, long n, void* stream);
 // tile_o[O] / tile_v[V]: spatial tile index of every orbital (host arrays).
 int build_split(const SpatialBufs& B, int O, int V, const int* tile_o, int nto, const int* tile_v,
                 int ntv, SplitBufs& S, void* stream);

@@ -329,7 +329,14 @@ struct xt_ctx {
   unsigned long long* d_qctr   = nullptr;
   unsigned long long* d_acc    = nullptr;
   unsigned long long* d_cost   = nullptr;
-  double *            d_task_e = nullptr, *d_e45 = nullptr;
+  double *            d_task_e = nullptr, *d_e45 = nullptr, *h_e45 = nullptr;
+  // Allocations the pointers above point into: queues (d_qtotal, d_qbeg, d_qtask,
+  // d_qtick) and, cleared in one go, counters and sums (d_qctr, d_acc, d_cost).
+  // A run's first kernel brings the queues from h_run and its last one leaves the
+  // task energies behind them (host memory, grown to the largest plan, freed with
+  // the context); d_e45 is h_e45's device address.
+  char * d_queues = nullptr, *d_sums = nullptr, *h_run = nullptr, *d_run = nullptr;
+  size_t h_run_cap = 0;
   long                dev_tasks_n = -1;
   // device-side gather: block descriptors of the last call (device copy and
   // the host list it was uploaded from, kept alive until the next call)
@@ -393,9 +400,10 @@ struct xt_ctx {
   }
   void free_plan_dev() {
     drop_graph();
-    void* ps[] = {d_tasks, d_qtask, d_qbeg, d_qtick, d_qtotal, d_qctr, d_acc, d_cost, d_task_e, d_e45};
+    void* ps[] = {d_tasks, d_queues, d_sums, d_task_e};
     for(void* p: ps)
       if(p) (void) hipFree(p);
+    d_queues = d_sums = nullptr;
     d_tasks  = nullptr;
     d_qtask  = nullptr;
     d_qbeg   = nullptr;
@@ -404,7 +412,7 @@ struct xt_ctx {
     d_qctr   = nullptr;
     d_acc    = nullptr;
     d_cost   = nullptr;
-    d_task_e = d_e45 = nullptr;
+    d_task_e = nullptr;
     dev_tasks_n      = -1;
   }
 };
@@ -442,9 +450,11 @@ int xt_create(int device, xt_ctx** out) {
   XT_HIP(hipGetDeviceProperties(&prop, device));
   c->n_cu = prop.multiProcessorCount;
   XT_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  XT_HIP(hipHostMalloc((void**) &c->h_prog, sizeof(unsigned long long) * (xt::kQueues + 2 * xt::kAsymGroups),
+  XT_HIP(hipHostMalloc((void**) &c->h_prog, sizeof(unsigned long long) * (xt::kQueues + 2 * xt::kAsymGroups + 4),
                        hipHostMallocMapped | hipHostMallocCoherent));
   XT_HIP(hipHostGetDevicePointer((void**) &c->d_prog, c->h_prog, 0));
+  c->h_e45 = reinterpret_cast<double*>(c->h_prog + xt::kQueues + 2 * xt::kAsymGroups);
+  c->d_e45 = reinterpret_cast<double*>(c->d_prog + xt::kQueues + 2 * xt::kAsymGroups);
   XT_HIP(hipEventCreate(&c->ev0));
   XT_HIP(hipEventCreate(&c->ev1));
   *out = c;
@@ -465,6 +475,7 @@ int xt_destroy(xt_ctx* c) {
   if(c->ev1) (void) hipEventDestroy(c->ev1);
   if(c->stream) (void) hipStreamDestroy(c->stream);
   if(c->h_prog) (void) hipHostFree(c->h_prog);
+  if(c->h_run) (void) hipHostFree(c->h_run);
   if(c->d_gather) (void) hipFree(c->d_gather);
   delete c;
   return XT_OK;
@@ -899,22 +910,51 @@ static xt::MixedDev mixed_dev(const xt_ctx* c) {
   return M;
 }
 
+// The ticket counters and, after them, the run's error flag, padded to a line.
+constexpr int kCounters = 16;
+static_assert(kCounters > xt::kQueues, "the counters and the flag");
+// Byte offsets in the queue buffer for nt tasks: d_qtotal, d_qbeg, d_qtask,
+// d_qtick; all are multiples of 8.
+struct QueueBytes {
+  size_t beg, task, tick, end;
+  explicit QueueBytes(long nt) {
+    beg  = sizeof(long long) * xt::kQueues;
+    task = beg + (sizeof(int) * (xt::kQueues + 1) + 7) / 8 * 8;
+    tick = task + (sizeof(int) * (size_t) nt + 7) / 8 * 8;
+    end  = tick + sizeof(long long) * (size_t) nt;
+  }
+};
+
+static const double* host_task_e(const xt_ctx* c) {
+  return (const double*) (c->h_run + QueueBytes(std::max<long>((long) c->plan.dev.size(), 1)).end);
+}
+
 static int ensure_plan_dev(xt_ctx* c) {
   const Plan& P  = c->plan;
   const long  nt = std::max<long>((long) P.dev.size(), 1);
   if(c->dev_tasks_n == (long) P.dev.size()) return XT_OK;
   c->free_plan_dev();
   XT_HIP(hipMalloc((void**) &c->d_tasks, sizeof(xt::TaskDev) * nt));
-  XT_HIP(hipMalloc((void**) &c->d_qtask, sizeof(int) * nt));
-  XT_HIP(hipMalloc((void**) &c->d_qtick, sizeof(long long) * nt));
-  XT_HIP(hipMalloc((void**) &c->d_qbeg, sizeof(int) * (xt::kQueues + 1)));
-  XT_HIP(hipMalloc((void**) &c->d_qtotal, sizeof(long long) * xt::kQueues));
-  // the ticket counters and, after them, the run's error flag
-  XT_HIP(hipMalloc((void**) &c->d_qctr, sizeof(unsigned long long) * (xt::kQueues + 1)));
-  XT_HIP(hipMalloc((void**) &c->d_acc, sizeof(unsigned long long) * 4 * nt));
-  XT_HIP(hipMalloc((void**) &c->d_cost, sizeof(unsigned long long) * nt));
+  const QueueBytes qb(nt);
+  const size_t run_bytes = qb.end + 2 * sizeof(double) * nt;
+  if(run_bytes > c->h_run_cap) {
+    if(c->h_run) (void) hipHostFree(c->h_run);
+    c->h_run     = nullptr;
+    c->h_run_cap = 0;
+    XT_HIP(hipHostMalloc((void**) &c->h_run, run_bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    XT_HIP(hipHostGetDevicePointer((void**) &c->d_run, c->h_run, 0));
+    c->h_run_cap = run_bytes;
+  }
+  XT_HIP(hipMalloc((void**) &c->d_queues, qb.end));
+  c->d_qtotal = (long long*) c->d_queues;
+  c->d_qbeg   = (int*) (c->d_queues + qb.beg);
+  c->d_qtask  = (int*) (c->d_queues + qb.task);
+  c->d_qtick  = (long long*) (c->d_queues + qb.tick);
+  XT_HIP(hipMalloc((void**) &c->d_sums, 8 * (kCounters + 5 * (size_t) nt)));
+  c->d_qctr = (unsigned long long*) c->d_sums;
+  c->d_acc  = c->d_qctr + kCounters;
+  c->d_cost = c->d_acc + 4 * nt;
   XT_HIP(hipMalloc((void**) &c->d_task_e, sizeof(double) * 2 * nt));
-  XT_HIP(hipMalloc((void**) &c->d_e45, sizeof(double) * 2));
   if(!P.dev.empty())
     XT_HIP(hipMemcpy(c->d_tasks, P.dev.data(), sizeof(xt::TaskDev) * P.dev.size(),
                      hipMemcpyHostToDevice));
@@ -1035,16 +1075,11 @@ static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
       return fail(XT_EINVAL, "run: a task of 2^31 or more box tickets");
   Queues      Q     = build_queues(P, sel, o.schedule, learned, mixed, glog);
   hipStream_t st = c->stream;
-  if(!Q.task.empty()) {
-    XT_HIP(hipMemcpyAsync(c->d_qtask, Q.task.data(), sizeof(int) * Q.task.size(),
-                          hipMemcpyHostToDevice, st));
-    XT_HIP(hipMemcpyAsync(c->d_qtick, Q.tick.data(), sizeof(long long) * Q.tick.size(),
-                          hipMemcpyHostToDevice, st));
-  }
-  XT_HIP(hipMemcpyAsync(c->d_qbeg, Q.beg.data(), sizeof(int) * Q.beg.size(), hipMemcpyHostToDevice,
-                        st));
-  XT_HIP(hipMemcpyAsync(c->d_qtotal, Q.total.data(), sizeof(long long) * Q.total.size(),
-                        hipMemcpyHostToDevice, st));
+  const QueueBytes qb(std::max<long>(nt, 1));
+  std::memcpy(c->h_run, Q.total.data(), sizeof(long long) * Q.total.size());
+  std::memcpy(c->h_run + qb.beg, Q.beg.data(), sizeof(int) * Q.beg.size());
+  std::memcpy(c->h_run + qb.task, Q.task.data(), sizeof(int) * Q.task.size());
+  std::memcpy(c->h_run + qb.tick, Q.tick.data(), sizeof(long long) * Q.tick.size());
   xt::SpatialDev S;
   S.O    = P.O;
   S.V    = P.V;
@@ -1091,18 +1126,18 @@ static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
     grid = o.workgroups > 0 ? o.workgroups : c->n_cu;
     grid = (int) std::max<long long>(1, std::min<long long>(grid, tickets));
   }
-  // the launch sequence; counters and accumulators are cleared by fill
-  // kernels (no memset nodes when captured)
+  // the launch sequence; counters and accumulators are cleared by a kernel (no
+  // memset nodes when captured), which also brings the queues
   auto body = [&](bool events) -> int {
-    int err = xt::launch_zero_u64(c->d_qctr, xt::kQueues + 1, st);
-    if(!err) err = xt::launch_zero_u64(c->d_acc, 4 * std::max<long>(nt, 1), st);
-    if(!err) err = xt::launch_zero_u64(c->d_cost, std::max<long>(nt, 1), st);
-    if(err) return fail(XT_EHIP, std::string("zero: ") + hipGetErrorString((hipError_t) err));
+    int err = xt::launch_begin((unsigned long long*) c->d_sums, kCounters + 5 * std::max<long>(nt, 1),
+                               (unsigned long long*) c->d_queues, (unsigned long long*) c->d_run, (long) (qb.end / 8), st);
+    if(err) return fail(XT_EHIP, std::string("begin: ") + hipGetErrorString((hipError_t) err));
     if(events) XT_HIP(hipEventRecord(c->ev0, st));
     err = mixed ? xt::launch_spatial_mixed(M, R, grid, st) : xt::launch_spatial_fp64(S, R, grid, st);
     if(err) return fail(XT_EHIP, std::string("launch: ") + hipGetErrorString((hipError_t) err));
     if(events) XT_HIP(hipEventRecord(c->ev1, st));
-    err = xt::launch_reduce(c->d_tasks, (int) nt, c->d_acc, c->d_task_e, c->d_e45, st);
+    err = xt::launch_reduce(c->d_tasks, (int) nt, c->d_acc, R.err, c->d_task_e, (double*) (c->d_run + qb.end),
+                            c->d_e45, st);
     if(err) return fail(XT_EHIP, std::string("reduce: ") + hipGetErrorString((hipError_t) err));
     return XT_OK;
   };
@@ -1154,13 +1189,16 @@ static int task_times(xt_ctx* c, long nt, float* task_ms) {
   return XT_OK;
 }
 
-// Error flag of the last run (after its stream has drained): a box whose
-// energy partial was not finite or beyond 2^62 Eh did not enter the exact
-// fixed-point sums, so the run's energies are not returned.
-static int check_run_flag(xt_ctx* c, const char* fn) {
-  unsigned long long flag = 0;
-  XT_HIP(hipMemcpy(&flag, c->d_qctr + xt::kQueues, sizeof(flag), hipMemcpyDeviceToHost));
-  if(flag)
+// Waits for the last run, which left E4, E5 and its error flag in h_e45 and the
+// task energies in h_run.  The flag: a box whose energy partial was not finite or
+// beyond 2^62 Eh did not enter the exact fixed-point sums, so the run's energies
+// are not returned.
+static int fetch_result(xt_ctx* c, const char* fn) {
+  XT_HIP(hipStreamSynchronize(c->stream));
+  float ms = 0;
+  XT_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
+  c->last_ms = ms;
+  if(c->h_e45[2] != 0.0)
     return fail(XT_ERANGE, std::string(fn) +
                              ": an energy partial was not finite or beyond 2^62 Eh (zero or "
                              "non-finite orbital-energy denominators, or non-finite inputs)");
@@ -1233,20 +1271,16 @@ int xt_run(xt_ctx* c, const xt_opts* opts, double* e45, double* task_partials, f
   if(rc) return rc;
   const long nt = (long) c->plan.dev.size();
   if((rc = run_units(c, o, nullptr))) return rc;
-  hipStream_t st = c->stream;
-  XT_HIP(hipMemcpyAsync(e45, c->d_e45, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-  if(task_partials)
-    XT_HIP(hipMemcpyAsync(task_partials, c->d_task_e, 2 * nt * sizeof(double),
-                          hipMemcpyDeviceToHost, st));
-  XT_HIP(hipStreamSynchronize(st));
-  float ms = 0;
-  XT_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-  c->last_ms = ms;
-  if((rc = check_run_flag(c, "xt_run"))) {
-    e45[0] = e45[1] = std::nan("");
-    if(task_partials) std::fill(task_partials, task_partials + 2 * nt, std::nan(""));
+  if((rc = fetch_result(c, "xt_run"))) {
+    if(rc == XT_ERANGE) {
+      e45[0] = e45[1] = std::nan("");
+      if(task_partials) std::fill(task_partials, task_partials + 2 * nt, std::nan(""));
+    }
     return rc;
   }
+  e45[0] = c->h_e45[0];
+  e45[1] = c->h_e45[1];
+  if(task_partials) std::memcpy(task_partials, host_task_e(c), 2 * nt * sizeof(double));
   if(o.record_task_time && task_ms) return task_times(c, nt, task_ms);
   return XT_OK;
 }
@@ -1255,7 +1289,7 @@ int xt_sum_task_energies(long n, const double* task_partials, double* e45) {
   if(n < 0 || !e45 || (n > 0 && !task_partials))
     return fail(XT_EINVAL, "xt_sum_task_energies: null argument or negative count");
   if(n > INT_MAX) return fail(XT_EINVAL, "xt_sum_task_energies: more than INT_MAX tasks");
-  // the order of k_reduce_final: kReduceThreads runs of ceil(n / kReduceThreads)
+  // the order of k_reduce: kReduceThreads runs of ceil(n / kReduceThreads)
   // consecutive tasks, each summed in task order, then a halving tree
   constexpr int kT = xt::kReduceThreads;
   double        ra[kT], rb[kT];
@@ -1298,18 +1332,14 @@ int xt_run_tasks(xt_ctx* c, const xt_opts* opts, long n, const long* which, doub
     sel[i]         = (int) which[i];
   }
   if((rc = run_units(c, o, &sel))) return rc;
-  std::vector<double> te(2 * nt);
-  XT_HIP(hipMemcpyAsync(te.data(), c->d_task_e, 2 * nt * sizeof(double), hipMemcpyDeviceToHost,
-                        c->stream));
-  XT_HIP(hipStreamSynchronize(c->stream));
-  float ms = 0;
-  XT_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-  c->last_ms = ms;
-  if((rc = check_run_flag(c, "xt_run_tasks"))) {
-    e45[0] = e45[1] = std::nan("");
-    if(task_partials) std::fill(task_partials, task_partials + 2 * n, std::nan(""));
+  if((rc = fetch_result(c, "xt_run_tasks"))) {
+    if(rc == XT_ERANGE) {
+      e45[0] = e45[1] = std::nan("");
+      if(task_partials) std::fill(task_partials, task_partials + 2 * n, std::nan(""));
+    }
     return rc;
   }
+  const double* te = host_task_e(c);
   e45[0] = e45[1] = 0.0;
   for(long i = 0; i < n; i++) {  // listed order
     e45[0] += te[2 * which[i]];

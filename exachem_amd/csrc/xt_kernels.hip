@@ -780,30 +780,38 @@ __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) 
   if(tid == 0) sums_flush(R, s_cur, s_sum);
 }
 
-// Per-task energy from the fixed-point accumulators, scaled by the task factor.
-__global__ void k_reduce_tasks(const TaskDev* tasks, int n_tasks, const unsigned long long* acc,
-                               double* task_e) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if(t >= n_tasks) return;
-  const double f             = tasks[t].factor;
-  task_e[2 * (size_t) t]     = f * fx_value(&acc[4 * (size_t) t]);
-  task_e[2 * (size_t) t + 1] = f * fx_value(&acc[4 * (size_t) t + 2]);
-}
-
-__global__ void k_zero_u64(unsigned long long* p, long n) {
+// Start of a run: clears the counters and sums and brings the queues from host
+// memory; three fills and four copies in its place were a gap of about 10 us each.
+// Bound by its launch.
+__global__ void k_begin(unsigned long long* zero, long nz, unsigned long long* dst,
+                        const unsigned long long* src, long n) {
   const long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
-  if(i < n) p[i] = 0ull;
+  if(i < nz) zero[i] = 0ull;
+  if(i < n) dst[i] = src[i];
 }
 
-// Fixed-shape sum over tasks in task order (one workgroup of NT threads):
+// Per-task energies from the fixed-point accumulators, scaled by the task's
+// factor, and their fixed-shape sum in task order (one workgroup of NT threads):
 // thread i sums tasks [i*per, (i+1)*per) in order, per = ceil(n/NT), then a
-// halving tree over the threads.
+// halving tree over the threads.  Bound by its launch and by what follows it:
+// all results go straight to host memory, as a copy back costs more than the sum.
+// With k_begin and this, a whole mixed run of O=8, V=48 takes 0.37 ms (0.43 with
+// fills, copies and two reduction kernels), an FP64 run of O=7, V=22 0.40 (0.47).
 static_assert(NT == kReduceThreads, "the host repeats this reduction with kReduceThreads");
-__global__ void __launch_bounds__(NT) k_reduce_final(const double* task_e, int n, double* e45) {
+__global__ void __launch_bounds__(NT) k_reduce(const TaskDev* tasks, int n, const unsigned long long* acc,
+                                              const unsigned long long* err, double* task_e, double* task_h,
+                                              double* e45) {
   __shared__ double ra[NT], rb[NT];
-  const int         per = (n + NT - 1) / NT;
-  const int         lo = threadIdx.x * per, hi = min(n, lo + per);
-  double            a = 0.0, b = 0.0;
+  for(int t = threadIdx.x; t < n; t += NT) {
+    const double f  = tasks[t].factor;
+    const double e4 = f * fx_value(&acc[4 * (size_t) t]), e5 = f * fx_value(&acc[4 * (size_t) t + 2]);
+    task_e[2 * (size_t) t]     = task_h[2 * (size_t) t]     = e4;
+    task_e[2 * (size_t) t + 1] = task_h[2 * (size_t) t + 1] = e5;
+  }
+  __syncthreads();
+  const int per = (n + NT - 1) / NT;
+  const int lo = threadIdx.x * per, hi = min(n, lo + per);
+  double    a = 0.0, b = 0.0;
   for(int t = lo; t < hi; t++) {
     a += task_e[2 * (size_t) t];
     b += task_e[2 * (size_t) t + 1];
@@ -821,6 +829,7 @@ __global__ void __launch_bounds__(NT) k_reduce_final(const double* task_e, int n
   if(threadIdx.x == 0) {
     e45[0] = ra[0];
     e45[1] = rb[0];
+    e45[2] = *err ? 1.0 : 0.0;
   }
 }
 
@@ -1005,10 +1014,10 @@ int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups,
   return (int) hipGetLastError();
 }
 
-int launch_zero_u64(unsigned long long* p, long n, void* stream) {
-  if(n <= 0) return 0;
-  hipLaunchKernelGGL(k_zero_u64, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0,
-                     (hipStream_t) stream, p, n);
+int launch_begin(unsigned long long* zero, long nz, unsigned long long* dst,
+                 const unsigned long long* src, long n, void* stream) {
+  hipLaunchKernelGGL(k_begin, dim3((unsigned) ((std::max(nz, n) + 255) / 256)), dim3(256), 0,
+                     (hipStream_t) stream, zero, nz, dst, src, n);
   return (int) hipGetLastError();
 }
 
@@ -1018,11 +1027,10 @@ int launch_spatial_fp64(const SpatialDev& S, const RunDev& R, int grid, void* st
 }
 
 int launch_reduce(const TaskDev* tasks, int n_tasks, const unsigned long long* acc,
-                  double* task_e, double* e45, void* stream) {
-  hipStream_t st = (hipStream_t) stream;
-  hipLaunchKernelGGL(k_reduce_tasks, dim3(n_tasks > 0 ? (n_tasks + 255) / 256 : 1), dim3(256), 0, st, tasks,
-                     n_tasks, acc, task_e);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(NT), 0, st, task_e, n_tasks, e45);
+                  const unsigned long long* err, double* task_e, double* task_h, double* e45,
+                  void* stream) {
+  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(NT), 0, (hipStream_t) stream, tasks, n_tasks, acc,
+                     err, task_e, task_h, e45);
   return (int) hipGetLastError();
 }
 
