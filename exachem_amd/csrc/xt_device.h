@@ -113,8 +113,7 @@ struct RunDev {
                                // beyond 2^62 Eh (zeroed before a run, read after it)
   unsigned long long* acc;     // [4*n_tasks] (E4 lo, E4 hi, E5 lo, E5 hi): 128-bit
                                // two's-complement fixed point, scale 2^64 per Eh
-  unsigned long long* cost;    // [n_tasks] summed workgroup wall-clock ticks, a box's times its
-                               // fold weight (optional)
+  unsigned long long* cost;    // [n_tasks] summed workgroup wall-clock ticks (optional)
   unsigned long long* prog;    // [kQueues] host-mapped mirror of the ticket counters (optional)
   int                 n_tasks;
   int                 glog[6];  // ticket group shape (log2 extent per position, sum 6)

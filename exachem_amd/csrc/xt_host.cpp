@@ -383,6 +383,7 @@ struct xt_ctx {
         *p = nullptr;
       }
     have_inputs = false;
+    fold        = false;
     free_split();
   }
   void free_split() {
@@ -976,18 +977,25 @@ static long long task_tickets(const xt::TaskDev& T, const int* glog, bool mixed)
   return xt::task_ticket_count(mixed ? T.nsubm : T.nsub, glog);
 }
 
-// Share of a task's boxes that run when the copies under the exchange of
-// equal tiles are skipped.
+// Share of a task's elements in the boxes that run when the copies under the
+// exchange of equal tiles are skipped.  Of two (three) equal positions cut into
+// boxes of extents x, the ascending ones hold sum_{a<=b} x_a x_b = (S1^2 + S2) / 2
+// (sum_{a<=b<=c} = (S1^3 + 3 S1 S2 + 2 S3) / 6) elements, Sk = sum_a x_a^k.
 static double fold_share(const xt::TaskDev& T, bool mixed) {
-  const int* nb    = mixed ? T.nsubm : T.nsub;
-  double     share = 1.0;
+  double share = 1.0;
   for(int s = 0; s < 6; s += 3) {
-    const int    e = (T.eq >> (s ? 2 : 0)) & 3;
-    const double n = nb[e == 2 ? s + 1 : s];  // boxes along the equal positions
-    if(e == 3) share *= (n + 1) * (n + 2) / (6 * n * n);
-    else if(e) share *= (n + 1) / (2 * n);
+    const int e = (T.eq >> (s ? 2 : 0)) & 3;
+    if(!e) continue;
+    const int    d = T.dim[e == 2 ? s + 1 : s], w = mixed && s ? 8 : 4;
+    const double n = d / w, x = w, r = d % w, S1 = d, S2 = n * x * x + r * r, S3 = n * x * x * x + r * r * r;
+    share *= e == 3 ? (S1 * S1 * S1 + 3 * S1 * S2 + 2 * S3) / (6 * S1 * S1 * S1) : (S1 * S1 + S2) / (2 * S1 * S1);
   }
   return share;
+}
+// Flops that a run computes of task t: the analytic count less what folding skips.
+static double run_flops(const xt_ctx* c, long t, bool mixed) {
+  const xt::TaskDev& T = c->plan.dev[t];
+  return T.flops * (c->fold ? fold_share(T, mixed) : 1.0);
 }
 
 static Queues build_queues(const Plan& P, const std::vector<int>& sel, int schedule,
@@ -1178,8 +1186,7 @@ static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
   return report_progress(c, o, Q);
 }
 
-// Summed workgroup time of each task (ms), from wall-clock ticks; a box that
-// stands for its copies (fold_weight) counts once for each.
+// Summed workgroup time of each task (ms), from wall-clock ticks.
 static int task_times(xt_ctx* c, long nt, float* task_ms) {
   std::vector<unsigned long long> ticks(nt);
   XT_HIP(hipMemcpy(ticks.data(), c->d_cost, nt * 8, hipMemcpyDeviceToHost));
@@ -1601,7 +1608,13 @@ int xt_task_features(xt_ctx* c, int precision, float* feats) {
   if(precision != XT_PREC_FP64 && precision != XT_PREC_MIXED)
     return fail(XT_EINVAL, "xt_task_features: unknown precision");
   for(size_t k = 0; k < c->plan.dev.size(); k++) {
-    for(int p = 0; p < 6; p++) feats[7 * k + p] = (float) c->plan.dev[k].dim[p] / 48.f;
+    const xt::TaskDev& T = c->plan.dev[k];
+    for(int p = 0; p < 6; p++) {
+      // equal extents need not be equal tiles (the other spin's tiles have the
+      // same): without the sign the model cannot tell the tasks that run in part
+      const bool same  = c->fold && p % 3 && (T.eq >> (p < 3 ? p - 1 : p - 2)) & 1;
+      feats[7 * k + p] = (same ? -1.f : 1.f) * (float) T.dim[p] / 48.f;
+    }
     feats[7 * k + 6] = precision == XT_PREC_MIXED ? 1.f : 0.f;
   }
   return XT_OK;
@@ -1638,7 +1651,7 @@ int xt_learn_schedule(xt_ctx* c, xt_mlp* m, const xt_opts* opts, long n_sample, 
   pick.erase(std::unique(pick.begin(), pick.end()), pick.end());
   // timing runs
   std::vector<float>  x, t;
-  std::vector<double> lt, lf;  // log time, log flops of each sample
+  std::vector<double> lt, lf;  // log time, log flops computed of each sample
   std::vector<float>  feats(7 * n);
   for(int prec = 0; prec < 2; prec++) {
     if(!(precision_mask & (1 << prec))) continue;
@@ -1653,7 +1666,7 @@ int xt_learn_schedule(xt_ctx* c, xt_mlp* m, const xt_opts* opts, long n_sample, 
     if((rc = xt_task_features(c, o.precision, feats.data()))) return rc;
     for(size_t i = 0; i < pick.size(); i++) {
       if(!(ms[i] > 0.f)) continue;
-      const double fl = c->plan.dev[pick[i]].flops;
+      const double fl = run_flops(c, pick[i], prec == 1);
       for(int j = 0; j < 7; j++) x.push_back(feats[7 * pick[i] + j]);
       lt.push_back(std::log((double) ms[i]));
       lf.push_back(std::log(fl));
@@ -1688,10 +1701,8 @@ int xt_learn_schedule(xt_ctx* c, xt_mlp* m, const xt_opts* opts, long n_sample, 
   if((rc = xt_mlp_predict(m, n, feats.data(), y.data()))) return rc;
   std::vector<double> cost(n);
   for(long k = 0; k < n; k++) {
-    const double fl = c->plan.dev[k].flops;
-    // predicted time of every box, times the share of them that runs
-    const double cc = fl * std::exp(mu + sd * (double) y[k]) *
-                      (c->fold ? fold_share(c->plan.dev[k], opts->precision == XT_PREC_MIXED) : 1.0);
+    const double fl = run_flops(c, k, opts->precision == XT_PREC_MIXED);
+    const double cc = fl * std::exp(mu + sd * (double) y[k]);
     cost[k]         = (std::isfinite(cc) && cc > 0.0) ? cc : fl;
   }
   c->learned_cost = cost;

@@ -903,8 +903,7 @@ __global__ void __launch_bounds__(NT) k_spatial_mixed(MixedDev M, RunDev R) {
           s_cur = ti;
         }
         sums_add(R, s_sum, s_weight * e4, s_weight * e5);
-        // a box's time counts for its copies too, so a task's time follows its extents
-        if(R.cost) atomicAdd(&R.cost[ti], s_weight * (wall_clock64() - t0));
+        if(R.cost) atomicAdd(&R.cost[ti], wall_clock64() - t0);
       }
     }
   }

@@ -297,7 +297,9 @@ class CCSDTriples:
                     task_ms=tm if record_task_time else None, kernel_ms=ms.value)
 
     def task_features(self, precision=PREC_FP64):
-        """Cost-model inputs of every task: (n, 7) float32."""
+        """Cost-model inputs of every task: (n, 7) float32, the extents / 48
+        (negative for an equal tile whose box copies are skipped) and the
+        precision flag."""
         f = np.zeros((max(self.num_tasks(), 1), MLP_IN), dtype=np.float32)
         check(lib().xt_task_features(self._ctx, precision, _fp(f)))
         return f[:self.num_tasks()]

@@ -215,7 +215,9 @@ int xt_prepare(xt_ctx* ctx, int precision);
  * correction, which includes E[4]), summed in task order in FP64 with the
  * factors applied per task.  task_partials[2*n] (optional) receives each
  * task's (E[4], E[5]) contribution, factor included; task_ms[n] (optional)
- * receives per-task device time in ms when opts->record_task_time is set.
+ * receives per-task device time in ms when opts->record_task_time is set: the
+ * summed time of the workgroups that computed its boxes (copies of boxes of
+ * equal tiles that are not computed take none).
  * XT_ERANGE if an energy partial was not finite or beyond 2^62 Eh (it cannot
  * enter the exact fixed-point sums); e45 and task_partials are then NaN.
  */
@@ -346,9 +348,12 @@ int xt_autotune(xt_ctx* ctx, const xt_opts* opts, long n_sample, int* best, doub
  * A 7 -> 64 -> 64 -> 1 FP32 perceptron (ReLU hidden layers) whose training
  * (forward, back-propagation, Adam) and inference run as HIP kernels on the
  * model's device.  Inputs per task (xt_task_features): the six tile extents
- * / 48 and the precision flag (0 FP64, 1 mixed).  The scheduler uses it to
- * predict log(task time / analytic flops); a task's cost is its flop count
- * times the predicted time per flop.
+ * / 48 (negative where a position lies on the tile of the one before it and
+ * copies of its boxes are not computed: uploaded integrals that have the
+ * symmetry (ai|bj) = (bj|ai)) and the precision flag (0 FP64, 1 mixed).  The
+ * scheduler uses it to predict log(task time / flops computed); a task's cost
+ * is that flop count (the analytic one less the skipped copies) times the
+ * predicted time per flop.
  * ------------------------------------------------------------------------ */
 #define XT_MLP_IN 7
 #define XT_MLP_HIDDEN 64
@@ -373,7 +378,8 @@ int xt_mlp_train(xt_mlp* m, long n, const float* x, const float* t, int steps, f
 /* y[n] = model(x[n][7]). */
 int xt_mlp_predict(xt_mlp* m, long n, const float* x, float* y);
 
-/* Model inputs of every task of the tiling at a precision: feats[n_tasks][7]. */
+/* Model inputs of every task of the tiling at a precision: feats[n_tasks][7]
+ * (extents are all positive before an upload). */
 int xt_task_features(xt_ctx* ctx, int precision, float* feats);
 /* Per-task costs used by XT_SCHED_LEARNED (any positive unit). */
 int xt_set_task_cost(xt_ctx* ctx, const double* cost);
@@ -391,8 +397,8 @@ typedef struct xt_learn_stats {
  * each precision in precision_mask (bit 0 FP64, bit 1 mixed), trains the
  * model on log(time/flops) (standardised), predicts every task at
  * opts->precision and installs flops * predicted time per flop as the
- * XT_SCHED_LEARNED costs.  The analytic flop count stays the fallback: a
- * non-finite or non-positive prediction leaves that task at its flop cost. */
+ * XT_SCHED_LEARNED costs.  The flop count stays the fallback: a non-finite or
+ * non-positive prediction leaves that task at its flop cost. */
 int xt_learn_schedule(xt_ctx* ctx, xt_mlp* m, const xt_opts* opts, long n_sample,
                       int precision_mask, int steps, float lr, xt_learn_stats* stats);
 
