@@ -1064,7 +1064,7 @@ static int report_progress(xt_ctx* c, const xt_opts& o, const Queues& Q) {
 
 // Launches the persistent kernel over the tasks `sel` (all if null), then the
 // per-task fixed-point -> FP64 conversion and the fixed-order sum.
-static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_sel) {
+static int queue_run(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_sel) {
   const Plan&      P  = c->plan;
   const long       nt = (long) P.dev.size();
   std::vector<int> sel;
@@ -1184,6 +1184,15 @@ static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
   XT_HIP(hipGraphLaunch(c->graph, st));
   XT_HIP(hipEventRecord(c->ev1, st));
   return report_progress(c, o, Q);
+}
+
+// As queue_run; after an error nothing of the run is left on the stream, whose
+// first kernel reads the queues from h_run, which the next run writes and a larger
+// plan frees.
+static int run_units(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_sel) {
+  const int rc = queue_run(c, o, tasks_sel);
+  if(rc) (void) hipStreamSynchronize(c->stream);
+  return rc;
 }
 
 // Summed workgroup time of each task (ms), from wall-clock ticks.
