@@ -148,14 +148,17 @@ int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups,
 int build_operands(int O, int V, double* t2, double* ovoo, double*& vvvo, SpatialBufs& B,
                    void* stream);
 int launch_spatial_fp64(const SpatialDev& S, const RunDev& R, int grid, void* stream);
-// Into host memory: the task energies (task_h) and E4, E5 and 1 where *err is
-// set, else 0 (e45); task_e is device memory.
-int launch_reduce(const TaskDev* tasks, int n_tasks, const unsigned long long* acc,
-                  const unsigned long long* err, double* task_e, double* task_h, double* e45,
-                  void* stream);
-// Clears zero[0, nz) and copies dst[0, n) = src[0, n) (src in host memory).
+// Into host memory: the energies of the tasks that the queues list (task_h) and
+// E4, E5 (0 where they do not list every task) and 1 where *err is set, else 0
+// (e45); task_e is device memory.
+int launch_reduce(const TaskDev* tasks, int n_tasks, const int* qbeg, const int* qtask,
+                  const unsigned long long* acc, const unsigned long long* err, double* task_e,
+                  double* task_h, double* e45, void* stream);
+// Clears zero[0, nz) and copies the queues, dst[0, n) = src[0, n) (src in host
+// memory), of the entries' tasks (from word task0) and first tickets (from word
+// tick0, one a word) at least those in use.
 int launch_begin(unsigned long long* zero, long nz, unsigned long long* dst,
-                 const unsigned long long* src, long n, void* stream);
+                 const unsigned long long* src, long n, long task0, long tick0, void* stream);
 // tile_o[O] / tile_v[V]: spatial tile index of every orbital (host arrays).
 int build_split(const SpatialBufs& B, int O, int V, const int* tile_o, int nto, const int* tile_v,
                 int ntv, SplitBufs& S, void* stream);

@@ -1138,14 +1138,15 @@ static int queue_run(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
   // memset nodes when captured), which also brings the queues
   auto body = [&](bool events) -> int {
     int err = xt::launch_begin((unsigned long long*) c->d_sums, kCounters + 5 * std::max<long>(nt, 1),
-                               (unsigned long long*) c->d_queues, (unsigned long long*) c->d_run, (long) (qb.end / 8), st);
+                               (unsigned long long*) c->d_queues, (unsigned long long*) c->d_run, (long) (qb.end / 8),
+                               (long) (qb.task / 8), (long) (qb.tick / 8), st);
     if(err) return fail(XT_EHIP, std::string("begin: ") + hipGetErrorString((hipError_t) err));
     if(events) XT_HIP(hipEventRecord(c->ev0, st));
     err = mixed ? xt::launch_spatial_mixed(M, R, grid, st) : xt::launch_spatial_fp64(S, R, grid, st);
     if(err) return fail(XT_EHIP, std::string("launch: ") + hipGetErrorString((hipError_t) err));
     if(events) XT_HIP(hipEventRecord(c->ev1, st));
-    err = xt::launch_reduce(c->d_tasks, (int) nt, c->d_acc, R.err, c->d_task_e, (double*) (c->d_run + qb.end),
-                            c->d_e45, st);
+    err = xt::launch_reduce(c->d_tasks, (int) nt, c->d_qbeg, c->d_qtask, c->d_acc, R.err, c->d_task_e,
+                            (double*) (c->d_run + qb.end), c->d_e45, st);
     if(err) return fail(XT_EHIP, std::string("reduce: ") + hipGetErrorString((hipError_t) err));
     return XT_OK;
   };

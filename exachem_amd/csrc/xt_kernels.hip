@@ -781,34 +781,61 @@ __global__ void __launch_bounds__(NT, 3) k_spatial_fp64(SpatialDev S, RunDev R) 
 
 // Start of a run: clears the counters and sums and brings the queues from host
 // memory; three fills and four copies in its place were a gap of about 10 us each.
-// Bound by its launch.
+// Bound by its launch, and by PCIe where the plan has many tasks: the first head
+// words are copied as they are; behind them (task0, tick0: where the entries'
+// tasks, two a word, and first tickets begin) only the entries in use, their count
+// at the end of qbeg, which is read over PCIe first.  One task of 97,344: 24 us
+// with every word copied.
 __global__ void k_begin(unsigned long long* zero, long nz, unsigned long long* dst,
-                        const unsigned long long* src, long n) {
+                        const unsigned long long* src, long n, long head, long task0, long tick0) {
   const long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
   if(i < nz) zero[i] = 0ull;
-  if(i < n) dst[i] = src[i];
+  if(i >= n) return;
+  if(i >= head) {
+    const int ne = reinterpret_cast<const int*>(src + kQueues)[kQueues];
+    if(i >= (i < tick0 ? task0 + (ne + 1) / 2 : tick0 + ne)) return;
+  }
+  dst[i] = src[i];
 }
 
-// Per-task energies from the fixed-point accumulators, scaled by the task's
-// factor, and their fixed-shape sum in task order (one workgroup of NT threads):
-// thread i sums tasks [i*per, (i+1)*per) in order, per = ceil(n/NT), then a
-// halving tree over the threads.  Bound by its launch and by what follows it:
-// all results go straight to host memory, as a copy back costs more than the sum.
-// With k_begin and this, a whole mixed run of O=8, V=48 takes 0.37 ms (0.43 with
-// fills, copies and two reduction kernels), an FP64 run of O=7, V=22 0.40 (0.47).
-static_assert(NT == kReduceThreads, "the host repeats this reduction with kReduceThreads");
-__global__ void __launch_bounds__(NT) k_reduce(const TaskDev* tasks, int n, const unsigned long long* acc,
-                                              const unsigned long long* err, double* task_e, double* task_h,
-                                              double* e45) {
-  __shared__ double ra[NT], rb[NT];
-  for(int t = threadIdx.x; t < n; t += NT) {
-    const double f  = tasks[t].factor;
+// Energies of the tasks of a run, the ones its queues list or all n in task
+// order, from the fixed-point accumulators, scaled by the task's factor: to
+// device memory and to host memory, as a copy back costs more than the sum.
+__device__ __forceinline__ void task_energies(const TaskDev* tasks, int n, const int* qbeg, const int* qtask,
+                                              const unsigned long long* acc, double* task_e, double* task_h,
+                                              int first, int step) {
+  const int ne = qbeg[kQueues];
+  for(int x = first; x < ne; x += step) {
+    const int    t = ne == n ? x : qtask[x];
+    const double f = tasks[t].factor;
     const double e4 = f * fx_value(&acc[4 * (size_t) t]), e5 = f * fx_value(&acc[4 * (size_t) t + 2]);
     task_e[2 * (size_t) t]     = task_h[2 * (size_t) t]     = e4;
     task_e[2 * (size_t) t + 1] = task_h[2 * (size_t) t + 1] = e5;
   }
-  __syncthreads();
-  const int per = (n + NT - 1) / NT;
+}
+__global__ void __launch_bounds__(NT) k_task_energies(const TaskDev* tasks, int n, const int* qbeg, const int* qtask,
+                                                     const unsigned long long* acc, double* task_e,
+                                                     double* task_h) {
+  task_energies(tasks, n, qbeg, qtask, acc, task_e, task_h, blockIdx.x * NT + threadIdx.x, gridDim.x * NT);
+}
+
+// Per-task energies (CONVERT: here, else by k_task_energies before) and, where
+// every task ran, their fixed-shape sum in task order (one workgroup of NT threads):
+// thread i sums tasks [i*per, (i+1)*per) in order, per = ceil(n/NT), then a
+// halving tree over the threads.  Bound by its launch and by what follows it.
+// With k_begin and this, a whole mixed run of O=8, V=48 takes 0.37 ms (0.43 with
+// fills, copies and two reduction kernels), an FP64 run of O=7, V=22 0.40 (0.47).
+static_assert(NT == kReduceThreads, "the host repeats this reduction with kReduceThreads");
+template<bool CONVERT>
+__global__ void __launch_bounds__(NT) k_reduce(const TaskDev* tasks, int n, const int* qbeg, const int* qtask,
+                                              const unsigned long long* acc, const unsigned long long* err,
+                                              double* task_e, double* task_h, double* e45) {
+  __shared__ double ra[NT], rb[NT];
+  if(CONVERT) {
+    task_energies(tasks, n, qbeg, qtask, acc, task_e, task_h, threadIdx.x, NT);
+    __syncthreads();
+  }
+  const int per = qbeg[kQueues] == n ? (n + NT - 1) / NT : 0;
   const int lo = threadIdx.x * per, hi = min(n, lo + per);
   double    a = 0.0, b = 0.0;
   for(int t = lo; t < hi; t++) {
@@ -1013,10 +1040,18 @@ int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups,
   return (int) hipGetLastError();
 }
 
+// Plans of more tasks bring only the queue entries in use and convert the task
+// energies with many workgroups (whole wall time of a run in us, with one and with
+// many: 148 tasks 196 and 199, 1,700 equal, 2,828 2,627 and 2,622, 4,180 371 and
+// 361, 13,920 14,488 and 14,450; of one task of 1,700 104 and 106).  One task of
+// 97,344 takes 89 us, 506 where one workgroup walked the plan.
+constexpr long kManyTasks = 2048;
+
 int launch_begin(unsigned long long* zero, long nz, unsigned long long* dst,
-                 const unsigned long long* src, long n, void* stream) {
+                 const unsigned long long* src, long n, long task0, long tick0, void* stream) {
+  const long head = n - tick0 <= kManyTasks ? n : task0;
   hipLaunchKernelGGL(k_begin, dim3((unsigned) ((std::max(nz, n) + 255) / 256)), dim3(256), 0,
-                     (hipStream_t) stream, zero, nz, dst, src, n);
+                     (hipStream_t) stream, zero, nz, dst, src, n, head, task0, tick0);
   return (int) hipGetLastError();
 }
 
@@ -1025,11 +1060,18 @@ int launch_spatial_fp64(const SpatialDev& S, const RunDev& R, int grid, void* st
   return (int) hipGetLastError();
 }
 
-int launch_reduce(const TaskDev* tasks, int n_tasks, const unsigned long long* acc,
-                  const unsigned long long* err, double* task_e, double* task_h, double* e45,
-                  void* stream) {
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(NT), 0, (hipStream_t) stream, tasks, n_tasks, acc,
-                     err, task_e, task_h, e45);
+int launch_reduce(const TaskDev* tasks, int n_tasks, const int* qbeg, const int* qtask,
+                  const unsigned long long* acc, const unsigned long long* err, double* task_e,
+                  double* task_h, double* e45, void* stream) {
+  const bool many = n_tasks > kManyTasks;
+  if(many) {
+    hipLaunchKernelGGL(k_task_energies, dim3((unsigned) std::min((n_tasks + NT - 1) / NT, 1024)), dim3(NT), 0,
+                       (hipStream_t) stream, tasks, n_tasks, qbeg, qtask, acc, task_e, task_h);
+    const hipError_t e = hipGetLastError();
+    if(e != hipSuccess) return (int) e;
+  }
+  hipLaunchKernelGGL(many ? k_reduce<false> : k_reduce<true>, dim3(1), dim3(NT), 0, (hipStream_t) stream, tasks,
+                     n_tasks, qbeg, qtask, acc, err, task_e, task_h, e45);
   return (int) hipGetLastError();
 }
 

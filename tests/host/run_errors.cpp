@@ -96,13 +96,13 @@ int build_operands(int, int, double*, double*, double*&, SpatialBufs&, void*) { 
 int build_xva(int, int, SpatialBufs&, void*) { return 0; }
 int cholesky_integrals(int, int, long, const double*, double*, double*, double*, void*) { std::abort(); }
 int launch_vvoo_asym(const double*, int, int, double*, int* groups, void*) { return *groups = 0; }
-int launch_begin(unsigned long long*, long, unsigned long long*, const unsigned long long*, long, void*) {
+int launch_begin(unsigned long long*, long, unsigned long long*, const unsigned long long*, long, long, long, void*) {
   return launched(false);
 }
 int launch_spatial_fp64(const SpatialDev&, const RunDev&, int, void*) { return launched(fault == kSpatial); }
 int launch_spatial_mixed(const MixedDev&, const RunDev&, int, void*) { return launched(fault == kSpatial); }
-int launch_reduce(const TaskDev*, int, const unsigned long long*, const unsigned long long*, double*, double*,
-                  double*, void*) {
+int launch_reduce(const TaskDev*, int, const int*, const int*, const unsigned long long*, const unsigned long long*,
+                  double*, double*, double*, void*) {
   return launched(fault == kReduce);
 }
 int launch_packed_fp64(const PackedArgs&, void*) { std::abort(); }
