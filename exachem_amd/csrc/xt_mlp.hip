@@ -105,6 +105,39 @@ __global__ void __launch_bounds__(SB * H) k_mlp_pass(const float* __restrict__ P
   }
 }
 
+// The forward pass of large batches, one thread per sample: every lane reads the
+// same weight from LDS at a time, four per read, where k_mlp_pass reads a weight
+// per lane and product and runs the last layer on one lane.  The same order of
+// every sum, so the same bits.  Bound: LDS reads and FP32 products.
+__global__ void __launch_bounds__(256) k_mlp_forward(const float* __restrict__ P,
+                                                     const float* __restrict__ X, long n,
+                                                     float* __restrict__ Y) {
+  __shared__ float w[kMlpParams];
+  for(int i = threadIdx.x; i < kMlpParams; i += blockDim.x) w[i] = P[i];
+  __syncthreads();
+  const long s = (long) blockIdx.x * blockDim.x + threadIdx.x;
+  if(s >= n) return;
+  float x[IN];
+#pragma unroll
+  for(int i = 0; i < IN; i++) x[i] = X[s * IN + i];
+  float a1[H];
+#pragma unroll
+  for(int h = 0; h < H; h++) {
+    float z = w[OB1 + h];
+#pragma unroll
+    for(int i = 0; i < IN; i++) z = fmaf(x[i], w[OW1 + i * H + h], z);
+    a1[h] = fmaxf(z, 0.f);
+  }
+  float y = w[OB3];
+  for(int b = 0; b < H; b++) {
+    float z = w[OB2 + b];
+#pragma unroll
+    for(int a = 0; a < H; a++) z = fmaf(a1[a], w[OW2 + a * H + b], z);
+    y = fmaf(fmaxf(z, 0.f), w[OW3 + b], y);
+  }
+  Y[s] = y;
+}
+
 // Parameter gradients, and with TRAIN the Adam update of the same parameters:
 // one thread per parameter, samples summed in order, chunks of CS samples of
 // the factors staged through LDS with samples contiguous.  Bound: latency.  With
@@ -269,9 +302,18 @@ inline unsigned blocks(long n, int t) { return (unsigned) ((n + t - 1) / t); }
 
 }  // namespace
 
+// From here on one thread per sample is faster (xt_mlp_predict, us, with a thread
+// per hidden unit and with one per sample: 16,384 samples 69 and 82, 32,768 97 and
+// 98, 65,536 162 and 141, 1,000,000 1,815 and 1,350).
+constexpr long kManySamples = 32768;
+
 int mlp_forward(const float* P, const float* X, long n, float* Y, float* A1, float* A2,
                 void* stream) {
   if(n <= 0) return 0;
+  if(n >= kManySamples && !A1 && !A2) {
+    hipLaunchKernelGGL(k_mlp_forward, dim3(blocks(n, 256)), dim3(256), 0, (hipStream_t) stream, P, X, n, Y);
+    return (int) hipGetLastError();
+  }
   // workgroups loop over samples: staging the parameters costs more than one group of samples
   hipLaunchKernelGGL(k_mlp_pass<false>, dim3(std::min(blocks(n, SB), 1024u)), dim3(SB * H), 0,
                      (hipStream_t) stream, P, X, (const float*) nullptr, n, Y, A1, A2, (float*) nullptr,
