@@ -71,6 +71,7 @@ def lib():
     L.xt_num_tasks.argtypes = [vp, lp]
     L.xt_task_list.argtypes = [vp, lp, dp]
     L.xt_flops.argtypes = [vp, dp, dp, dp]
+    L.xt_run_flops.argtypes = [vp, C.c_int, dp, dp]
     L.xt_upload_closed_shell.argtypes = [vp] + [dp] * 7
     L.xt_synth_upload.argtypes = [vp, C.c_uint64, C.c_double, C.c_double]
     L.xt_synth_closed_shell.argtypes = [C.c_int, C.c_int, C.c_uint64, C.c_double,
@@ -111,7 +112,7 @@ def lib():
         [vp, sz] + [sz] * 6 + [vp] * 6 + [ip] * 6 + [sz] * 8 + [vp] * 6 + [vp, vp])
     L.xt_fully_fused_ccsd_t_gpu_noalloc.argtypes = L.xt_fully_fused_ccsd_t_gpu.argtypes
     for name in ("xt_create", "xt_destroy", "xt_set_tiling", "xt_num_tasks", "xt_task_list",
-                 "xt_flops", "xt_upload_closed_shell", "xt_synth_upload", "xt_synth_closed_shell",
+                 "xt_flops", "xt_run_flops", "xt_upload_closed_shell", "xt_synth_upload", "xt_synth_closed_shell",
                  "xt_run", "xt_last_kernel_ms", "xt_fully_fused_ccsd_t_gpu",
                  "xt_fully_fused_ccsd_t_gpu_noalloc", "xt_run_tasks",
                  "xt_sum_task_energies", "xt_memory_required", "xt_upload_peak_bytes",

@@ -418,6 +418,27 @@ struct xt_ctx {
   }
 };
 
+// Share of a task's elements in the boxes that run when the copies under the
+// exchange of equal tiles are skipped.  Of two (three) equal positions cut into
+// boxes of extents x, the ascending ones hold sum_{a<=b} x_a x_b = (S1^2 + S2) / 2
+// (sum_{a<=b<=c} = (S1^3 + 3 S1 S2 + 2 S3) / 6) elements, Sk = sum_a x_a^k.
+static double fold_share(const xt::TaskDev& T, bool mixed) {
+  double share = 1.0;
+  for(int s = 0; s < 6; s += 3) {
+    const int e = (T.eq >> (s ? 2 : 0)) & 3;
+    if(!e) continue;
+    const int    d = T.dim[e == 2 ? s + 1 : s], w = mixed && s ? 8 : 4;
+    const double n = d / w, x = w, r = d % w, S1 = d, S2 = n * x * x + r * r, S3 = n * x * x * x + r * r * r;
+    share *= e == 3 ? (S1 * S1 * S1 + 3 * S1 * S2 + 2 * S3) / (6 * S1 * S1 * S1) : (S1 * S1 + S2) / (2 * S1 * S1);
+  }
+  return share;
+}
+// Flops that a run computes of task t: the analytic count less what folding skips.
+static double run_flops(const xt_ctx* c, long t, bool mixed) {
+  const xt::TaskDev& T = c->plan.dev[t];
+  return T.flops * (c->fold ? fold_share(T, mixed) : 1.0);
+}
+
 extern "C" {
 
 const char* xt_last_error(void) { return g_err.c_str(); }
@@ -547,6 +568,21 @@ int xt_flops(xt_ctx* c, double* per_task, double* total, double* parts) {
     parts[1] = (double) d1;
     parts[2] = (double) d2;
   }
+  return XT_OK;
+}
+
+int xt_run_flops(xt_ctx* c, int precision, double* per_task, double* total) {
+  if(!c) return fail(XT_EINVAL, "xt_run_flops: null context");
+  if(!c->have_plan) return fail(XT_ESTATE, "xt_run_flops: no tiling");
+  if(precision != XT_PREC_FP64 && precision != XT_PREC_MIXED)
+    return fail(XT_EINVAL, "xt_run_flops: unknown precision");
+  long double sum = 0;
+  for(size_t k = 0; k < c->plan.dev.size(); k++) {
+    const double f = run_flops(c, (long) k, precision == XT_PREC_MIXED);
+    if(per_task) per_task[k] = f;
+    sum += f;
+  }
+  if(total) *total = (double) sum;
   return XT_OK;
 }
 
@@ -975,27 +1011,6 @@ struct Queues {
 // Tickets of task T under group shape glog: one per box.
 static long long task_tickets(const xt::TaskDev& T, const int* glog, bool mixed) {
   return xt::task_ticket_count(mixed ? T.nsubm : T.nsub, glog);
-}
-
-// Share of a task's elements in the boxes that run when the copies under the
-// exchange of equal tiles are skipped.  Of two (three) equal positions cut into
-// boxes of extents x, the ascending ones hold sum_{a<=b} x_a x_b = (S1^2 + S2) / 2
-// (sum_{a<=b<=c} = (S1^3 + 3 S1 S2 + 2 S3) / 6) elements, Sk = sum_a x_a^k.
-static double fold_share(const xt::TaskDev& T, bool mixed) {
-  double share = 1.0;
-  for(int s = 0; s < 6; s += 3) {
-    const int e = (T.eq >> (s ? 2 : 0)) & 3;
-    if(!e) continue;
-    const int    d = T.dim[e == 2 ? s + 1 : s], w = mixed && s ? 8 : 4;
-    const double n = d / w, x = w, r = d % w, S1 = d, S2 = n * x * x + r * r, S3 = n * x * x * x + r * r * r;
-    share *= e == 3 ? (S1 * S1 * S1 + 3 * S1 * S2 + 2 * S3) / (6 * S1 * S1 * S1) : (S1 * S1 + S2) / (2 * S1 * S1);
-  }
-  return share;
-}
-// Flops that a run computes of task t: the analytic count less what folding skips.
-static double run_flops(const xt_ctx* c, long t, bool mixed) {
-  const xt::TaskDev& T = c->plan.dev[t];
-  return T.flops * (c->fold ? fold_share(T, mixed) : 1.0);
 }
 
 static Queues build_queues(const Plan& P, const std::vector<int>& sel, int schedule,

@@ -224,6 +224,15 @@ class CCSDTriples:
         check(lib().xt_flops(self._ctx, _dp(per), C.byref(tot), _dp(parts)))
         return tot.value, per[:n], parts
 
+    def run_flops(self, precision=PREC_FP64):
+        """(total, per task) of the analytic flops that a run computes: less than
+        flops() where copies of boxes of equal tiles are skipped."""
+        n = self.num_tasks()
+        per = np.zeros(max(n, 1))
+        tot = C.c_double()
+        check(lib().xt_run_flops(self._ctx, precision, _dp(per), C.byref(tot)))
+        return tot.value, per[:n]
+
     def memory_required(self, nchol=0):
         """Device bytes of the inputs of the current tiling: dict with the
         resident FP64 operands, the upload staging (closed-shell upload, or

@@ -151,6 +151,13 @@ int xt_task_list(xt_ctx* ctx, long* tasks, double* factors);
  * per_task[n] (optional) and the total (exact integer held in a double up to 2^53,
  * also returned split as s1/d1/d2 in parts[3], optional). */
 int xt_flops(xt_ctx* ctx, double* per_task, double* total, double* parts);
+/* The part of that count which a run at `precision` computes: per_task[n] and
+ * the total (both optional).  Boxes of equal tiles that are copies of another
+ * under the exchange of those tiles are computed once where the uploaded vvoo
+ * has the symmetry (ai|bj) = (bj|ai), to 1e-13 of its largest element.  Equal to
+ * xt_flops where it misses it (every box then runs, the whole-problem path takes
+ * up to 2.5 times as long) and before an upload. */
+int xt_run_flops(xt_ctx* ctx, int precision, double* per_task, double* total);
 
 /*
  * Closed-shell spatial inputs (host memory, row-major FP64):
