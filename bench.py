@@ -16,8 +16,10 @@ the timed steps are as many of those requested as fit after the bounded legs
 below, at least one; the line reports steps and warm-up requested beside those
 run.  The calibration launches (autotuner, cost model, comparison sample) run
 the same kernel and graph before the timed steps.
-roofline: the reference's analytic flop count per launch over the persistent
-kernel's HIP-event time.  Beside it:
+roofline: the flops that a launch computes (the reference's analytic count less
+the copies of boxes of equal tiles, which are computed once) over the persistent
+kernel's HIP-event time; tflops is the same with the reference's whole count, a
+measure of time and not of the hardware's load.  Beside it:
   * fp64_compare: the plain FP64 kernel and the measured precision on the same
     seeded task sample (or on the whole workload with --fp64-full): time ratio
     and |dE4|, |dE5| of the measured precision against FP64;
@@ -213,6 +215,8 @@ def dropin_leg(xt, ctx, tiling, s, per_task, n_tasks):
             "packed_kernel_ms": kernel_ms, "packed_tflops": tf,
             "persistent_fp64_ms": r["kernel_ms"], "persistent_fp64_tflops":
             flops / r["kernel_ms"] / 1e9,
+            "persistent_fp64_computed_tflops":
+            float(ctx.run_flops(xt.PREC_FP64)[1][pick].sum()) / r["kernel_ms"] / 1e9,
             "max_rel_dE_task_vs_persistent": float(d.max()),
             "roofline": {"bound": "mfma", "achieved": tf, "peak": 78.6, "unit": "TFLOP/s",
                          "frac": tf / 78.6, "kernel": "k_packed_fp64"}}
@@ -464,6 +468,9 @@ def main():
         rng = np.random.default_rng(1)
         which = np.sort(rng.choice(n_tasks, min(args.task_sample, n_tasks), replace=False))
         total_flops = float(per_task[which].sum())
+    run_flops, run_per = ctx.run_flops(prec)  # what the boxes that run take of it
+    if which is not None:
+        run_flops = float(run_per[which].sum())
     log(f"{args.config} O={O_} V={V_} tasks={n_tasks} flops={total_flops:.4e} "
         f"upload={upload_s:.1f}s operands={operand_s:.1f}s occ={tiling.occ} vir={tiling.vir}")
 
@@ -646,7 +653,7 @@ def main():
         log(f"cpu baseline: {line['cpu_baseline']}")
     sec = float(np.mean(times))
     kernel_s = float(np.mean(kms)) / 1e3
-    achieved = total_flops / kernel_s / 1e12
+    achieved = run_flops / kernel_s / 1e12
     peak = PEAK_TFLOPS[args.precision]
     line.update({
         "value": sec, "steps": len(times), "warmup": n_warm, "ms_per_step": sec * 1e3,
@@ -656,7 +663,7 @@ def main():
                    "estimated_step_s": est_step,
                    "warmup_note": "autotuner, cost-model and comparison launches of the same "
                                   "kernel and graph precede the timed steps"},
-        "E4": res["e4"], "E5": res["e5"], "tflops": achieved,
+        "E4": res["e4"], "E5": res["e5"], "tflops": total_flops / kernel_s / 1e12,
         "setup_s": {"upload_and_layout": upload_s, "operand_split": operand_s,
                     "autotune": tune_s, "learn_schedule": learn_s},
         "autotune": tune or None,
@@ -665,13 +672,16 @@ def main():
                      "frac": achieved / peak, "traffic": None,
                      "traffic_note": "HBM bytes per launch come from rocprofv3 --pmc passes "
                                      "outside this run (profiles/)",
-                     "flops_per_launch": total_flops, "flop_count": "reference analytic count",
+                     "flops_per_launch": run_flops,
+                     "flop_count": "reference analytic count of the boxes that run",
+                     "reference_flops_per_launch": total_flops,
                      "kernel_ms": kernel_s * 1e3},
     })
     if args.precision == "mixed":
-        # three FP16 MFMA products per d1/d2 multiply-add
-        issued = (3 * (parts[1] + parts[2]) + parts[0]) if which is None else 3 * total_flops
-        line["roofline"]["mfma_issued_tflops"] = issued / kernel_s / 1e12
+        # three FP16 MFMA products per d1/d2 multiply-add of the boxes that run
+        # (s1, a small part of the count, is not a matrix product)
+        d12 = (parts[1] + parts[2]) / parts.sum()
+        line["roofline"]["mfma_issued_tflops"] = 3 * d12 * run_flops / kernel_s / 1e12
     line["wall_s"] = elapsed()
     print(json.dumps(line), flush=True)
     ctx.close()
