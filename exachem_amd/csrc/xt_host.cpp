@@ -1013,15 +1013,16 @@ static long long task_tickets(const xt::TaskDev& T, const int* glog, bool mixed)
   return xt::task_ticket_count(mixed ? T.nsubm : T.nsub, glog);
 }
 
-static Queues build_queues(const Plan& P, const std::vector<int>& sel, int schedule,
+static Queues build_queues(const xt_ctx* ctx, const std::vector<int>& sel, int schedule,
                            const std::vector<double>* cost, bool mixed, const int* glog) {
+  const Plan&                   P  = ctx->plan;
   const int                     nq = xt::kQueues;
   std::vector<std::vector<int>> per(nq);
   if(schedule == XT_SCHED_DRIVER) {
     for(size_t i = 0; i < sel.size(); i++) per[i % nq].push_back(sel[i]);
   }
   else {
-    auto c = [&](int t) { return cost ? (*cost)[t] : P.dev[t].flops; };
+    auto c = [&](int t) { return cost ? (*cost)[t] : run_flops(ctx, t, mixed); };
     std::vector<int> order = sel;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return c(a) > c(b); });
     std::vector<double> load(nq, 0.0);
@@ -1096,7 +1097,7 @@ static int queue_run(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
   for(int t: sel)  // the kernels decode a task's tickets in 32-bit arithmetic
     if(task_tickets(P.dev[t], glog, mixed) >= (1ll << 31))
       return fail(XT_EINVAL, "run: a task of 2^31 or more box tickets");
-  Queues      Q     = build_queues(P, sel, o.schedule, learned, mixed, glog);
+  Queues      Q     = build_queues(c, sel, o.schedule, learned, mixed, glog);
   hipStream_t st = c->stream;
   const QueueBytes qb(std::max<long>(nt, 1));
   std::memcpy(c->h_run, Q.total.data(), sizeof(long long) * Q.total.size());
@@ -1418,7 +1419,7 @@ int xt_queue_layout(xt_ctx* c, const xt_opts* opts, long n, const long* which, i
                                                                                : nullptr;
   const bool mixed = opts->precision == XT_PREC_MIXED;
   const int* g     = mixed ? c->glog_mixed : c->glog_fp64;
-  Queues     Q     = build_queues(c->plan, sel, opts->schedule, learned, mixed, g);
+  Queues     Q     = build_queues(c, sel, opts->schedule, learned, mixed, g);
   std::copy(Q.beg.begin(), Q.beg.end(), qbeg);
   std::copy(Q.task.begin(), Q.task.end(), qtask);
   std::copy(Q.tick.begin(), Q.tick.end(), qtick);

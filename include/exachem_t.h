@@ -52,7 +52,7 @@ extern "C" {
 
 /* Task ordering of the device work queue. */
 #define XT_SCHED_DRIVER 0   /* reference driver order (ccsd_t_fused_driver.hpp:368-383)   */
-#define XT_SCHED_ANALYTIC 1 /* longest-first by the analytic flop model                    */
+#define XT_SCHED_ANALYTIC 1 /* longest-first by the flops a run computes (xt_run_flops)    */
 #define XT_SCHED_LEARNED 2  /* longest-first by the learned cost model (falls back to 1)   */
 
 /* ---------------------------------------------------------------- errors */

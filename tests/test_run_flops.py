@@ -51,3 +51,22 @@ def test_count_of_the_boxes_that_run(xt, occ, vir):
     ctx.upload(dict(s, vvoo=s["vvoo"] + 0.1 * rng.normal(size=s["vvoo"].shape)))  # no symmetry: every box
     assert np.array_equal(ctx.run_flops(1)[1], per)
     ctx.close()
+
+
+@pytest.mark.gpu
+def test_analytic_schedule_follows_what_runs(xt):
+    """Largest first onto the least-loaded queue, by the flops that a run computes."""
+    tiling = xt.Tiling.uneven(16, 64, (3, 8), (9, 24), seed=4)
+    ctx = xt.CCSDTriples(0)
+    ctx.set_tiling(tiling)
+    ctx.synth_upload(1)
+    for prec in (0, 1):
+        _, cost = ctx.run_flops(prec)
+        lay = ctx.queue_layout(precision=prec, schedule=xt.SCHED_ANALYTIC)
+        loads = []
+        for q in range(8):
+            c = cost[lay["qtask"][lay["qbeg"][q]:lay["qbeg"][q + 1]]]
+            assert np.all(np.diff(c) <= 0)
+            loads.append(c.sum())
+        assert max(loads) - min(loads) <= cost.max()
+    ctx.close()
