@@ -148,9 +148,9 @@ int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups,
 int build_operands(int O, int V, double* t2, double* ovoo, double*& vvvo, SpatialBufs& B,
                    void* stream);
 int launch_spatial_fp64(const SpatialDev& S, const RunDev& R, int grid, void* stream);
-// Into host memory: the energies of the tasks that the queues list (task_h) and
-// E4, E5 (0 where they do not list every task) and 1 where *err is set, else 0
-// (e45); task_e is device memory.
+// Into host memory: the energies of at least the tasks that the queues list
+// (task_h), E4 and E5 (meant where they list every task) and 1 where *err is set,
+// else 0 (e45); task_e is device memory.
 int launch_reduce(const TaskDev* tasks, int n_tasks, const int* qbeg, const int* qtask,
                   const unsigned long long* acc, const unsigned long long* err, double* task_e,
                   double* task_h, double* e45, void* stream);

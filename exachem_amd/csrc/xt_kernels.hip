@@ -798,44 +798,42 @@ __global__ void k_begin(unsigned long long* zero, long nz, unsigned long long* d
   dst[i] = src[i];
 }
 
-// Energies of the tasks of a run, the ones its queues list or all n in task
-// order, from the fixed-point accumulators, scaled by the task's factor: to
-// device memory and to host memory, as a copy back costs more than the sum.
-__device__ __forceinline__ void task_energies(const TaskDev* tasks, int n, const int* qbeg, const int* qtask,
-                                              const unsigned long long* acc, double* task_e, double* task_h,
-                                              int first, int step) {
-  const int ne = qbeg[kQueues];
-  for(int x = first; x < ne; x += step) {
-    const int    t = ne == n ? x : qtask[x];
-    const double f = tasks[t].factor;
-    const double e4 = f * fx_value(&acc[4 * (size_t) t]), e5 = f * fx_value(&acc[4 * (size_t) t + 2]);
-    task_e[2 * (size_t) t]     = task_h[2 * (size_t) t]     = e4;
-    task_e[2 * (size_t) t + 1] = task_h[2 * (size_t) t + 1] = e5;
-  }
+// Energy of task t from the fixed-point accumulators, scaled by the task's factor:
+// to device memory and to host memory, as a copy back costs more than the sum.
+__device__ __forceinline__ void task_energy(int t, const TaskDev* tasks, const unsigned long long* acc,
+                                            double* task_e, double* task_h) {
+  const double f  = tasks[t].factor;
+  const double e4 = f * fx_value(&acc[4 * (size_t) t]), e5 = f * fx_value(&acc[4 * (size_t) t + 2]);
+  task_e[2 * (size_t) t]     = task_h[2 * (size_t) t]     = e4;
+  task_e[2 * (size_t) t + 1] = task_h[2 * (size_t) t + 1] = e5;
 }
+// Of the tasks that the queues list, or of all n in task order.
 __global__ void __launch_bounds__(NT) k_task_energies(const TaskDev* tasks, int n, const int* qbeg, const int* qtask,
                                                      const unsigned long long* acc, double* task_e,
                                                      double* task_h) {
-  task_energies(tasks, n, qbeg, qtask, acc, task_e, task_h, blockIdx.x * NT + threadIdx.x, gridDim.x * NT);
+  const int ne = qbeg[kQueues];
+  for(int x = blockIdx.x * NT + threadIdx.x; x < ne; x += gridDim.x * NT)
+    task_energy(ne == n ? x : qtask[x], tasks, acc, task_e, task_h);
 }
 
-// Per-task energies (CONVERT: here, else by k_task_energies before) and, where
-// every task ran, their fixed-shape sum in task order (one workgroup of NT threads):
+// Fixed-shape sum of the task energies in task order (one workgroup of NT threads):
 // thread i sums tasks [i*per, (i+1)*per) in order, per = ceil(n/NT), then a
-// halving tree over the threads.  Bound by its launch and by what follows it.
+// halving tree over the threads.  CONVERT: the energies are formed here first, of
+// all tasks; else k_task_energies has formed them, and there is no sum unless the
+// queues list every task.  Bound by its launch and by what follows it.
 // With k_begin and this, a whole mixed run of O=8, V=48 takes 0.37 ms (0.43 with
 // fills, copies and two reduction kernels), an FP64 run of O=7, V=22 0.40 (0.47).
 static_assert(NT == kReduceThreads, "the host repeats this reduction with kReduceThreads");
 template<bool CONVERT>
-__global__ void __launch_bounds__(NT) k_reduce(const TaskDev* tasks, int n, const int* qbeg, const int* qtask,
+__global__ void __launch_bounds__(NT) k_reduce(const TaskDev* tasks, int n, const int* qbeg,
                                               const unsigned long long* acc, const unsigned long long* err,
                                               double* task_e, double* task_h, double* e45) {
   __shared__ double ra[NT], rb[NT];
   if(CONVERT) {
-    task_energies(tasks, n, qbeg, qtask, acc, task_e, task_h, threadIdx.x, NT);
+    for(int t = threadIdx.x; t < n; t += NT) task_energy(t, tasks, acc, task_e, task_h);
     __syncthreads();
   }
-  const int per = qbeg[kQueues] == n ? (n + NT - 1) / NT : 0;
+  const int per = CONVERT || qbeg[kQueues] == n ? (n + NT - 1) / NT : 0;
   const int lo = threadIdx.x * per, hi = min(n, lo + per);
   double    a = 0.0, b = 0.0;
   for(int t = lo; t < hi; t++) {
@@ -1071,7 +1069,7 @@ int launch_reduce(const TaskDev* tasks, int n_tasks, const int* qbeg, const int*
     if(e != hipSuccess) return (int) e;
   }
   hipLaunchKernelGGL(many ? k_reduce<false> : k_reduce<true>, dim3(1), dim3(NT), 0, (hipStream_t) stream, tasks,
-                     n_tasks, qbeg, qtask, acc, err, task_e, task_h, e45);
+                     n_tasks, qbeg, acc, err, task_e, task_h, e45);
   return (int) hipGetLastError();
 }
 
