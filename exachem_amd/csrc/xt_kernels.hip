@@ -1039,11 +1039,12 @@ int launch_vvoo_asym(const double* vvoo, int O, int V, double* out, int* groups,
 }
 
 // Plans of more tasks bring only the queue entries in use and convert the task
-// energies with many workgroups (whole wall time of a run in us, with one and with
-// many: 148 tasks 196 and 199, 1,700 equal, 2,828 2,627 and 2,622, 4,180 371 and
-// 361, 13,920 14,488 and 14,450; of one task of 1,700 104 and 106).  One task of
-// 97,344 takes 89 us, 506 where one workgroup walked the plan.
-constexpr long kManyTasks = 2048;
+// energies with many workgroups (wall time in us with one and with many: a whole
+// run of 148 tasks 201.5 and 202.3, of 920 164.3 and 164.8, of 2,000 224.5 and 221.7,
+// of 3,700 320 and 314; one task of 148 88.4 and 89.5, of 920 74.6 and 74.4, of 2,000
+// 82.6 and 76.2, of 3,700 88.8 and 78.5).  One task of 97,344 takes 87 us, 505 where
+// one workgroup walked the plan.
+constexpr long kManyTasks = 1024;
 
 int launch_begin(unsigned long long* zero, long nz, unsigned long long* dst,
                  const unsigned long long* src, long n, long task0, long tick0, void* stream) {

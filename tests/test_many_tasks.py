@@ -8,7 +8,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-PLANS = {1700: (5, 14), 2000: (7, 11), 2208: (3, 23), 4368: (5, 20)}
+PLANS = {980: (3, 17), 1012: (1, 32), 1512: (3, 20), 4368: (5, 20)}
 
 
 @pytest.mark.parametrize("n", list(PLANS))
