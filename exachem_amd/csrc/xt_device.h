@@ -196,9 +196,7 @@ struct GatherDesc {
 GatherDesc gather_desc(const GatherBlock& B, long O, long V, long Op, long Vp);
 struct GatherSrc {
   long          O, V, Op, Vp;
-  const double* t1;    // [V][O]
-  const double* t2h;   // [V][V][O][Op]
-  const double* a[kGatherArrays];  // t1, t2h, t2p [O][O][V][Vp], vvoo [V][V][O][O],
+  const double* a[kGatherArrays];  // t1 [V][O], t2h [V][V][O][Op], t2p [O][O][V][Vp], vvoo [V][V][O][O],
                                    // ovk [O][V][O][Op], xv [V][V][O][Vp] (xv[c][b][i][a] = vvvo[a][c][b][i])
 };
 struct GatherDst {
@@ -243,7 +241,8 @@ constexpr int kMaxNoab = 50, kMaxNvab = 140;
 // d1_exec[9*noab], d2_size[7*nvab], d2_exec[9*nvab], s1_size[6], s1_exec[9],
 // then the K tile lists the host builds from them: kKlistCountInts counts
 // (one per bipartition: its entries) and, for bipartition g = 0..8 in turn, an
-// int4 per enabled K tile (family 0 d1 / 1 d2, exec slot, K, 0).
+// int4 per enabled K tile (family 0 d1 / 1 d2, exec slot, K, and a 0 that makes
+// an entry one 16-byte load).
 // kPackedMetaInts is the size at the reference's tile-count limits.
 constexpr int kKlistCountInts = 9;  // 15 + 9 ints after the size/exec arrays: 16-byte aligned
 constexpr int kPackedMetaInts =

@@ -120,11 +120,12 @@ __global__ __launch_bounds__(GT) void k_gather(const GatherDesc* __restrict__ bl
 // blockIdx.y strides over rows (A for T1, the (A, B) pair for T2), threads
 // over the occupied index (pair) of the row.
 __global__ void k_expand_t(GatherSrc S, double* __restrict__ t1_so, double* __restrict__ t2_so) {
-  const long nv = 2 * S.V, no = 2 * S.O;
+  const long    nv = 2 * S.V, no = 2 * S.O;
+  const double* t2h = S.a[kArrT2h];
   if(t1_so)
     for(long a = blockIdx.y; a < nv; a += gridDim.y)
       for(long i = (long) blockIdx.x * blockDim.x + threadIdx.x; i < no; i += (long) gridDim.x * blockDim.x) {
-        t1_so[a * no + i] = a / S.V == i / S.O ? S.t1[(a % S.V) * S.O + i % S.O] : 0.0;
+        t1_so[a * no + i] = a / S.V == i / S.O ? S.a[kArrT1][(a % S.V) * S.O + i % S.O] : 0.0;
       }
   if(t2_so) {
     // spin = index >= n, spatial = index - spin * n: no divide per element
@@ -139,7 +140,7 @@ __global__ void k_expand_t(GatherSrc S, double* __restrict__ t1_so, double* __re
         const int      si = i >= uo, sj = j >= uo;
         const long     ab = ((a - sa * S.V) * S.V + (b - sb * S.V)) * S.O, i0 = i - si * uo, j0 = j - sj * uo;
         const bool     on1 = sa == si && sb == sj, on2 = sa == sj && sb == si;
-        const double   u = on1 ? S.t2h[(ab + i0) * S.Op + j0] : 0.0, w = on2 ? S.t2h[(ab + j0) * S.Op + i0] : 0.0;
+        const double   u = on1 ? t2h[(ab + i0) * S.Op + j0] : 0.0, w = on2 ? t2h[(ab + j0) * S.Op + i0] : 0.0;
         row[q]           = on1 && on2 ? u - w : on1 ? u : on2 ? -w : 0.0;
       }
     }
@@ -163,7 +164,7 @@ __global__ void __launch_bounds__(256) k_expand_t2(GatherSrc S, double* __restri
     __syncthreads();  // the previous pair's reads are done
     for(unsigned x = threadIdx.x; x < oo; x += 256) {
       const unsigned i = q(x), j = x - i * O;
-      t[i * ld + j] = S.t2h[(p * O + i) * S.Op + j];
+      t[i * ld + j] = S.a[kArrT2h][(p * O + i) * S.Op + j];
     }
     __syncthreads();
     double2* row[4];

@@ -352,7 +352,7 @@ struct xt_ctx {
   // ticket group shapes (log2 extents per position), set by the autotuner
   int glog_fp64[6]  = {1, 1, 1, 1, 1, 1};
   int glog_mixed[6] = {1, 1, 1, 1, 1, 1};
-  // Captured launch sequence (zero fills, persistent kernel, reductions).  It
+  // Captured launch sequence (k_begin, persistent kernel, task energies and sum).  It
   // reads the queues from the device buffers above, so one instantiation
   // serves every schedule and task subset of the same precision / grid /
   // timing mode; it is dropped whenever a buffer it names is reallocated.
@@ -1196,7 +1196,7 @@ static int queue_run(xt_ctx* c, const xt_opts& o, const std::vector<int>* tasks_
     }
     c->graph_key = key;
   }
-  // with a graph the timed span also holds the two small fill and reduce kernels
+  // with a graph the timed span also holds k_begin and the small kernels at the end
   XT_HIP(hipEventRecord(c->ev0, st));
   XT_HIP(hipGraphLaunch(c->graph, st));
   XT_HIP(hipEventRecord(c->ev1, st));
@@ -1503,8 +1503,6 @@ int xt_gather_task(xt_ctx* c, const long* task, void* stream, double* d1_t2, dou
   S.V             = P.V;
   S.Op            = Op;
   S.Vp            = Vp;
-  S.t1            = c->in.t1;
-  S.t2h           = c->in.t2h;
   const double* arrays[xt::kGatherArrays] = {c->in.t1, c->in.t2h, c->in.t2p, c->in.vvoo, c->in.ovk, c->in.xv};
   std::copy(arrays, arrays + xt::kGatherArrays, S.a);
   xt::GatherDst D = {{d1_t2, d1_v2, d2_t2, d2_v2, s1_t1, s1_v2}};
@@ -1526,9 +1524,9 @@ int xt_expand_amplitudes(xt_ctx* c, void* stream, double* t1_so, double* t2_so) 
   S.V             = P.V;
   S.Op            = (P.O + 7) / 8 * 8;
   S.Vp            = (P.V + 7) / 8 * 8;
-  S.t1            = c->in.t1;
-  S.t2h           = c->in.t2h;
-  const int err   = xt::launch_expand_t(S, t1_so, t2_so, stream);
+  S.a[xt::kArrT1]  = c->in.t1;
+  S.a[xt::kArrT2h] = c->in.t2h;
+  const int err    = xt::launch_expand_t(S, t1_so, t2_so, stream);
   if(err) return fail(XT_EHIP, std::string("xt_expand_amplitudes: ") + hipGetErrorString((hipError_t) err));
   return XT_OK;
 }
@@ -1806,7 +1804,7 @@ int packed_prepare(const char* fn, const PackedCall& P, int* meta, int* n_meta, 
   for(size_t b = 0; b < P.nvab; b++)
     if(P.d2_size[7 * b + 6] <= 0 || P.d2_size[7 * b + 6] > 4096)
       return fail(XT_EINVAL, f + ": bad p7 tile size");
-  // exec slots are limited to 30 bits
+  // a limit of the interface (include/exachem_t.h), far beyond any buffer that fits a GPU
   for(size_t i = 0; i < 9 * P.noab; i++)
     if(P.d1_exec[i] >= (1 << 30)) return fail(XT_EINVAL, f + ": d1 exec slot out of range");
   for(size_t i = 0; i < 9 * P.nvab; i++)

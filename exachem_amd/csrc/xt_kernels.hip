@@ -10,9 +10,11 @@
 //     t3 indices: M = {single hole hs, particle pair (pA,pB)} and
 //     N = {hole pair (hA,hB), single particle ps}.  Each bipartition g is
 //     fed by exactly one d1 equation (K = h7) and one d2 equation (K = p7),
-//     so the two run back to back into one 64x64 FP64 accumulator held in
-//     MFMA registers (v_mfma_f64_16x16x4f64, 2x2 tiles per wave) and the
-//     result is added once into the LDS t3 tile;
+//     so the two run back to back into FP64 accumulators held in MFMA
+//     registers (v_mfma_f64_16x16x4f64) and the result is added once into the
+//     LDS t3 tile.  Up to 64 x 64, cut to the task tile: the 16 x 16 tiles that
+//     are needed are dealt to the four waves (wave_share; quadrant in the
+//     per-task kernel);
 //   * operands are staged through LDS in K-chunks of 16 (aligned 16-byte
 //     loads from zero-padded arrays) with a register prefetch of the next chunk;
 //     a workgroup holds 53 KB of LDS, so three share a CU;

@@ -102,7 +102,7 @@ int xt_fully_fused_ccsd_t_gpu(void* stream, size_t num_blocks, size_t base_size_
  * xt_fully_fused_ccsd_t_gpu; it calls no hipMalloc, hipFree or other
  * allocating routine.  The launcher's metadata (the host size/exec arrays
  * and the K tile lists built from them) goes into one fixed device array per
- * GPU of 9,940 ints (39,760 bytes: its size at the reference's MAX_NOAB = 50
+ * GPU of 9,904 ints (39,616 bytes: its size at the reference's MAX_NOAB = 50
  * / MAX_NVAB = 140 limits, larger noab / nvab fail with XT_EINVAL), held
  * until the process ends and written by small copy kernels
  * on `stream` whose arguments carry the host arrays, so the caller may reuse
@@ -378,7 +378,7 @@ int xt_mlp_set_params(xt_mlp* m, const float* params);
  * respect to every parameter (grad[XT_MLP_PARAMS]); parameters unchanged. */
 int xt_mlp_loss_grad(xt_mlp* m, long n, const float* x, const float* t, float* loss, float* grad);
 /* `steps` full-batch Adam steps (beta 0.9/0.999, eps 1e-8) at rate lr,
- * replayed from one captured graph; loss_hist[steps] (optional) receives the
+ * captured in blocks and replayed; loss_hist[steps] (optional) receives the
  * loss before each step.  Deterministic. */
 int xt_mlp_train(xt_mlp* m, long n, const float* x, const float* t, int steps, float lr,
                  float* loss_hist);
