@@ -240,10 +240,12 @@ constexpr int kMaxNoab = 50, kMaxNvab = 140;
 // The launcher's packed metadata, in ints: the host arrays d1_size[7*noab],
 // d1_exec[9*noab], d2_size[7*nvab], d2_exec[9*nvab], s1_size[6], s1_exec[9],
 // then the K tile lists the host builds from them: kKlistCountInts counts
-// (one per bipartition: its entries) and, for bipartition g = 0..8 in turn, an
-// int4 per enabled K tile (family 0 d1 / 1 d2, exec slot, K, and a 0 that makes
-// an entry one 16-byte load).
+// (one per bipartition: entries | d1 entries << 16) and, for bipartition
+// g = 0..8 in turn, an int4 per enabled K tile (family 0 d1 / 1 d2, exec slot, K,
+// first k with the tiles of a family end to end and the d2 ones from a multiple
+// of kPackedKC, the kernel's K chunk, on).
 // kPackedMetaInts is the size at the reference's tile-count limits.
+constexpr int kPackedKC       = 16;
 constexpr int kKlistCountInts = 9;  // 15 + 9 ints after the size/exec arrays: 16-byte aligned
 constexpr int kPackedMetaInts =
   16 * kMaxNoab + 16 * kMaxNvab + 15 + kKlistCountInts + 4 * 9 * (kMaxNoab + kMaxNvab);
@@ -263,6 +265,7 @@ struct PackedArgs {
   const double* evl[6];
   double*       partial;  // [2*num_blocks]
   long          num_blocks;
+  bool          ends;  // the kernel form with K tiles end to end in its chunks
 };
 int launch_packed_fp64(const PackedArgs& A, void* stream);
 // The same launch without allocating: the n_meta ints of host_meta go into a

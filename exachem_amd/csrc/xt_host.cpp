@@ -1779,6 +1779,18 @@ struct PackedCall {
   double*       partial;
 };
 
+// Chunks of K consecutive k in the per-task kernel.
+long chunks(int K) { return (K + xt::kPackedKC - 1) / xt::kPackedKC; }
+// The per-task kernel's form from its chunks over the nine bipartitions: `tile` with
+// a chunk per K tile, `ends` with the tiles of a family end to end.  A chunk of
+// the second form takes longer (a look-up per thread).  Six tasks, us, first and
+// second form: O=16 V=48 in tiles of 2 and 4 (5.0 times the chunks) 907 and 479, O=16
+// V=64 in 8 and 8 (2.0) 684 and 563, O=24 V=160 in 12 and 20 (1.5) 7,873 and 7,403, O=22
+// V=110 in 11 and 22 (1.33) 8,720 and 8,596, O=30 V=120 in 10 and 24 (1.30) 9,264 and
+// 9,345, O=36 V=180 in 18 and 36 (1.27) 194,600 and 200,200, O=32 V=128 in 16 and 32
+// (1.0) 53,260 and 56,920.
+bool packed_ends(long tile, long ends) { return 10 * tile > 13 * ends; }
+
 // Checks a launcher call, packs its host size/exec arrays into meta
 // (kMetaInts ints: d1_size, d1_exec, d2_size, d2_exec, s1_size, s1_exec) and
 // fills the kernel arguments except the device copy of meta.
@@ -1826,23 +1838,32 @@ int packed_prepare(const char* fn, const PackedCall& P, int* meta, int* n_meta, 
   // (ccsd_t_all_fused_cpu.hpp:173-270, 331-428)
   int* counts = m;
   m += xt::kKlistCountInts;
+  long n_tile = 0, n_ends = 0;  // chunks of the two forms
   for(int g = 0; g < 9; g++) {
     const int hs = g / 3, ps = g % 3, s1d = 3 * ((ps + 1) % 3) + hs, s2d = 3 * ps + (hs + 1) % 3;
-    int       n     = 0;
+    int       n = 0, first = 0;
     auto      entry = [&](int fam, int ex, int K) {
       m[0] = fam;
       m[1] = ex;
       m[2] = K;
-      m[3] = 0;
+      m[3] = first;
       m += 4;
+      first += K;
+      n_tile += chunks(K);
       n++;
     };
     for(size_t tb = 0; tb < P.noab; tb++)
       if(P.d1_exec[s1d + 9 * tb] >= 0) entry(0, P.d1_exec[s1d + 9 * tb], P.d1_size[3 + 7 * tb]);
+    const int nd1 = n;
+    n_ends += chunks(first);
+    first         = (first + xt::kPackedKC - 1) / xt::kPackedKC * xt::kPackedKC;
+    const int d2  = first;
     for(size_t tb = 0; tb < P.nvab; tb++)
       if(P.d2_exec[s2d + 9 * tb] >= 0) entry(1, P.d2_exec[s2d + 9 * tb], P.d2_size[6 + 7 * tb]);
-    counts[g] = n;
+    n_ends += chunks(first - d2);
+    counts[g] = n | nd1 << 16;
   }
+  A.ends = packed_ends(n_tile, n_ends);
   *n_meta = (int) (m - meta);
   for(int i = 0; i < 6; i++) A.dim[i] = (int) P.d[i];
   A.d1_t2      = P.d1_t2;

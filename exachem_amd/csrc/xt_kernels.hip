@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <mutex>
 
@@ -1084,22 +1085,29 @@ int launch_reduce(const TaskDev* tasks, int n_tasks, const int* qbeg, const int*
 // LDS of the per-task kernel, sized for three workgroups per CU (12 waves): the
 // 4^6 tile, one staged K chunk of 16 (rows padded to 18 doubles, so the 16x16x4
 // fragment reads of a half-wave hit distinct banks), which later holds the s1 V
-// blocks.  A chunk is of one K tile, so its addresses come from scalars and one
-// row pointer a thread (40.5 ms on six tasks of O=24, V=160; 41.9 with tiles
-// packed end to end into the chunks and a pointer per load).
-constexpr int PKC  = 16;
+// blocks.  Two forms of the K chunks (packed_ends in xt_host.cpp chooses): a chunk of
+// one K tile has its addresses from scalars and one row pointer a thread; with
+// the tiles of a family end to end there are fewer chunks where tiles are
+// short, and each thread looks its k up in the list of tiles, which the LDS of the
+// s1 T1 blocks holds until then.
+constexpr int PKC  = kPackedKC;
 constexpr int PLDK = PKC + 2;
 static_assert(2 * 64 * PLDK >= 9 * 256, "staging too small for the s1 V blocks");
 struct __align__(16) PSmem {
   double t3[T3N];
   double stage[2 * 64 * PLDK];
-  double t1s[S1_T1];  // s1 T1 blocks
+  union {
+    int2   klist[kMaxNoab + kMaxNvab + 1];  // (family | exec slot << 1, K - 1 | first k << 12)
+    double t1s[S1_T1];                      // later: the s1 T1 blocks
+  };
   double eps[24];
   double red[8];
   Tables tab;
   int    ext[6];  // orbitals of the block inside the tile
 };
+static_assert((kMaxNoab + kMaxNvab) * 4096 + kPackedKC < (1 << 20), "first k must fit 20 bits");
 
+template<bool ENDS>
 __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
   __shared__ PSmem sm;
   const int        tid = threadIdx.x;
@@ -1139,7 +1147,7 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
   int first = 0;  // first list entry of the bipartition
 #pragma unroll 1
   for(int g = 0; g < 9; g++) {
-    const int   nk   = k_n[g];
+    const int   nk   = k_n[g] & 0xffff, nd1 = k_n[g] >> 16;
     const int4* list = k_list + first;
     first += nk;
     if(nk == 0) continue;
@@ -1205,6 +1213,64 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
     double av[4], bv[4];
     int    clen = 0;      // k of the loaded chunk
     bool   cd2  = false;  // its family
+    // ENDS: k1 k of d1 from 0 on, the d2 ones from the chunk kd2 / PKC on; chunk c of
+    // nc; the tile of the thread's k (ia, la; na: the next one's first k) and, for the
+    // d1 <ij||ka> block, of its wave's (ib, lb, nb).
+    int  c = 0, nc = 0, k1 = 0, kd2 = 0, kall = 0, ia = 0, ib = 0, na = 0, nb = 0;
+    int2 la = {};
+    int4 lb = {};
+    auto end_of = [&](int i) { return __builtin_amdgcn_readfirstlane(list[i].z + list[i].w); };
+    auto next_b = [&]() { return ib + 1 < nk ? __builtin_amdgcn_readfirstlane(list[ib + 1].w) : INT_MAX; };
+    if(ENDS) {
+      k1   = nd1 ? end_of(nd1 - 1) : 0;
+      kd2  = cdiv(k1, PKC) * PKC;
+      kall = nk > nd1 ? end_of(nk - 1) : kd2;
+      nc   = cdiv(kall, PKC);
+      __syncthreads();  // every thread is done with the list before
+      for(int x = tid; x <= nk; x += NT) {
+        const int4 e = x < nk ? list[x] : make_int4(0, 0, 1, (1 << 20) - 1);
+        sm.klist[x]  = make_int2(e.x | e.y << 1, (int) ((unsigned) (e.z - 1) | (unsigned) e.w << 12));
+      }
+      __syncthreads();
+      la = sm.klist[0];
+      na = (int) ((unsigned) sm.klist[1].y >> 12);
+      lb = list[0];
+      nb = next_b();
+    }
+    auto load_ends = [&]() {
+      cd2  = c * PKC >= kd2;
+      clen = min(PKC, (cd2 ? kall : k1) - c * PKC);
+      const int k = c * PKC + min(kk, clen - 1);
+      while(k >= na) {
+        la = sm.klist[++ia];
+        na = (int) ((unsigned) sm.klist[ia + 1].y >> 12);
+      }
+      const long ex = la.x >> 1, Kt = (la.y & 0xfff) + 1, kl = k - (int) ((unsigned) la.y >> 12);
+      // third positions j outside the block read the last one inside
+      auto row = [&](const double* q, long s, int n, double(&v)[4]) {
+        v[0] = *q;
+#pragma unroll
+        for(int j = 1; j < 4; j++) {
+          if(j < n) q += s;
+          v[j] = *q;
+        }
+      };
+      row(cd2 ? A.d2_v2 + A.max_d2_v2 * ex + a2 * Kt + kl : A.d1_t2 + A.max_d1_t2 * ex + a1 * Kt + kl,
+          (cd2 ? DHS : DPA) * Kt, ePB, av);
+      if(cd2) row(A.d2_t2 + A.max_d2_t2 * ex + b2 * Kt + kl, Kt, ePS, bv);
+      else {
+#pragma unroll
+        for(int j = 0; j < 4; j++) {
+          const int kj = c * PKC + min(4 * kq + j, clen - 1);
+          while(kj >= nb) {
+            lb = list[++ib];
+            nb = next_b();
+          }
+          bv[j] = A.d1_v2[A.max_d1_v2 * (long) lb.y + rB1 + (kj - lb.w) * bstr1];
+        }
+      }
+      c++;
+    };
     // Issues every load of the next chunk, so that they are in flight together
     // while the previous chunk is multiplied; k past the tile's end reads its
     // last one.
@@ -1229,8 +1295,11 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
       }
       kt += clen;
     };
-    tile();
-    load();
+    if(ENDS) load_ends();
+    else {
+      tile();
+      load();
+    }
     bool more = true, lead = true;
 #pragma unroll 1
     while(more) {
@@ -1256,8 +1325,11 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
         for(int j = 0; j < 4; j++) Bs[n1 * PLDK + 4 * kq + j] = 4 * kq + j < len ? bv[j] : 0.0;
       }
       __syncthreads();
-      more = kt < K || it + 1 < nk;
-      if(more) load();
+      more = ENDS ? c < nc : kt < K || it + 1 < nk;
+      if(more) {
+        if(ENDS) load_ends();
+        else load();
+      }
       mfma_chunk<PKC, PLDK>(As, Bs, quad, acc, len);
     }
     acc_to_t3(sm.t3, sm.tab, quad, store, acc);
@@ -1310,7 +1382,7 @@ __global__ void __launch_bounds__(NT, 3) k_packed_fp64(PackedArgs A) {
 }
 
 int launch_packed_fp64(const PackedArgs& A, void* stream) {
-  hipLaunchKernelGGL(k_packed_fp64, dim3((unsigned) A.num_blocks), dim3(NT), 0,
+  hipLaunchKernelGGL(A.ends ? k_packed_fp64<true> : k_packed_fp64<false>, dim3((unsigned) A.num_blocks), dim3(NT), 0,
                      (hipStream_t) stream, A);
   return (int) hipGetLastError();
 }
