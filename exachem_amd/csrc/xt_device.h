@@ -163,37 +163,20 @@ int launch_begin(unsigned long long* zero, long nz, unsigned long long* dst,
 int build_split(const SpatialBufs& B, int O, int V, const int* tile_o, int nto, const int* tile_v,
                 int ntv, SplitBufs& S, void* stream);
 // Device gather of the per-task packed buffers (xt_gather.hip, xt_gather.cpp).
-// One GatherBlock is one Tensor::get + hptt permute of the host gathers: the
-// source block's extents, spins and spatial starts per dimension (source
-// order), the permutation (destination dimension k is source dimension
-// perm[k], row-major), the factor, and where it lands.
-enum GatherKind { kGatherT1 = 0, kGatherT2 = 1, kGatherIJAB = 2, kGatherIJKA = 3, kGatherIABC = 4 };
-struct GatherBlock {
-  long   dst;       // element offset in the destination buffer
-  long   n;         // elements
-  int    buf;       // destination: 0 d1_t2, 1 d1_v2, 2 d2_t2, 3 d2_v2, 4 s1_t1, 5 s1_v2
-  int    kind;      // GatherKind
-  int    nd;        // 2 (T1) or 4
-  int    size[4];   // source extents
-  int    start[4];  // spatial start per source dimension
-  int    spin[4];   // 0 alpha, 1 beta
-  int    perm[4];
-  double alpha;     // +1 or -1
-};
-// The same block as the kernel reads it (gather_desc): element (i0, i1, i2, i3)
-// in destination order, row-major over ext (leading extents 1 for T1), is
-// alpha * (x - y) of the terms that the spins leave, x at px + sum i sx of
-// array src, y at py + sum i sy; kS is the destination position of the first
-// term's contiguous index.
+// One GatherDesc is one Tensor::get + hptt permute of the host gathers as the kernel
+// reads it: element (i0, i1, i2, i3) in destination order, row-major over ext (leading
+// extents 1 for T1), goes to dst + its index of destination buf (0 d1_t2, 1 d1_v2, 2
+// d2_t2, 3 d2_v2, 4 s1_t1, 5 s1_v2) and is alpha * (x - y) of the terms that the spins
+// leave, x at px + sum i sx of array src, y at py + sum i sy; kS is the destination
+// position of the first term's contiguous index.
 enum GatherArray { kArrT1, kArrT2h, kArrT2p, kArrVvoo, kArrOvk, kArrXv, kGatherArrays };
 struct GatherDesc {
-  long     dst, n;
+  long     dst, n;  // n: elements
   long     px, py, sx[4], sy[4];
-  double   alpha;
   unsigned ext[4];
+  double   alpha;  // +1 or -1
   int      buf, src, on1, on2, kS;
 };
-GatherDesc gather_desc(const GatherBlock& B, long O, long V, long Op, long Vp);
 struct GatherSrc {
   long          O, V, Op, Vp;
   const double* a[kGatherArrays];  // t1 [V][O], t2h [V][V][O][Op], t2p [O][O][V][Vp], vvoo [V][V][O][O],

@@ -44,24 +44,62 @@ struct Tiles {
   }
 };
 
-GatherBlock block(int buf, int kind, long dst, const Tiles& tl, const long* tiles, int nd,
-                  const int* perm, double alpha) {
-  GatherBlock B = {};
-  B.buf         = buf;
-  B.kind        = kind;
-  B.dst         = dst;
-  B.nd          = nd;
-  B.alpha       = alpha;
-  B.n           = 1;
-  for(int d = 0; d < nd; d++) {
-    B.size[d]  = tl.range(tiles[d]);
-    B.start[d] = tl.T.spatial_off[tiles[d]];
-    B.spin[d]  = tl.spin(tiles[d]) == 2 ? 1 : 0;
-    B.perm[d]  = perm[d];
-    B.n *= B.size[d];
+// What each block of one kind has in common: the array it reads, the steps of its
+// two terms per source dimension and what pairs of equal spins enable them.
+struct Rule {
+  int src;
+  int x[4], y[4];
+};
+
+// Appends the block of `tiles` (source order) that lands at dst of buffer buf: one
+// Tensor::get + hptt permute of the host gathers (destination dimension k is source
+// dimension perm[k], row-major), times alpha.
+template<int ND>
+void block(std::vector<GatherDesc>& out, const Rule& R, int buf, long dst, const Tiles& tl,
+           const long (&tiles)[ND], const int (&perm)[ND], float alpha) {
+  constexpr int lead = 4 - ND;
+  GatherDesc&   D    = out.emplace_back();
+  int           spin[ND];
+  D.dst   = dst;
+  D.alpha = alpha;
+  D.buf   = buf;
+  D.src   = R.src;
+  long n = 1, px = 0, py = 0;
+  for(int d = 0; d < ND; d++) {
+    const long b = tiles[d];
+    spin[d]      = tl.spin(b);
+    n *= tl.range(b);
+    px += (long) tl.T.spatial_off[b] * R.x[d];
+    py += (long) tl.T.spatial_off[b] * R.y[d];
   }
-  return B;
+  D.n   = n;
+  D.px  = px;
+  D.py  = py;
+  D.on1 = ND == 2 ? spin[0] == spin[1] : spin[0] == spin[2 % ND] && spin[1] == spin[3 % ND];
+  D.on2 = ND == 2 ? 0 : spin[0] == spin[3 % ND] && spin[1] == spin[2 % ND];
+  const int* c = D.on1 || !D.on2 ? R.x : R.y;
+  D.kS         = 3;
+  for(int k = 0; k < 4; k++) {
+    D.ext[k] = 1u;
+    D.sx[k] = D.sy[k] = 0;
+    if(k < lead) continue;
+    const int d = perm[k - lead], e = tl.range(tiles[d]);
+    D.ext[k]    = (unsigned) e;
+    D.sx[k]     = R.x[d];
+    D.sy[k]     = R.y[d];
+    if(c[d] == 1 && e > 1) D.kS = k;
+  }
 }
+
+// The orders of a tuple's slots that are the task's own: equations of the task
+// that read the tuple's blocks (the same for every contracted tile).
+struct Hits {
+  int n = 0, k[9];
+  Hits(const Tuple& ref, const Tuple (&pat)[9]) {
+    for(int i = 0; i < 9; i++)
+      if(ref == pat[i]) k[n++] = i;
+  }
+};
 
 }  // namespace
 
@@ -86,7 +124,7 @@ void packed_sizes(const GatherTiling& T, long out[8]) {
   out[7] = kd2;                                  // max d2 kernels per task
 }
 
-int plan_gather(const GatherTiling& T, bool restricted, const long* t, std::vector<GatherBlock>& out,
+int plan_gather(const GatherTiling& T, bool restricted, const long* t, std::vector<GatherDesc>& out,
                 int* s1_size, int* s1_exec, int* d1_size, int* d1_exec, int* d2_size, int* d2_exec,
                 int* counts) {
   const Tiles tl{T};
@@ -96,6 +134,15 @@ int plan_gather(const GatherTiling& T, bool restricted, const long* t, std::vect
   long        sz[8];
   packed_sizes(T, sz);
   out.clear();
+  // steps of arrays that fit a GPU, so below 2^31
+  const int O = (int) T.O, V = (int) T.V, Op = (O + 7) / 8 * 8, Vp = (V + 7) / 8 * 8;
+  const Rule t1   = {kArrT1, {O, 1, 0, 0}, {0, 0, 0, 0}};  // t1[a][i]
+  // t2h[a][b][i][j], or t2p[i][j][a][b] where the destination runs over a virtual index
+  const Rule t2h  = {kArrT2h, {V * O * Op, O * Op, Op, 1}, {V * O * Op, O * Op, 1, Op}};
+  const Rule t2p  = {kArrT2p, {Vp, 1, O * V * Vp, V * Vp}, {Vp, 1, V * Vp, O * V * Vp}};
+  const Rule ijab = {kArrVvoo, {O, 1, V * O * O, O * O}, {O, 1, O * O, V * O * O}};  // vvoo[a][b][i][j], [b][a][i][j]
+  const Rule ijka = {kArrOvk, {Op, V * O * Op, 1, O * Op}, {V * O * Op, Op, 1, O * Op}};  // ovk[j][a][i][k], [i][a][j][k]
+  const Rule iabc = {kArrXv, {Vp, 1, O * Vp, V * O * Vp}, {Vp, 1, V * O * Vp, O * Vp}};   // xv[c][b][i][a], [b][c][i][a]
   std::fill(s1_exec, s1_exec + 9, -1);
   std::fill(d1_exec, d1_exec + 9 * noab, -1);
   std::fill(d2_exec, d2_exec + 9 * nvab, -1);
@@ -117,14 +164,14 @@ int plan_gather(const GatherTiling& T, bool restricted, const long* t, std::vect
       const Tuple pat[9] = {{P4, P5, P6, H1, H2, H3}, {P4, P5, P6, H2, H1, H3}, {P4, P5, P6, H2, H3, H1},
                             {P5, P4, P6, H1, H2, H3}, {P5, P4, P6, H2, H1, H3}, {P5, P4, P6, H2, H3, H1},
                             {P5, P6, P4, H1, H2, H3}, {P5, P6, P4, H2, H1, H3}, {P5, P6, P4, H2, H3, H1}};
-      for(int k = 0; k < 9; k++)
-        if(ref == pat[k]) s1_exec[k] = idx;
+      const Hits hit(ref, pat);
+      for(int j = 0; j < hit.n; j++) s1_exec[hit.k[j]] = idx;
       const long bt1[2] = {P4, H1};
       const int  pm1[2] = {1, 0};
-      out.push_back(block(4, kGatherT1, idx * dima, tl, bt1, 2, pm1, 1.0));
+      block(out, t1, 4, idx * dima, tl, bt1, pm1, 1.f);
       const long bt2[4] = {H3, H2, P6, P5};
       const int  pm2[4] = {3, 2, 1, 0};
-      out.push_back(block(5, kGatherIJAB, idx * dimb, tl, bt2, 4, pm2, 1.0));
+      block(out, ijab, 5, idx * dimb, tl, bt2, pm2, 1.f);
       idx++;
     }
     counts[0] = idx;
@@ -150,25 +197,25 @@ int plan_gather(const GatherTiling& T, bool restricted, const long* t, std::vect
       const Tuple pat[9] = {{P4, P5, P6, H1, H2, H3}, {P4, P5, P6, H2, H1, H3}, {P4, P5, P6, H2, H3, H1},
                             {P6, P4, P5, H1, H2, H3}, {P6, P4, P5, H2, H1, H3}, {P6, P4, P5, H2, H3, H1},
                             {P4, P6, P5, H1, H2, H3}, {P4, P6, P5, H2, H1, H3}, {P4, P6, P5, H2, H3, H1}};
+      const Hits hit(ref, pat);
       for(long h7 = 0; h7 < noab; h7++) {
         if(tl.spin(P4) + tl.spin(P5) != tl.spin(H1) + tl.spin(h7)) continue;
         if(!tl.all_nonempty(x) || !(h7 <= P6)) continue;
-        for(int k = 0; k < 9; k++)
-          if(ref == pat[k]) d1_exec[k + 9 * h7] = idx;
+        for(int j = 0; j < hit.n; j++) d1_exec[hit.k[j] + 9 * h7] = idx;
         if(h7 < H1) {  // doubles1.hpp:218-232: t2(p4,p5,h7,h1), perm {3,1,0,2}, -1
           const long bt[4] = {P4, P5, h7, H1};
           const int  pm[4] = {3, 1, 0, 2};
-          out.push_back(block(0, kGatherT2, idx * dima, tl, bt, 4, pm, -1.0));
+          block(out, t2h, 0, idx * dima, tl, bt, pm, -1.f);
         }
         else {  // doubles1.hpp:233-247: t2(p4,p5,h1,h7), perm {2,1,0,3}
           const long bt[4] = {P4, P5, H1, h7};
           const int  pm[4] = {2, 1, 0, 3};
-          out.push_back(block(0, kGatherT2, idx * dima, tl, bt, 4, pm, 1.0));
+          block(out, t2h, 0, idx * dima, tl, bt, pm, 1.f);
         }
         // doubles1.hpp:278-290: v2ijka(h2,h3,h7,p6), perm {2,3,0,1}
         const long bt[4] = {H2, H3, h7, P6};
         const int  pm[4] = {2, 3, 0, 1};
-        out.push_back(block(1, kGatherIJKA, idx * dimb, tl, bt, 4, pm, 1.0));
+        block(out, ijka, 1, idx * dimb, tl, bt, pm, 1.f);
         idx++;
       }
     }
@@ -195,91 +242,31 @@ int plan_gather(const GatherTiling& T, bool restricted, const long* t, std::vect
       const Tuple pat[9] = {{P4, P5, P6, H1, H2, H3}, {P4, P5, P6, H3, H1, H2}, {P4, P5, P6, H1, H3, H2},
                             {P5, P4, P6, H1, H2, H3}, {P5, P4, P6, H3, H1, H2}, {P5, P4, P6, H1, H3, H2},
                             {P5, P6, P4, H1, H2, H3}, {P5, P6, P4, H3, H1, H2}, {P5, P6, P4, H1, H3, H2}};
+      const Hits hit(ref, pat);
       for(long p7 = noab; p7 < noab + nvab; p7++) {
         if(tl.spin(P4) + tl.spin(p7) != tl.spin(H1) + tl.spin(H2)) continue;
         if(!tl.all_nonempty(x) || !(H3 <= p7)) continue;
-        for(int k = 0; k < 9; k++)
-          if(ref == pat[k]) d2_exec[k + 9 * (p7 - noab)] = idx;
+        for(int j = 0; j < hit.n; j++) d2_exec[hit.k[j] + 9 * (p7 - noab)] = idx;
         if(p7 < P4) {  // doubles2.hpp:211-225: t2(p7,p4,h1,h2), perm {3,2,1,0}, -1
           const long bt[4] = {p7, P4, H1, H2};
           const int  pm[4] = {3, 2, 1, 0};
-          out.push_back(block(2, kGatherT2, idx * dima, tl, bt, 4, pm, -1.0));
+          block(out, t2p, 2, idx * dima, tl, bt, pm, -1.f);
         }
         else {  // doubles2.hpp:226-239: t2(p4,p7,h1,h2), perm {3,2,0,1}
           const long bt[4] = {P4, p7, H1, H2};
           const int  pm[4] = {3, 2, 0, 1};
-          out.push_back(block(2, kGatherT2, idx * dima, tl, bt, 4, pm, 1.0));
+          block(out, t2p, 2, idx * dima, tl, bt, pm, 1.f);
         }
         // doubles2.hpp:335-345: v2iabc(h3,p7,p5,p6), perm {2,3,0,1}
         const long bt[4] = {H3, p7, P5, P6};
         const int  pm[4] = {2, 3, 0, 1};
-        out.push_back(block(3, kGatherIABC, idx * dimb, tl, bt, 4, pm, 1.0));
+        block(out, iabc, 3, idx * dimb, tl, bt, pm, 1.f);
         idx++;
       }
     }
     counts[2] = idx;
   }
   return 0;
-}
-
-GatherDesc gather_desc(const GatherBlock& B, long O, long V, long Op, long Vp) {
-  GatherDesc D = {};
-  D.dst        = B.dst;
-  D.n          = B.n;
-  D.alpha      = B.alpha;
-  D.buf        = B.buf;
-  const int s0 = B.spin[0], s1 = B.spin[1], s2 = B.nd > 2 ? B.spin[2] : 0, s3 = B.nd > 2 ? B.spin[3] : 0;
-  D.on1 = s0 == s2 && s1 == s3;
-  D.on2 = s0 == s3 && s1 == s2;
-  std::array<long, 4> x = {}, y = {};  // steps of the two terms per source dimension
-  switch(B.kind) {
-    case kGatherT1:  // t1[a][i]
-      D.src = kArrT1;
-      D.on1 = s0 == s1;
-      D.on2 = 0;
-      x     = {O, 1, 0, 0};
-      break;
-    case kGatherT2:
-      if(B.perm[3] < 2) {  // the destination runs over a virtual index: t2p[i][j][a][b]
-        D.src = kArrT2p;
-        x     = {Vp, 1, O * V * Vp, V * Vp};
-        y     = {Vp, 1, V * Vp, O * V * Vp};
-      }
-      else {  // t2h[a][b][i][j]
-        D.src = kArrT2h;
-        x     = {V * O * Op, O * Op, Op, 1};
-        y     = {V * O * Op, O * Op, 1, Op};
-      }
-      break;
-    case kGatherIJAB:  // vvoo[a][b][i][j], vvoo[b][a][i][j]
-      D.src = kArrVvoo;
-      x     = {O, 1, V * O * O, O * O};
-      y     = {O, 1, O * O, V * O * O};
-      break;
-    case kGatherIJKA:  // ovk[j][a][i][k], ovk[i][a][j][k]
-      D.src = kArrOvk;
-      D.on2 = s1 == s2 && s0 == s3;
-      x     = {Op, V * O * Op, 1, O * Op};
-      y     = {V * O * Op, Op, 1, O * Op};
-      break;
-    default:  // kGatherIABC: xv[c][b][i][a], xv[b][c][i][a]
-      D.src = kArrXv;
-      x     = {Vp, 1, O * Vp, V * O * Vp};
-      y     = {Vp, 1, V * O * Vp, O * Vp};
-  }
-  for(int d = 0; d < B.nd; d++) {
-    D.px += B.start[d] * x[d];
-    D.py += B.start[d] * y[d];
-  }
-  D.kS = 3;
-  for(int k = 0; k < 4; k++) {
-    const int kk = k - (4 - B.nd);
-    D.ext[k]     = kk >= 0 ? (unsigned) B.size[B.perm[kk]] : 1u;
-    D.sx[k]      = kk >= 0 ? x[B.perm[kk]] : 0;
-    D.sy[k]      = kk >= 0 ? y[B.perm[kk]] : 0;
-    if((D.on1 || !D.on2 ? D.sx[k] : D.sy[k]) == 1 && D.ext[k] > 1) D.kS = k;
-  }
-  return D;
 }
 
 }  // namespace xt

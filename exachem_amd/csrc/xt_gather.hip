@@ -54,7 +54,7 @@ constexpr int SLAB = 48 * 49;  // LDS slab (doubles): extents up to 48 with one 
 //
 // Bound: memory.  Per element the spin tests, the array's index rule and four
 // 32-bit divisions used to cost more than the copy: the host works the rules
-// out once per block (gather_desc), the divisions are multiplies, and T2 blocks
+// out once per block (plan_gather), the divisions are multiplies, and T2 blocks
 // that run over a virtual index are read from t2p, whose rows are virtual.
 __global__ __launch_bounds__(GT) void k_gather(const GatherDesc* __restrict__ blocks, GatherSrc S,
                                                GatherDst D) {

@@ -342,7 +342,6 @@ struct xt_ctx {
   // the host list it was uploaded from, kept alive until the next call)
   xt::GatherDesc*               d_gather     = nullptr;
   long                          d_gather_cap = 0;
-  std::vector<xt::GatherBlock>  h_blocks;
   std::vector<xt::GatherDesc>   h_gather;
   long                          gather_elems = 0;  // doubles written by the last gather
   hipEvent_t          ev0 = nullptr, ev1 = nullptr;
@@ -1445,7 +1444,7 @@ int xt_task_codes(xt_ctx* c, long task, uint64_t* codes) {
 // ----------------------------------------------------- device-side gather
 static xt::GatherTiling gather_tiling(const xt_ctx* c) {
   const Plan& P = c->plan;
-  return xt::GatherTiling{P.noab, P.nvab, P.k_range.data(), P.k_spin.data(), P.spatial_off.data()};
+  return xt::GatherTiling{P.noab, P.nvab, P.k_range.data(), P.k_spin.data(), P.spatial_off.data(), P.O, P.V};
 }
 
 int xt_packed_sizes(xt_ctx* c, long* sizes) {
@@ -1471,18 +1470,18 @@ int xt_gather_task(xt_ctx* c, const long* task, void* stream, double* d1_t2, dou
     const long lo = occ ? 0 : P.noab, hi = occ ? P.noab : P.noab + P.nvab;
     if(task[k] < lo || task[k] >= hi) return fail(XT_EINVAL, "xt_gather_task: tile index out of range");
   }
-  xt::plan_gather(gather_tiling(c), P.restricted, task, c->h_blocks, s1_size, s1_exec, d1_size,
+  xt::plan_gather(gather_tiling(c), P.restricted, task, c->h_gather, s1_size, s1_exec, d1_size,
                   d1_exec, d2_size, d2_exec, counts);
-  const long n  = (long) c->h_blocks.size();
-  const long Op = (P.O + 7) / 8 * 8, Vp = (P.V + 7) / 8 * 8;
+  const long n = (long) c->h_gather.size();
   c->gather_elems = 0;
-  for(const auto& B: c->h_blocks) {
+  long elems = 0, max_elems = 0;
+  for(const auto& B: c->h_gather) {
     if(B.n >= (1l << 31)) return fail(XT_EINVAL, "xt_gather_task: block of 2^31 or more doubles");
-    c->gather_elems += B.n;
+    elems += B.n;
+    max_elems = std::max(max_elems, B.n);
   }
+  c->gather_elems = elems;
   if(n == 0) return XT_OK;
-  c->h_gather.clear();
-  for(const auto& B: c->h_blocks) c->h_gather.push_back(xt::gather_desc(B, P.O, P.V, Op, Vp));
   XT_HIP(hipSetDevice(c->device));
   hipStream_t st = (hipStream_t) stream;
   if(n > c->d_gather_cap) {
@@ -1496,13 +1495,11 @@ int xt_gather_task(xt_ctx* c, const long* task, void* stream, double* d1_t2, dou
   }
   XT_HIP(hipMemcpyAsync(c->d_gather, c->h_gather.data(), sizeof(xt::GatherDesc) * n,
                         hipMemcpyHostToDevice, st));
-  long max_elems = 0;
-  for(const auto& B: c->h_gather) max_elems = std::max(max_elems, B.n);
   xt::GatherSrc S = {};
   S.O             = P.O;
   S.V             = P.V;
-  S.Op            = Op;
-  S.Vp            = Vp;
+  S.Op            = (P.O + 7) / 8 * 8;
+  S.Vp            = (P.V + 7) / 8 * 8;
   const double* arrays[xt::kGatherArrays] = {c->in.t1, c->in.t2h, c->in.t2p, c->in.vvoo, c->in.ovk, c->in.xv};
   std::copy(arrays, arrays + xt::kGatherArrays, S.a);
   xt::GatherDst D = {{d1_t2, d1_v2, d2_t2, d2_v2, s1_t1, s1_v2}};
