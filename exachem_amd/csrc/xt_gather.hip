@@ -115,6 +115,11 @@ __global__ __launch_bounds__(GT) void k_gather(const GatherDesc* __restrict__ bl
   }
 }
 
+// Element [a][i] of the spin-orbital T1.
+__device__ __forceinline__ double t1_so_value(const GatherSrc& S, long a, long i) {
+  return a / S.V == i / S.O ? S.a[kArrT1][(a % S.V) * S.O + i % S.O] : 0.0;
+}
+
 // Dense spin-orbital amplitudes, [alpha, beta] per space:
 //   t1_so[A][I] (2V x 2O), t2_so[A][B][I][J] ((2V)^2 (2O)^2), A = spin * V + a.
 // blockIdx.y strides over rows (A for T1, the (A, B) pair for T2), threads
@@ -125,7 +130,7 @@ __global__ void k_expand_t(GatherSrc S, double* __restrict__ t1_so, double* __re
   if(t1_so)
     for(long a = blockIdx.y; a < nv; a += gridDim.y)
       for(long i = (long) blockIdx.x * blockDim.x + threadIdx.x; i < no; i += (long) gridDim.x * blockDim.x) {
-        t1_so[a * no + i] = a / S.V == i / S.O ? S.a[kArrT1][(a % S.V) * S.O + i % S.O] : 0.0;
+        t1_so[a * no + i] = t1_so_value(S, a, i);
       }
   if(t2_so) {
     // spin = index >= n, spatial = index - spin * n: no divide per element
@@ -151,15 +156,24 @@ __global__ void k_expand_t(GatherSrc S, double* __restrict__ t1_so, double* __re
 // t2(a, b) of one spatial pair and writes its four spin rows, each one run of
 // 16-byte stores of two elements.  Bound: the write of 8 (2V)^2 (2O)^2 bytes
 // (an element-wise kernel made two dependent reads behind spin tests per
-// element: 2.3 TB/s at O=20, V=120).  t2_so must be 16-byte aligned.
+// element: 2.3 TB/s at O=20, V=120).  t2_so must be 16-byte aligned.  Workgroups
+// beyond the `pairs` ones write T1: as a second kernel it took a small system's
+// expansion (O=7, V=22) from 4.6 to 7.6 us.
 constexpr int kExpandMaxO = 84;  // O (O + 1) doubles of LDS
 
-__global__ void __launch_bounds__(256) k_expand_t2(GatherSrc S, double* __restrict__ t2_so) {
+__global__ void __launch_bounds__(256) k_expand_t2(GatherSrc S, double* __restrict__ t1_so,
+                                                   double* __restrict__ t2_so, unsigned pairs) {
   extern __shared__ double t[];
+  if(blockIdx.x >= pairs) {
+    const long no = 2 * S.O, n = 2 * S.V * no;
+    for(long x = (blockIdx.x - pairs) * 256l + threadIdx.x; x < n; x += (gridDim.x - pairs) * 256l)
+      t1_so[x] = t1_so_value(S, x / no, x % no);
+    return;
+  }
   const unsigned O = (unsigned) S.O, ld = O + 1, oo = O * O, np = 2 * oo;  // pairs of elements per row
   const long     V = S.V, nv = 2 * V;
   const Div      q(O, true);
-  for(long p = blockIdx.x; p < V * V; p += gridDim.x) {
+  for(long p = blockIdx.x; p < V * V; p += pairs) {
     const long a = p / V, b = p - a * V;
     __syncthreads();  // the previous pair's reads are done
     for(unsigned x = threadIdx.x; x < oo; x += 256) {
@@ -193,11 +207,11 @@ __global__ void __launch_bounds__(256) k_expand_t2(GatherSrc S, double* __restri
 
 int launch_expand_t(const GatherSrc& S, double* t1_so, double* t2_so, void* stream) {
   if(t2_so && S.O <= kExpandMaxO && ((uintptr_t) t2_so & 15) == 0) {
-    hipLaunchKernelGGL(k_expand_t2, dim3((unsigned) std::min<long>(S.V * S.V, 1l << 16)), dim3(256),
-                       (unsigned) (sizeof(double) * S.O * (S.O + 1)), (hipStream_t) stream, S, t2_so);
-    const hipError_t e = hipGetLastError();
-    if(e != hipSuccess || !t1_so) return (int) e;
-    t2_so = nullptr;  // T1 below
+    const unsigned pairs = (unsigned) std::min<long>(S.V * S.V, 1l << 16);
+    const unsigned more  = t1_so ? (unsigned) std::min<long>((4 * S.V * S.O + 255) / 256, 64) : 0;
+    hipLaunchKernelGGL(k_expand_t2, dim3(pairs + more), dim3(256), (unsigned) (sizeof(double) * S.O * (S.O + 1)),
+                       (hipStream_t) stream, S, t1_so, t2_so, pairs);
+    return (int) hipGetLastError();
   }
   const long     no = 2 * S.O, nv = 2 * S.V;
   const unsigned gx = (unsigned) std::min<long>(((t2_so ? no * no : no) + 255) / 256, 64);
