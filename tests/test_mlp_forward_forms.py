@@ -11,7 +11,7 @@ from test_cost_model import rand_params
 @pytest.mark.parametrize("n", [32767, 32768, 32769, 33023])
 def test_predictions_of_both_forms_are_the_same_bits(xt, n):
     """Both sum in the same order, so a batch equals its parts bit for bit; the
-    tolerance against the checker is that of test_mlp_batches."""
+    tolerance against the oracle is that of test_mlp_batches."""
     m = xt.CostModel(0, seed=1)
     p = rand_params(7).astype(np.float32)
     m.set_params(p)
